@@ -169,7 +169,8 @@ def project_pinhole_gaussians(means3d: Tensor, scales: Tensor, quats: Tensor, op
                                              fx, fy, cx, cy, camera_to_world, near_plane)
     if was_batched:
         return out
-    return tuple(t[0] for t in out)
+    # (squeeze, not t[0]: its backward is a view, an index's zero-fills and copies each gradient)
+    return tuple(t.squeeze(0) for t in out)
 
 
 def rasterize_pinhole_gaussians(means3d: Tensor, scales: Tensor, quats: Tensor, opacities: Tensor, colors: Tensor,
@@ -190,4 +191,4 @@ def rasterize_pinhole_gaussians(means3d: Tensor, scales: Tensor, quats: Tensor, 
         m_b.contiguous(), s_b.contiguous(), q_b.contiguous(), o_b.contiguous(), fx, fy, cx, cy, camera_to_world,
         near_plane)
     out = _rasterize_batched(means2d, conics, colors_b.contiguous(), opac, depths, config, depth_grad=False)
-    return out if was_batched else out[0]
+    return out if was_batched else out.squeeze(0)
