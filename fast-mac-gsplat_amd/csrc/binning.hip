@@ -74,9 +74,10 @@ struct SplatGeom {
 constexpr int kWaves = kThreads / 64;
 
 // Splats per wavefront in the tile walk.  A wavefront's 64 lanes test the
-// candidates of kWalkSplats splats together; fewer splats per wavefront
+// candidates of kS splats together; fewer splats per wavefront
 // than lanes gives each launch more wavefronts (the walk is latency bound)
-// and a shorter slot search.
+// and a shorter slot search.  kS is kWalkSplats, or fewer in the small-image
+// path where few splats have many candidates each (walk_splats).
 constexpr int kWalkSplats = 32;
 constexpr int kWalkBlockSplats = kWaves * kWalkSplats;
 // Emit launches with at most this many workgroups add their pair-sort
@@ -85,17 +86,18 @@ constexpr int kDirectHistBlocks = 1024;
 // Copies of the emit's digit histograms (see emit_kernel).
 constexpr int kHistCopies = 2;
 
-// One wavefront's kWalkSplats splats, staged for the cooperative tile walk.
+// One wavefront's kS splats, staged for the cooperative tile walk.
+template <int kS>
 struct WalkSlots {
-  float4 g0[kWalkSplats];  // mx, my, a, b
-  float4 g1[kWalkSplats];  // c, tau, kc, ka
-  int4 box[kWalkSplats];   // tx0, ty0, tiles per bbox row, first tile of the image
-  int4 inner[kWalkSplats]; // the certain hits (inner_tiles): x, y relative to
+  float4 g0[kS];  // mx, my, a, b
+  float4 g1[kS];  // c, tau, kc, ka
+  int4 box[kS];   // tx0, ty0, tiles per bbox row, first tile of the image
+  int4 inner[kS]; // the certain hits (inner_tiles): x, y relative to
                            // the box corner, width, height
-  int flags[kWalkSplats];  // bit 0: use_c, bit 1: use_a
-  int cend[kWalkSplats];   // inclusive prefix sum of candidate counts
-  int first[kWalkSplats];  // exclusive prefix sum: the splat's first candidate
-  int ni_incl[kWalkSplats];  // inclusive prefix sum of the certain hits
+  int flags[kS];  // bit 0: use_c, bit 1: use_a
+  int cend[kS];   // inclusive prefix sum of candidate counts
+  int first[kS];  // exclusive prefix sum: the splat's first candidate
+  int ni_incl[kS];  // inclusive prefix sum of the certain hits
   uint32_t own[64];        // per walk step: splats starting at each position
 };
 
@@ -140,13 +142,6 @@ __device__ __forceinline__ uint64_t readlane64(uint64_t v, int l) {
   const uint32_t hi =
       (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(v >> 32), l);
   return ((uint64_t)hi << 32) | lo;
-}
-
-// Index of this thread's splat in the walk order of count / emit: lanes
-// 0..kWalkSplats-1 of each wavefront take consecutive splats.
-__device__ __forceinline__ int walk_splat_index() {
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  return ((int)blockIdx.x * kWaves + wave) * kWalkSplats + lane;
 }
 
 // Smallest number of certain hits (inner_tiles) taken out of the walk: the
@@ -200,14 +195,18 @@ __device__ __forceinline__ int4 inner_tiles(float mx, float my, float a,
   return make_int4(ix0 - tx0, iy0 - ty0, iw, ih);
 }
 
-// Stages this lane's splat (lanes below kWalkSplats) and returns the
+// Stages this lane's splat (lanes below kS) and returns the
 // wavefront's candidate total: the tiles of each splat's box outside its
-// certain hits (inner_tiles), whose count goes to n_inner.  Candidate
+// certain hits (inner_tiles), whose count goes to n_inner.  With P.live the
+// box is P.boxes[source], whole: it holds the live tiles, few of which are
+// certain hits.  Candidate
 // counts fit in int32: tiles per image are limited to 2^24 on the host, so
 // a wavefront has at most 2^28 candidates.
+template <int kS>
 __device__ __forceinline__ int walk_setup(const RasterParams& P, bool valid,
                                           const SplatGeom& s, int batch,
-                                          WalkSlots& W, int& n_inner) {
+                                          int source,
+                                          WalkSlots<kS>& W, int& n_inner) {
 #pragma clang fp contract(off)
   const int lane = threadIdx.x & 63;
   int ncand = 0;
@@ -217,7 +216,17 @@ __device__ __forceinline__ int walk_setup(const RasterParams& P, bool valid,
   float4 g1 = make_float4(s.c, 0.0f, 0.0f, 0.0f);
   int flags = 0;
   float tau;
-  if (valid && alpha_support(s.o, P.alpha_thr, P.eps, tau)) {
+  if (valid && P.live != nullptr) {
+    const uint2 lb = P.boxes[source];
+    if (alpha_support(s.o, P.alpha_thr, P.eps, tau) && lb.y != 0u) {
+      box = make_int4((int)(lb.x & 0xffffu), (int)(lb.x >> 16),
+                      (int)(lb.y & 0xffffu), batch * P.tiles_per_image);
+      ncand = box.z * (int)(lb.y >> 16);
+      const ConicSlopes k = conic_slopes(s.a, s.b, s.c);
+      g1 = make_float4(s.c, tau, k.kc, k.ka);
+      flags = (k.use_c ? 1 : 0) | (k.use_a ? 2 : 0);
+    }
+  } else if (valid && alpha_support(s.o, P.alpha_thr, P.eps, tau)) {
     const PixBox bb =
         snugbox(s.mx, s.my, s.a, s.b, s.c, tau, P.width, P.height, P.eps);
     if (bb.x0 <= bb.x1 && bb.y0 <= bb.y1) {
@@ -238,7 +247,7 @@ __device__ __forceinline__ int walk_setup(const RasterParams& P, bool valid,
   }
   int inc = ncand, inc_i = n_inner;
 #pragma unroll
-  for (int off = 1; off < kWalkSplats; off <<= 1) {
+  for (int off = 1; off < kS; off <<= 1) {
     const int y = __shfl_up(inc, off, 64);
     const int yi = __shfl_up(inc_i, off, 64);
     if (lane >= off) {
@@ -246,7 +255,7 @@ __device__ __forceinline__ int walk_setup(const RasterParams& P, bool valid,
       inc_i += yi;
     }
   }
-  if (lane < kWalkSplats) {
+  if (lane < kS) {
     W.g0[lane] = make_float4(s.mx, s.my, s.a, s.b);
     W.g1[lane] = g1;
     W.box[lane] = box;
@@ -257,11 +266,11 @@ __device__ __forceinline__ int walk_setup(const RasterParams& P, bool valid,
     W.ni_incl[lane] = inc_i;
   }
   __builtin_amdgcn_wave_barrier();
-  return __shfl(inc, kWalkSplats - 1, 64);
+  return __shfl(inc, kS - 1, 64);
 }
 
 // Tests the wavefront's candidates 64 at a time and calls on_hit(slot, tile)
-// for every hit (slot = 0..kWalkSplats-1, the splat's lane in walk_setup).
+// for every hit (slot = 0..kS-1, the splat's lane in walk_setup).
 // A candidate's slot is the last splat whose first candidate is at or
 // before it (a splat without candidates shares its first index with the
 // next one and loses to it): the owner of the step's first candidate is
@@ -281,17 +290,17 @@ __device__ __forceinline__ int walk_setup(const RasterParams& P, bool valid,
 // k's ballot at rec[k], as count_block records them for the same splats):
 // the steps they cover take their hits from there instead of the exact
 // test, and steps without a hit are skipped (on_step is not called).
-template <typename Fn>
+template <int kS, typename Fn>
 __device__ __forceinline__ void walk_candidates(const RasterParams& P,
-                                                WalkSlots& W, int total,
+                                                WalkSlots<kS>& W, int total,
                                                 const uint64_t* __restrict__ rec,
                                                 Fn&& on_step) {
 #pragma clang fp contract(off)
   static_assert(kHitSlab % 64 == 0, "a slab is loaded 64 words at a time");
   const int lane = threadIdx.x & 63;
-  const int first = lane < kWalkSplats ? W.first[lane] : 0x7fffffff;
+  const int first = lane < kS ? W.first[lane] : 0x7fffffff;
   // (without certain hits in the wavefront every box is walked whole)
-  const bool any_inner = W.ni_incl[kWalkSplats - 1] != 0;
+  const bool any_inner = W.ni_incl[kS - 1] != 0;
   uint64_t chunk = 0ull;  // lane l: the recorded ballot of step 64 (k / 64) + l
   for (int c0 = 0; c0 < total; c0 += 64) {
     const int step = c0 >> 6;
@@ -341,9 +350,12 @@ __device__ __forceinline__ void walk_candidates(const RasterParams& P,
         tx = bx.x + (k - q * bx.z);
         ty = bx.y + q;
       }
+      tile = bx.w + ty * P.tiles_x + tx;
       if (recorded) {
+        // (of the live tiles' hits, with P.live)
         hit = ((hm >> lane) & 1ull) != 0ull;
-      } else {
+      } else if (P.live == nullptr ||
+                 ((P.live[tile >> 5] >> (tile & 31)) & 1u) != 0u) {
         const float4 g0 = W.g0[sl], g1 = W.g1[sl];
         const int fl = W.flags[sl];
         ConicSlopes ks;
@@ -356,7 +368,6 @@ __device__ __forceinline__ void walk_candidates(const RasterParams& P,
         hit = ellipse_hits_rect(g0.x, g0.y, g0.z, g0.w, g1.x, ks, g1.y, rx0,
                                 ry0, rx1, ry1);
       }
-      tile = bx.w + ty * P.tiles_x + tx;
     }
     if (!recorded) hm = __ballot(hit);
     on_step(hm, hit, sl, tile, c0);
@@ -368,10 +379,10 @@ __device__ __forceinline__ int hits_below(uint64_t hm, int rel) {
   return __popcll(rel >= 64 ? hm : (hm & ((1ull << rel) - 1ull)));
 }
 
-// LDS of a count block of kW wavefronts.
-template <int kW>
+// LDS of a count block of kW wavefronts of kS splats.
+template <int kW, int kS>
 struct CountLds {
-  WalkSlots walk[kW];
+  WalkSlots<kS> walk[kW];
   int wsum[kW];
 };
 
@@ -429,6 +440,13 @@ __device__ __forceinline__ void store_record(float4* __restrict__ dst,
   for (int k = 0; k < kRecordVec4; ++k) d[k] = r.v[k];
 }
 
+// The original index that the record of depth rank gid carries.
+__device__ __forceinline__ int source_of(const float4* __restrict__ packed,
+                                         int gid) {
+  return (int)(__float_as_uint(packed[kRecordVec4 * (int64_t)gid + 2].y) &
+               0x7fffffffu);
+}
+
 // The record of splat orig at depth rank gid.
 __device__ __forceinline__ void pack_record(
     const RasterParams& P, const float* __restrict__ means2d,
@@ -437,10 +455,11 @@ __device__ __forceinline__ void pack_record(
     int orig) {
   store_record(packed, gid,
                record_of(P, means2d, conics, colors, opacities, orig,
-                         (uint32_t)orig));
+                         (uint32_t)(P.orig_map != nullptr ? P.orig_map[orig]
+                                                          : orig)));
 }
 
-// Count block vb of nvb (kW wavefronts, kWalkSplats splats each), original
+// Count block vb of nvb (kW wavefronts, kS splats each), original
 // order: splat_count[orig] = tile hits of splat orig and, with block_sums,
 // block_sums[vb] = the block's total; with rec_orig also the splat's record
 // in original order, its count in the slot (pack_kernel then copies one
@@ -453,15 +472,15 @@ __device__ __forceinline__ void pack_record(
 // the two differ only when the capacity is short, and then the binning is
 // redone).  With hit_bits the block records each wavefront's first kHitSlab
 // step ballots at hit_bits[w * kHitSlab + step] (w = vb * kW + wavefront:
-// the splats' index / kWalkSplats), for an emit that walks the same splats.
-template <int kW>
+// the splats' index / kS), for an emit that walks the same splats.
+template <int kW, int kS>
 __device__ __forceinline__ void count_block(
     const RasterParams& P, const float* __restrict__ means2d,
     const float* __restrict__ conics, const float* __restrict__ opacities,
     const float* __restrict__ colors, float4* __restrict__ rec_orig,
     int32_t* __restrict__ splat_count, int32_t* __restrict__ block_sums,
     uint32_t* __restrict__ zero_words, int64_t n_zero_words, int vb, int nvb,
-    CountLds<kW>& S, uint32_t* lds_hist = nullptr,
+    CountLds<kW, kS>& S, uint32_t* lds_hist = nullptr,
     uint32_t* __restrict__ hist_row = nullptr, int hist_shift = 0,
     uint64_t* __restrict__ hit_bits = nullptr) {
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -472,8 +491,8 @@ __device__ __forceinline__ void count_block(
     for (int i = threadIdx.x; i < 2 * 257; i += 64 * kW) lds_hist[i] = 0u;
     __syncthreads();
   }
-  const int orig = (vb * kW + wave) * kWalkSplats + lane;
-  const bool valid = lane < kWalkSplats && orig < P.num_splats;
+  const int orig = (vb * kW + wave) * kS + lane;
+  const bool valid = lane < kS && orig < P.num_splats;
   const int o = valid ? orig : P.num_splats - 1;
   SplatGeom s;
   s.mx = means2d[2 * o + 0];
@@ -482,14 +501,16 @@ __device__ __forceinline__ void count_block(
   s.b = conics[3 * o + 1];
   s.c = conics[3 * o + 2];
   s.o = opacities[o];
-  WalkSlots& W = S.walk[wave];
+  WalkSlots<kS>& W = S.walk[wave];
   int n_inner;
-  const int total = walk_setup(P, valid, s, o / P.gpb, W, n_inner);
+  const int total =
+      walk_setup(P, valid, s, o / P.gpb,
+                 P.orig_map != nullptr ? P.orig_map[o] : o, W, n_inner);
   // Hits before the end of this lane's splat's candidates (lanes below
-  // kWalkSplats): the running total of the steps before plus the hits below
+  // kS): the running total of the steps before plus the hits below
   // the end inside its step; a splat's count is the difference to the
   // previous lane's.
-  const int my_end = lane < kWalkSplats ? W.cend[lane] : 0;
+  const int my_end = lane < kS ? W.cend[lane] : 0;
   int run = 0, hits_to_end = 0;
   // the recorded ballots, one store by the first lane per step (holding
   // them in the lanes until 64 are stored together costs the walk more)
@@ -509,7 +530,7 @@ __device__ __forceinline__ void count_block(
   if (lds_hist != nullptr) {
     // the certain hits: each row of the splat's inner rectangle, cut where
     // the digit changes
-    if (lane < kWalkSplats && n_inner > 0) {
+    if (lane < kS && n_inner > 0) {
       const int4 in = W.inner[lane];
       const int4 bx = W.box[lane];
       for (int r = 0; r < in.w; ++r) {
@@ -556,8 +577,8 @@ __global__ __launch_bounds__(kThreads) void count_kernel(
     int32_t* __restrict__ splat_count, int32_t* __restrict__ block_sums,
     uint32_t* __restrict__ zero_words, int64_t n_zero_words,
     uint64_t* __restrict__ hit_bits) {
-  __shared__ CountLds<kWaves> S;
-  count_block<kWaves>(P, means2d, conics, opacities, colors, rec_orig,
+  __shared__ CountLds<kWaves, kWalkSplats> S;
+  count_block<kWaves, kWalkSplats>(P, means2d, conics, opacities, colors, rec_orig,
                       splat_count, block_sums, zero_words, n_zero_words,
                       (int)blockIdx.x, (int)gridDim.x, S, nullptr, nullptr, 0,
                       hit_bits);
@@ -567,18 +588,20 @@ __global__ __launch_bounds__(kThreads) void count_kernel(
 // launch: workgroups below run_blocks sort one depth run each (a few CUs for
 // most of the launch), the others are count blocks of kRunWaves wavefronts
 // and fill the remaining CUs.  The two parts touch disjoint memory.
+template <int kS>
 union CountRunsLds {
   run_step::RunSortLds runs;
-  CountLds<run_step::kRunWaves> count;
+  CountLds<run_step::kRunWaves, kS> count;
 };
 
+template <int kS>
 __global__ __launch_bounds__(run_step::kRunThreads) void count_depth_runs_kernel(
     RasterParams P, const float* __restrict__ means2d,
     const float* __restrict__ conics, const float* __restrict__ opacities,
     int32_t* __restrict__ splat_count, uint32_t* __restrict__ zero_words,
     int64_t n_zero_words, const float* __restrict__ depths, int runs,
     int run_blocks, run_step::RunBuffers runs_out, CountHist H) {
-  __shared__ CountRunsLds S;
+  __shared__ CountRunsLds<kS> S;
   __shared__ uint32_t hist[2 * 257];
   if ((int)blockIdx.x < run_blocks) {
     run_step::run_sort_block(depths, P.gpb, runs, (int)blockIdx.x, runs_out,
@@ -586,7 +609,7 @@ __global__ __launch_bounds__(run_step::kRunThreads) void count_depth_runs_kernel
     return;
   }
   const int vb = (int)blockIdx.x - run_blocks;
-  count_block<run_step::kRunWaves>(
+  count_block<run_step::kRunWaves, kS>(
       P, means2d, conics, opacities, nullptr, nullptr, splat_count, nullptr,
       zero_words, n_zero_words, vb, (int)gridDim.x - run_blocks, S.count,
       H.parts != nullptr ? hist : nullptr,
@@ -627,7 +650,7 @@ __global__ __launch_bounds__(kThreads) void sum_kernel(
 // emit_kernel<true>).
 // Emit workgroups whose totals a rank_pack workgroup adds in LDS first (its
 // 256 gids are increasing and usually span a few dozen of them).
-constexpr int kAggBlocks = 128;
+constexpr int kAggBlocks = 512;
 
 __global__ __launch_bounds__(run_step::kRankBlock) void rank_pack_kernel(
     RasterParams P, const float* __restrict__ means2d,
@@ -636,7 +659,7 @@ __global__ __launch_bounds__(run_step::kRankBlock) void rank_pack_kernel(
     int runs, const int32_t* __restrict__ splat_count,
     int32_t* __restrict__ perm, float4* __restrict__ packed,
     int32_t* __restrict__ gid_count, uint32_t* __restrict__ block_totals,
-    CountHist H) {
+    int emit_splats, CountHist H) {
   __shared__ run_step::RankLds S;
   __shared__ uint32_t agg[kAggBlocks];
   __shared__ int agg_first;
@@ -685,11 +708,11 @@ __global__ __launch_bounds__(run_step::kRankBlock) void rank_pack_kernel(
   // workgroups start from these): the chunk's element 0 has its smallest
   // gid, so workgroups first .. first + kAggBlocks - 1 are summed in LDS,
   // any further one directly.
-  if (t == 0) agg_first = my_gid / kWalkBlockSplats;
+  if (t == 0) agg_first = my_gid / emit_splats;
   __syncthreads();
   const int first = agg_first;
   if (my_gid >= 0 && my_n != 0) {
-    const int wb = my_gid / kWalkBlockSplats;
+    const int wb = my_gid / emit_splats;
     if (wb - first < kAggBlocks)
       atomicAdd(&agg[wb - first], (uint32_t)my_n);
     else
@@ -730,7 +753,8 @@ __global__ __launch_bounds__(kThreads) void pack_kernel(
         r.v[k] = rec_orig[(int64_t)kRecordVec4 * orig + k];
       const uint32_t slot = __float_as_uint(r.v[2].y);
       n = (int)(slot & 0x7fffffffu);
-      r.v[2].y = __uint_as_float((uint32_t)orig | (slot & 0x80000000u));
+      const int source = P.orig_map != nullptr ? P.orig_map[orig] : orig;
+      r.v[2].y = __uint_as_float((uint32_t)source | (slot & 0x80000000u));
       store_record(packed, gid, r);
     } else {
       pack_record(P, means2d, conics, colors, opacities, packed, gid, orig);
@@ -836,7 +860,7 @@ __device__ __forceinline__ void put_pair(uint32_t* __restrict__ keys,
 // start at eo.slot[orig].x, its certain hits first, then its walk hits,
 // numbered by the wavefront's walk hits of the splats before it (its count
 // less its certain hits).
-template <bool kScan, bool kOrig>
+template <bool kScan, bool kOrig, int kS>
 __global__ __launch_bounds__(kThreads) void emit_kernel(
     RasterParams P, const float4* __restrict__ packed,
     const int32_t* __restrict__ splat_offsets, int64_t capacity,
@@ -846,12 +870,12 @@ __global__ __launch_bounds__(kThreads) void emit_kernel(
     uint32_t* ghist_direct, uint32_t* pair_status, int64_t pair_status_words,
     EmitScan sc, EmitOrig eo) {
   static_assert(!(kScan && kOrig), "one source of offsets");
-  __shared__ WalkSlots walk[kWaves];
-  __shared__ int base[kWaves][kWalkSplats];
+  __shared__ WalkSlots<kS> walk[kWaves];
+  __shared__ int base[kWaves][kS];
   // kOrig: per splat the first position of its walk hits less the wave's
   // walk hits before it, and its gid
-  __shared__ int wbase[kOrig ? kWaves : 1][kWalkSplats];
-  __shared__ int wgid[kOrig ? kWaves : 1][kWalkSplats];
+  __shared__ int wbase[kOrig ? kWaves : 1][kS];
+  __shared__ int wgid[kOrig ? kWaves : 1][kS];
   // the pair sort's digit histograms in kHistCopies copies (lane l adds to
   // copy l % kHistCopies; rows 257 words apart, so that one digit's copies
   // lie in different LDS banks): hits of one tile row share the row's
@@ -869,14 +893,14 @@ __global__ __launch_bounds__(kThreads) void emit_kernel(
   __syncthreads();
   // (2) pair emission (gid: the splat's index in the walk's order, its
   // original index with kOrig)
-  const int gid = (vb * kWaves + wave) * kWalkSplats + lane;
-  const bool valid = lane < kWalkSplats && gid < P.num_splats;
+  const int gid = (vb * kWaves + wave) * kS + lane;
+  const bool valid = lane < kS && gid < P.num_splats;
   const int g = valid ? gid : P.num_splats - 1;
   const float4* __restrict__ src = kOrig ? eo.rec : packed;
   const float4 p0 = src[kRecordVec4 * (int64_t)g + 0];
   const float4 p1 = src[kRecordVec4 * (int64_t)g + 1];
   const SplatGeom s{p0.x, p0.y, p0.z, p0.w, p1.x, p1.y};
-  WalkSlots& W = walk[wave];
+  WalkSlots<kS>& W = walk[wave];
   int64_t n_eff;
   int total, n_inner;
   if (kScan) {
@@ -888,12 +912,13 @@ __global__ __launch_bounds__(kThreads) void emit_kernel(
     for (int j = t; j < vb; j += kThreads) before += sc.block_totals[j];
     int inc = n;
 #pragma unroll
-    for (int off = 1; off < kWalkSplats; off <<= 1) {
+    for (int off = 1; off < kS; off <<= 1) {
       const int y = __shfl_up(inc, off, 64);
       if (lane >= off) inc += y;
     }
-    if (lane == kWalkSplats - 1) wsum[wave] = inc;
-    total = walk_setup(P, valid, s, g / P.gpb, W, n_inner);
+    if (lane == kS - 1) wsum[wave] = inc;
+    total = walk_setup(P, valid, s, g / P.gpb,
+                       P.live != nullptr ? source_of(src, g) : 0, W, n_inner);
 #pragma unroll
     for (int off = 32; off > 0; off >>= 1) before += __shfl_xor(before, off, 64);
     if (lane == 0) wbefore[wave] = before;
@@ -922,24 +947,26 @@ __global__ __launch_bounds__(kThreads) void emit_kernel(
               : 0;
     const int2 sg = valid ? eo.slot[g] : make_int2(0, 0);
     n_eff = min(capacity, (int64_t)max(splat_offsets[P.num_splats], 0));
-    total = walk_setup(P, valid, s, g / P.gpb, W, n_inner);
+    total = walk_setup(P, valid, s, g / P.gpb,
+                       P.orig_map != nullptr ? P.orig_map[g] : g, W, n_inner);
     // walk hits of the wavefront's splats up to this one
     const int w = n - n_inner;
     int inc = w;
 #pragma unroll
-    for (int off = 1; off < kWalkSplats; off <<= 1) {
+    for (int off = 1; off < kS; off <<= 1) {
       const int y = __shfl_up(inc, off, 64);
       if (lane >= off) inc += y;
     }
-    if (lane < kWalkSplats) {
+    if (lane < kS) {
       base[wave][lane] = sg.x;
       wbase[kOrig ? wave : 0][lane] = sg.x + n_inner - (inc - w);
       wgid[kOrig ? wave : 0][lane] = sg.y;
     }
   } else {
-    if (lane < kWalkSplats) base[wave][lane] = splat_offsets[g];
+    if (lane < kS) base[wave][lane] = splat_offsets[g];
     n_eff = min(capacity, (int64_t)max(splat_offsets[P.num_splats], 0));
-    total = walk_setup(P, valid, s, g / P.gpb, W, n_inner);
+    total = walk_setup(P, valid, s, g / P.gpb,
+                       P.live != nullptr ? source_of(src, g) : 0, W, n_inner);
   }
   const int gid0 = gid - lane;
   // The wavefront's splats own consecutive ranges starting at the first
@@ -975,7 +1002,7 @@ __global__ __launch_bounds__(kThreads) void emit_kernel(
     }
   });
   // The certain hits of each splat, row by row at the start of its range.
-  uint64_t with_inner = __ballot(lane < kWalkSplats && n_inner > 0);
+  uint64_t with_inner = __ballot(lane < kS && n_inner > 0);
   for (; with_inner != 0ull; with_inner &= with_inner - 1ull) {
     const int sl = (int)__builtin_ctzll(with_inner);
     const int4 in = W.inner[sl];
@@ -1422,25 +1449,43 @@ int launch_count(const RasterParams& P, const float* means2d,
   return check_launch("sum_kernel");
 }
 
-int count_depth_runs_blocks(const RasterParams& P) {
-  constexpr int kSplatsPerBlock = run_step::kRunWaves * kWalkSplats;
-  return (P.num_splats + kSplatsPerBlock - 1) / kSplatsPerBlock;
+// Splats of many tiles each: a wavefront of 32 of them walks for long while
+// few wavefronts run (two images of 100K 3D splats at 35 pairs per splat:
+// emit 80 us with 32, 68 with 16), and with few splats in all fewer per
+// wavefront only fill the chip (512 splats: emit 8.5 us with 32, 6.6 with
+// 16).  64K splats of 5 to 13 pairs are as fast or faster with 32 (their
+// rank launch adds to more totals otherwise, 15 against 22 us).
+constexpr int kFewSplatPairs = 24;
+constexpr int kFewSplats = 1 << 14;
+
+int walk_splats(const RasterParams& P, int64_t capacity) {
+  if (capacity >= (int64_t)kFewSplatPairs * P.num_splats)
+    return P.num_splats <= kWaves * 8 * kScanEmitMaxBlocks ? 8 : 16;
+  return P.num_splats <= kFewSplats ? 16 : kWalkSplats;
+}
+
+int count_depth_runs_blocks(const RasterParams& P, int walk) {
+  const int per_block = run_step::kRunWaves * walk;
+  return (P.num_splats + per_block - 1) / per_block;
 }
 
 int launch_count_depth_runs(const RasterParams& P, const float* means2d,
                             const float* conics, const float* opacities,
                             int32_t* splat_count, uint32_t* zero_words,
                             int64_t n_zero_words, const float* depths,
-                            void* depth_buffers, hipStream_t stream,
-                            const CountHist& H) {
+                            void* depth_buffers, int walk,
+                            hipStream_t stream, const CountHist& H) {
   if (P.num_splats == 0 || !depth_small_ok(P.gpb)) {
     set_error("count + depth runs: needs 1..131072 splats per image");
     return GSPLAT_ERR_INVALID_ARGUMENT;
   }
   const int runs = run_step::runs_of(P.gpb);
   const int run_blocks = P.batch * runs;
-  const int cblocks = count_depth_runs_blocks(P);
-  launch_traced("count_depth_runs_kernel", count_depth_runs_kernel,
+  const int cblocks = count_depth_runs_blocks(P, walk);
+  launch_traced("count_depth_runs_kernel",
+                walk == 8    ? count_depth_runs_kernel<8>
+                : walk == 16 ? count_depth_runs_kernel<16>
+                             : count_depth_runs_kernel<kWalkSplats>,
                 dim3((unsigned)(run_blocks + cblocks)),
                 dim3(run_step::kRunThreads), 0, stream, P, means2d, conics,
                 opacities, splat_count, zero_words, n_zero_words, depths, runs,
@@ -1453,7 +1498,7 @@ int launch_rank_pack(const RasterParams& P, const float* means2d,
                      const float* conics, const float* colors,
                      const float* opacities, void* depth_buffers,
                      const int32_t* splat_count, int32_t* perm, float* packed,
-                     int32_t* gid_count, uint32_t* block_totals,
+                     int32_t* gid_count, uint32_t* block_totals, int walk,
                      hipStream_t stream, const CountHist& H) {
   if (P.num_splats == 0 || !depth_small_ok(P.gpb)) {
     set_error("rank + pack: needs 1..131072 splats per image");
@@ -1468,7 +1513,8 @@ int launch_rank_pack(const RasterParams& P, const float* means2d,
                 colors, opacities,
                 run_step::run_buffers(depth_buffers, P.gpb, P.batch),
                 run_step::runs_of(P.gpb), splat_count, perm,
-                reinterpret_cast<float4*>(packed), gid_count, block_totals, H);
+                reinterpret_cast<float4*>(packed), gid_count, block_totals,
+                kWaves * walk, H);
   return check_launch("rank_pack_kernel");
 }
 
@@ -1505,8 +1551,8 @@ int count_scan_blocks(const RasterParams& P) {
   return (P.num_splats + kThreads - 1) / kThreads;
 }
 
-int emit_blocks(const RasterParams& P) {
-  return (P.num_splats + kWalkBlockSplats - 1) / kWalkBlockSplats;
+int emit_blocks(const RasterParams& P, int walk) {
+  return (P.num_splats + kWaves * walk - 1) / (kWaves * walk);
 }
 
 int launch_emit(const RasterParams& P, const float* packed,
@@ -1517,14 +1563,17 @@ int launch_emit(const RasterParams& P, const float* packed,
                 const EmitScanArgs* scan, int hist_shift,
                 uint8_t* key_bytes, const EmitOrigArgs* orig) {
   if (P.num_splats == 0) return GSPLAT_OK;
-  const int nblk = emit_blocks(P);
+  const int nblk = emit_blocks(P, scan != nullptr ? scan->walk : kWalkSplats);
   // Few workgroups add their histograms atomically (pair_ghist is zeroed
   // by count_kernel), which saves the reduction launch; many would contend.
   const bool direct = nblk <= kDirectHistBlocks;
   if (scan != nullptr) {
     const EmitScan sc{scan->gid_count, scan->splat_offsets,
                       scan->block_totals};
-    launch_traced("emit_kernel<true>", emit_kernel<true, false>,
+    launch_traced("emit_kernel<true>",
+                  scan->walk == 8    ? emit_kernel<true, false, 8>
+                  : scan->walk == 16 ? emit_kernel<true, false, 16>
+                                     : emit_kernel<true, false, kWalkSplats>,
                   dim3((unsigned)nblk), dim3(kThreads), 0, stream, P,
                   reinterpret_cast<const float4*>(packed), nullptr, capacity,
                   keys, vals, key_bytes, pair_passes, hist_shift, hist_partials,
@@ -1534,7 +1583,7 @@ int launch_emit(const RasterParams& P, const float* packed,
     const EmitOrig eo{reinterpret_cast<const float4*>(orig->rec_orig),
                       reinterpret_cast<const int2*>(orig->orig_slot),
                       orig->hit_bits};
-    launch_traced("emit_kernel<orig>", emit_kernel<false, true>,
+    launch_traced("emit_kernel<orig>", emit_kernel<false, true, kWalkSplats>,
                   dim3((unsigned)nblk), dim3(kThreads), 0, stream, P,
                   reinterpret_cast<const float4*>(packed), splat_offsets,
                   capacity, keys, vals, key_bytes, pair_passes, hist_shift,
@@ -1542,7 +1591,7 @@ int launch_emit(const RasterParams& P, const float* packed,
                   direct ? pair_ghist : nullptr, pair_status, pair_status_words,
                   EmitScan{}, eo);
   } else {
-    launch_traced("emit_kernel<false>", emit_kernel<false, false>,
+    launch_traced("emit_kernel<false>", emit_kernel<false, false, kWalkSplats>,
                   dim3((unsigned)nblk), dim3(kThreads), 0, stream, P,
                   reinterpret_cast<const float4*>(packed), splat_offsets,
                   capacity, keys, vals, key_bytes, pair_passes, hist_shift,

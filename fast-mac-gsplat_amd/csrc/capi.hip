@@ -140,6 +140,9 @@ int make_params(const gsplat_raster_meta* m, RasterParams& P) {
   P.bg_b = m->background[2];
   P.eps = m->eps;
   P.max_alpha = m->max_alpha;
+  P.orig_map = nullptr;
+  P.live = nullptr;
+  P.boxes = nullptr;
   return GSPLAT_OK;
 }
 
@@ -182,9 +185,10 @@ CountLayout count_layout(const RasterParams& P) {
   L.depth = gs::radix_plan(P.gpb, P.batch, 0, 32);
   size_t off = gs::radix_ctl_bytes(L.depth);
   L.scan_status = off;  // the pack scan's, or the emit scan's in gsplat_hip_bin
-  off += gs::align_up((size_t)std::max(gs::count_scan_blocks(P), gs::emit_blocks(P)) *
-                          sizeof(uint64_t),
-                      256);
+  off += gs::align_up(
+      std::max((size_t)gs::count_scan_blocks(P) * sizeof(uint64_t),
+               (size_t)gs::emit_blocks(P, 8) * sizeof(uint32_t)),
+      256);
   L.scan_ticket = off;
   off += 256;
   L.pair_ghist = off;
@@ -236,7 +240,9 @@ EmitLayout emit_layout(const RasterParams& P, int64_t n) {
   L.status = off;
   off += gs::align_up((size_t)L.pairs.status_words * sizeof(uint32_t), 256);
   L.hist = off;
-  off += gs::align_up((size_t)gs::emit_blocks(P) * 4 * 256 * sizeof(uint32_t), 256);
+  off += gs::align_up((size_t)gs::emit_blocks(P, gs::walk_splats(P, n)) * 4 *
+                          256 * sizeof(uint32_t),
+                      256);
   L.sorted_keys = off;
   off += vec;
   L.buffers = off;
@@ -304,6 +310,23 @@ int gsplat_hip_time_next_launch(int which, void* start_event,
 }  // extern "C"
 
 namespace {
+// The splats of a slice (slice.hip): what RasterParams holds beside the meta.
+struct SliceView {
+  const int32_t* orig_map;
+  const uint32_t* live;
+  const uint2* boxes;
+};
+int make_view_params(const gsplat_raster_meta* meta, const SliceView* view,
+                     RasterParams& P) {
+  const int rc = make_params(meta, P);
+  if (!rc && view != nullptr) {
+    P.orig_map = view->orig_map;
+    P.live = view->live;
+    P.boxes = view->boxes;
+  }
+  return rc;
+}
+
 // gsplat_hip_bin_count; with colors the count also writes the
 // original-order records that bin_pack_impl copies (use_records).  A null
 // pair_count skips the total (the one-call binning reports N from the pack
@@ -311,9 +334,10 @@ namespace {
 int bin_count_impl(const gsplat_raster_meta* meta, const float* means2d,
                    const float* conics, const float* opacities,
                    const float* colors, int32_t* pair_count, void* workspace,
-                   size_t workspace_bytes, void* stream) {
+                   size_t workspace_bytes, void* stream,
+                   const SliceView* view = nullptr) {
   RasterParams P;
-  int rc = make_params(meta, P);
+  int rc = make_view_params(meta, view, P);
   if (rc) return rc;
   rc = null_check({means2d, conics, opacities, workspace},
                   "gsplat_hip_bin_count");
@@ -423,9 +447,10 @@ int bin_pack_impl(const gsplat_raster_meta* meta, const float* means2d,
                   const float* conics, const float* colors,
                   const float* opacities, const int32_t* perm, float* packed,
                   int32_t* splat_offsets, void* workspace,
-                  size_t workspace_bytes, void* stream, bool use_records) {
+                  size_t workspace_bytes, void* stream, bool use_records,
+                  const SliceView* view = nullptr) {
   RasterParams P;
-  int rc = make_params(meta, P);
+  int rc = make_view_params(meta, view, P);
   if (rc) return rc;
   rc = null_check({means2d, conics, colors, opacities, perm, packed,
                    splat_offsets, workspace},
@@ -511,9 +536,10 @@ int bin_emit_impl(const gsplat_raster_meta* meta, const float* packed,
                   void* workspace, size_t workspace_bytes, void* stream,
                   int32_t* long_flag, const gs::ZeroSpan* zero = nullptr,
                   const gs::EmitScanArgs* scan = nullptr,
-                  bool hist_counted = false, bool orig_walk = false) {
+                  bool hist_counted = false, bool orig_walk = false,
+                  const SliceView* view = nullptr) {
   RasterParams P;
-  int rc = make_params(meta, P);
+  int rc = make_view_params(meta, view, P);
   if (rc) return rc;
   if (n_pairs < 0 || n_pairs > 0x7fffffffLL) {
     gs::set_error("gsplat_hip_bin_emit: invalid pair count %lld",
@@ -686,11 +712,6 @@ size_t gsplat_hip_bin_workspace_bytes(const gsplat_raster_meta* meta,
 }  // extern "C"
 
 namespace {
-// Largest number of emit workgroups (128 splats each) of the small-image
-// one-call binning: 4096 (524,288 splats in the batch), where an emit
-// workgroup adds at most 4096 totals (16 per thread).
-constexpr int kScanEmitMaxBlocks = 4096;
-
 // gsplat_hip_bin; zero (may be null): two spans that the tile-range launch
 // zeroes on the side (or a launch of their own where it does not run).
 // With report_out the report of host_words is left to the caller's next
@@ -703,9 +724,10 @@ int bin_impl(const gsplat_raster_meta* meta, const float* means2d,
              int32_t* tile_offsets, int32_t* host_words, void* workspace,
              size_t workspace_bytes, void* stream, void* count_stream,
              void* inputs_event, void* count_event, void* status_event,
-             const gs::ZeroSpan* zero, gs::HostReport* report_out) {
+             const gs::ZeroSpan* zero, gs::HostReport* report_out,
+             const SliceView* view = nullptr) {
   RasterParams P;
-  int rc = make_params(meta, P);
+  int rc = make_view_params(meta, view, P);
   if (rc) return rc;
   if (capacity < 0 || capacity > 0x7fffffffLL) {
     gs::set_error("gsplat_hip_bin: invalid capacity %lld", (long long)capacity);
@@ -766,9 +788,10 @@ int bin_impl(const gsplat_raster_meta* meta, const float* means2d,
   // all workgroups before it, work that grows with the square of their
   // count, so batches of more than kScanEmitMaxBlocks emit workgroups take
   // the look-back path below.
+  const int walk = gs::walk_splats(P, capacity);
   if (host_words != nullptr && capacity > 0 && P.num_tiles > 0 &&
       P.num_splats > 0 && gs::depth_small_ok(P.gpb) &&
-      gs::emit_blocks(P) <= kScanEmitMaxBlocks) {
+      gs::emit_blocks(P, walk) <= gs::kScanEmitMaxBlocks) {
     const CountLayout C = count_layout(P);
     char* cb = static_cast<char*>(cws);
     const size_t z0 = gs::radix_ctl_bytes(C.depth);
@@ -782,7 +805,7 @@ int bin_impl(const gsplat_raster_meta* meta, const float* means2d,
       hist.parts = reinterpret_cast<uint32_t*>(static_cast<char*>(ews) +
                                                emit_layout(P, capacity).hist);
       hist.shift = low_bits;
-      hist.nparts = gs::count_depth_runs_blocks(P);
+      hist.nparts = gs::count_depth_runs_blocks(P, walk);
       hist.ghist = reinterpret_cast<uint32_t*>(cb + C.pair_ghist);
     }
     rc = gs::launch_count_depth_runs(
@@ -790,7 +813,7 @@ int bin_impl(const gsplat_raster_meta* meta, const float* means2d,
         reinterpret_cast<int32_t*>(cb + C.splat_count),
         reinterpret_cast<uint32_t*>(cb + z0),
         (int64_t)((C.ctl_end - z0) / sizeof(uint32_t)), depths,
-        cb + C.depth_buffers, s, hist);
+        cb + C.depth_buffers, walk, s, hist);
     // ranks with the records packed at them, then the emit scans the pair
     // offsets itself
     int32_t* gid_count = reinterpret_cast<int32_t*>(cb + C.gid_count);
@@ -801,12 +824,13 @@ int bin_impl(const gsplat_raster_meta* meta, const float* means2d,
       rc = gs::launch_rank_pack(
           P, means2d, conics, colors, opacities, cb + C.depth_buffers,
           reinterpret_cast<const int32_t*>(cb + C.splat_count), perm, packed,
-          gid_count, block_totals, s, hist);
-    const gs::EmitScanArgs scan{gid_count, splat_offsets, block_totals};
+          gid_count, block_totals, walk, s, hist);
+    const gs::EmitScanArgs scan{gid_count, splat_offsets, block_totals, walk};
     if (!rc)
       rc = bin_emit_impl(meta, packed, splat_offsets, capacity, binned_ids,
                          nullptr, tile_offsets, status_dev, cws, cbytes, ews,
-                         ebytes, s, long_dev, zero, &scan, low_bits >= 1);
+                         ebytes, s, long_dev, zero, &scan, low_bits >= 1,
+                         false, view);
     // N is written by the emit's scan
     return rc ? rc : report(splat_offsets + P.num_splats);
   }
@@ -820,7 +844,7 @@ int bin_impl(const gsplat_raster_meta* meta, const float* means2d,
     if (rc) return rc;
   }
   rc = bin_count_impl(meta, means2d, conics, opacities, colors, nullptr, cws,
-                      cbytes, cs);
+                      cbytes, cs, view);
   if (!rc && ev_n != nullptr)
     rc = hip_status(hipEventRecord(ev_n, cs), "gsplat_hip_bin: event record");
   if (rc) return rc;
@@ -835,12 +859,12 @@ int bin_impl(const gsplat_raster_meta* meta, const float* means2d,
   // 3. records and offsets, 4. pairs, pair sort, tile ranges and the
   //    look-back status (next to N in the workspace header)
   rc = bin_pack_impl(meta, means2d, conics, colors, opacities, perm, packed,
-                     splat_offsets, cws, cbytes, s, true);
+                     splat_offsets, cws, cbytes, s, true, view);
   if (rc) return rc;
   rc = bin_emit_impl(meta, packed, splat_offsets, capacity, binned_ids,
                      nullptr, tile_offsets, status_dev, cws, cbytes, ews,
                      ebytes, s, host_words != nullptr ? long_dev : nullptr,
-                     zero, nullptr, false, true);
+                     zero, nullptr, false, true, view);
   if (rc || host_words == nullptr) return rc;
   // 5. N (from the pack scan), the status and the long-range flag to the host
   return report(splat_offsets + P.num_splats);
@@ -1206,6 +1230,331 @@ int gsplat_hip_radix_sort_pairs_u32(const uint32_t* keys_in,
                               n_per_segment, segments, begin_bit, end_bit,
                               workspace, workspace_bytes,
                               static_cast<hipStream_t>(stream), status);
+}
+
+}  // extern "C"
+
+namespace {
+
+// gsplat_slice.splats: the compacted attributes, their original indices and
+// the binning's depth order and pair offsets.
+struct SplatsLayout {
+  size_t means2d, conics, colors, opacities, depths, orig, perm, offsets, total;
+};
+SplatsLayout splats_layout(int64_t n) {
+  SplatsLayout L{};
+  size_t off = 0;
+  auto take = [&](int64_t words) {
+    const size_t at = off;
+    off += gs::align_up((size_t)words * 4, 256);
+    return at;
+  };
+  L.means2d = take(2 * n);
+  L.conics = take(3 * n);
+  L.colors = take(3 * n);
+  L.opacities = take(n);
+  L.depths = take(n);
+  L.orig = take(n);
+  L.perm = take(n);
+  L.offsets = take(n + 1);
+  L.total = off;
+  return L;
+}
+gs::SliceSplats splats_at(const SplatsLayout& L, void* p) {
+  char* b = static_cast<char*>(p);
+  return gs::SliceSplats{reinterpret_cast<float*>(b + L.means2d),
+                         reinterpret_cast<float*>(b + L.conics),
+                         reinterpret_cast<float*>(b + L.colors),
+                         reinterpret_cast<float*>(b + L.opacities),
+                         reinterpret_cast<float*>(b + L.depths),
+                         reinterpret_cast<int32_t*>(b + L.orig)};
+}
+
+// The slicing workspace: what slice.hip shares between the front and the
+// back.  The first ctl_end bytes are zeroed by the front.
+struct SliceLayout {
+  size_t ctl, sums, back_count, hist, status_front, status_back,
+      ctl_end, cross, limit, box, back_list, live_bits, tile_live, total;
+};
+SliceLayout slice_layout(const RasterParams& P) {
+  SliceLayout L{};
+  size_t off = 0;
+  auto take = [&](size_t bytes) {
+    const size_t at = off;
+    off += gs::align_up(bytes, 256);
+    return at;
+  };
+  const size_t B = (size_t)P.batch;
+  L.ctl = take(8 * 4);
+  L.sums = take(gs::kSliceSums * 8);
+  L.back_count = take(B * 4);
+  L.hist = take(2 * B * gs::kSliceBins * 8);
+  L.status_front = take((size_t)gs::slice_status_words(P) * 8);
+  L.status_back = take((size_t)gs::slice_status_words(P) * 8);
+  L.ctl_end = off;
+  L.cross = take(B * sizeof(gs::SliceCrossing));
+  L.limit = take(B * 4);
+  L.box = take((size_t)P.num_splats * 8);
+  L.back_list = take((size_t)P.num_splats * 4);
+  L.live_bits = take(((size_t)P.num_tiles / 32 + 2) * 4);
+  L.tile_live = take((size_t)P.num_tiles * 4);
+  L.total = off;
+  return L;
+}
+gs::SliceBuffers slice_at(const SliceLayout& L, void* p, int32_t* live_list,
+                          const gs::SliceSplats& front) {
+  char* b = static_cast<char*>(p);
+  gs::SliceBuffers Q{};
+  Q.ctl = reinterpret_cast<uint32_t*>(b + L.ctl);
+  Q.sums = reinterpret_cast<unsigned long long*>(b + L.sums);
+  Q.back_count = reinterpret_cast<uint32_t*>(b + L.back_count);
+  Q.hist = reinterpret_cast<unsigned long long*>(b + L.hist);
+  Q.status_front = reinterpret_cast<uint64_t*>(b + L.status_front);
+  Q.status_back = reinterpret_cast<uint64_t*>(b + L.status_back);
+  Q.cross = reinterpret_cast<gs::SliceCrossing*>(b + L.cross);
+  Q.limit = reinterpret_cast<uint32_t*>(b + L.limit);
+  Q.box = reinterpret_cast<uint2*>(b + L.box);
+  Q.back_list = reinterpret_cast<int32_t*>(b + L.back_list);
+  Q.live_bits = reinterpret_cast<uint32_t*>(b + L.live_bits);
+  Q.live_list = live_list;
+  Q.front = front;
+  return Q;
+}
+
+// Checks of a slice against the scene's parameters; PS: the slice's own.
+int slice_params(const gsplat_raster_meta* meta, const gsplat_slice* slice,
+                 const char* what, bool training, RasterParams& P,
+                 gsplat_raster_meta& ms, RasterParams& PS) {
+  int rc = make_params(meta, P);
+  if (rc) return rc;
+  rc = null_check({slice}, what);
+  if (rc) return rc;
+  if (!gs::slice_ok(P)) {
+    gs::set_error("%s: needs at most 64 images of at most 2^18 tiles "
+                  "and fewer than 2^22 splats", what);
+    return GSPLAT_ERR_INVALID_ARGUMENT;
+  }
+  ms = *meta;
+  ms.gaussians_per_batch = slice->slots;
+  rc = make_params(&ms, PS);
+  if (rc) return rc;
+  if (slice->capacity <= 0 || slice->capacity > 0x7fffffffLL ||
+      !gs::radix_size_ok(slice->capacity, 1)) {
+    gs::set_error("%s: invalid capacity %lld", what,
+                  (long long)slice->capacity);
+    return GSPLAT_ERR_INVALID_ARGUMENT;
+  }
+  rc = null_check({slice->packed, slice->binned_ids, slice->tile_offsets,
+                   slice->tile_stop, slice->render_workspace},
+                  what);
+  if (rc) return rc;
+  if (slice->render_workspace_bytes <
+      gs::render_workspace_bytes(PS, training ? slice->capacity : 0)) {
+    gs::set_error("%s: render workspace too small", what);
+    return GSPLAT_ERR_WORKSPACE;
+  }
+  return GSPLAT_OK;
+}
+
+// The slice's binning and forward on compacted splats C; with acc the
+// tile-range launch zeroes the scene's gradient records.
+int slice_render(const gsplat_raster_meta& ms, const RasterParams& PS,
+                 const gsplat_slice* slice, const gs::SliceSplats& C,
+                 const SliceView& view, const SplatsLayout& SL, float* out_rgb,
+                 float* out_T, int32_t* out_last, const gs::ZeroSpan& acc,
+                 int32_t* host_words, void* stream, void* count_stream,
+                 void* inputs_event, void* count_event,
+                 const gs::TileSet& tiles, gs::HostReport* report,
+                 bool report_now) {
+  char* b = static_cast<char*>(slice->splats);
+  gs::ZeroSpan zero[2];
+  gs::render_forward_zero_spans(PS, slice->capacity, slice->render_workspace,
+                                out_T != nullptr, zero);
+  zero[1] = acc;
+  int rc = bin_impl(
+      &ms, C.means2d, C.conics, C.colors, C.opacities, C.depths,
+      slice->capacity, reinterpret_cast<int32_t*>(b + SL.perm), slice->packed,
+      reinterpret_cast<int32_t*>(b + SL.offsets), slice->binned_ids,
+      slice->tile_offsets, host_words, slice->bin_workspace,
+      slice->bin_workspace_bytes, stream, count_stream, inputs_event,
+      count_event, nullptr, zero, report, &view);
+  if (rc) return rc;
+  return gs::launch_render_forward(
+      PS, slice->packed, slice->tile_offsets, slice->binned_ids, out_rgb, out_T,
+      out_last, slice->tile_stop, slice->capacity, slice->render_workspace,
+      static_cast<hipStream_t>(stream),
+      gs::kForwardPreZeroed | gs::kForwardStoppedLast,
+      report_now ? report : nullptr, &tiles);
+}
+
+}  // namespace
+
+extern "C" {
+
+size_t gsplat_hip_slice_workspace_bytes(const gsplat_raster_meta* meta) {
+  RasterParams P;
+  if (make_params(meta, P) || !gs::slice_ok(P)) return 0;
+  return slice_layout(P).total;
+}
+
+size_t gsplat_hip_slice_splats_bytes(int32_t batch, int32_t slots) {
+  if (batch <= 0 || slots <= 0) return 0;
+  return splats_layout((int64_t)batch * slots).total;
+}
+
+int gsplat_hip_front_render(const gsplat_raster_meta* meta,
+                            const float* means2d, const float* conics,
+                            const float* colors, const float* opacities,
+                            const float* depths, const gsplat_slice* front,
+                            float* out_rgb, float* out_final_T,
+                            int32_t* out_last, float* grad_records,
+                            int32_t* live_list, void* workspace,
+                            size_t workspace_bytes, int32_t* host_words,
+                            void* stream) {
+  const char* what = "gsplat_hip_front_render";
+  RasterParams P, PS;
+  gsplat_raster_meta ms;
+  const bool training = out_final_T != nullptr;
+  int rc = slice_params(meta, front, what, training, P, ms, PS);
+  if (!rc)
+    rc = null_check({means2d, conics, colors, opacities, depths, front->splats,
+                     front->bin_workspace, out_rgb, live_list, workspace,
+                     host_words},
+                    what);
+  if (rc) return rc;
+  if (training != (out_last != nullptr) || training != (grad_records != nullptr)) {
+    gs::set_error("%s: out_final_T, out_last and grad_records must all be "
+                  "given or all be NULL", what);
+    return GSPLAT_ERR_INVALID_ARGUMENT;
+  }
+  const SliceLayout L = slice_layout(P);
+  const SplatsLayout SL = splats_layout(PS.num_splats);
+  if (workspace_bytes < L.total || front->splats_bytes < SL.total) {
+    gs::set_error("%s: workspace too small", what);
+    return GSPLAT_ERR_WORKSPACE;
+  }
+  hipStream_t s = static_cast<hipStream_t>(stream);
+  const gs::SliceSplats C = splats_at(SL, front->splats);
+  const gs::SliceBuffers Q = slice_at(L, workspace, live_list, C);
+  uint32_t* tile_live = reinterpret_cast<uint32_t*>(
+      static_cast<char*>(workspace) + L.tile_live);
+  for (int k = 0; k < 16; ++k) host_words[k] = 0;
+  rc = gs::launch_zero_u32(static_cast<uint32_t*>(workspace),
+                           (int64_t)(L.ctl_end / 4), s);
+  if (!rc)
+    rc = gs::launch_slice_front(P, Q, means2d, conics, colors, opacities,
+                                depths, front->slots,
+                                front->capacity / P.batch, s);
+  gs::HostReport report{};
+  const SliceView view{C.orig, nullptr, nullptr};
+  const gs::ZeroSpan acc{reinterpret_cast<uint32_t*>(grad_records),
+                         training ? (int64_t)P.num_splats *
+                                        GSPLAT_GRAD_RECORD_FLOATS
+                                  : 0};
+  if (!rc)
+    rc = slice_render(ms, PS, front, C, view, SL, out_rgb, out_final_T,
+                      out_last, acc, host_words, stream, nullptr, nullptr,
+                      nullptr, gs::TileSet{nullptr, 0, tile_live}, &report,
+                      false);
+  if (!rc)
+    rc = gs::launch_slice_back(P, Q, depths, tile_live, front->tile_stop,
+                               report.status, host_words, s);
+  return rc;
+}
+
+int gsplat_hip_back_render(const gsplat_raster_meta* meta,
+                           const float* means2d, const float* conics,
+                           const float* colors, const float* opacities,
+                           const float* depths, const gsplat_slice* back,
+                           float* out_rgb, float* out_final_T,
+                           int32_t* out_last, int32_t* live_list,
+                           int32_t n_live, void* workspace,
+                           size_t workspace_bytes, int32_t* host_words,
+                           void* stream, void* count_stream,
+                           void* inputs_event, void* count_event) {
+  const char* what = "gsplat_hip_back_render";
+  RasterParams P, PS;
+  gsplat_raster_meta ms;
+  int rc = slice_params(meta, back, what, out_final_T != nullptr, P, ms, PS);
+  if (!rc)
+    rc = null_check({means2d, conics, colors, opacities, depths, back->splats,
+                     back->bin_workspace, out_rgb, live_list, workspace,
+                     host_words},
+                    what);
+  if (rc) return rc;
+  if ((out_final_T == nullptr) != (out_last == nullptr)) {
+    gs::set_error("%s: out_final_T and out_last must both be given or both "
+                  "be NULL", what);
+    return GSPLAT_ERR_INVALID_ARGUMENT;
+  }
+  if (n_live <= 0 || n_live > P.num_tiles) {
+    gs::set_error("%s: invalid number of tiles %d", what, (int)n_live);
+    return GSPLAT_ERR_INVALID_ARGUMENT;
+  }
+  const SliceLayout L = slice_layout(P);
+  const SplatsLayout SL = splats_layout(PS.num_splats);
+  if (workspace_bytes < L.total || back->splats_bytes < SL.total) {
+    gs::set_error("%s: workspace too small", what);
+    return GSPLAT_ERR_WORKSPACE;
+  }
+  const gs::SliceSplats C = splats_at(SL, back->splats);
+  const gs::SliceBuffers Q = slice_at(L, workspace, live_list, gs::SliceSplats{});
+  rc = gs::launch_slice_gather(P, Q, C, back->slots, means2d, conics, colors,
+                               opacities, depths,
+                               static_cast<hipStream_t>(stream));
+  gs::HostReport report{};
+  const SliceView view{C.orig, Q.live_bits, Q.box};
+  if (!rc)
+    rc = slice_render(ms, PS, back, C, view, SL, out_rgb, out_final_T, out_last,
+                      gs::ZeroSpan{nullptr, 0}, host_words, stream,
+                      count_stream, inputs_event, count_event,
+                      gs::TileSet{live_list, n_live, nullptr}, &report, true);
+  return rc;
+}
+
+int gsplat_hip_sliced_backward(const gsplat_raster_meta* meta,
+                               const gsplat_slice* front,
+                               const gsplat_slice* back,
+                               const int32_t* live_list, int32_t n_live,
+                               const float* final_T, const int32_t* last,
+                               const float* grad_rgb, float* grad_records,
+                               float* g_means2d, float* g_conics,
+                               float* g_colors, float* g_opacities,
+                               void* stream) {
+  const char* what = "gsplat_hip_sliced_backward";
+  RasterParams P, PS;
+  gsplat_raster_meta ms;
+  int rc = slice_params(meta, front, what, true, P, ms, PS);
+  if (!rc)
+    rc = null_check({final_T, last, grad_rgb, grad_records, g_means2d, g_conics,
+                     g_colors, g_opacities},
+                    what);
+  if (rc) return rc;
+  RasterParams PB{};
+  if (back != nullptr) {
+    rc = slice_params(meta, back, what, true, P, ms, PB);
+    if (!rc) rc = null_check({live_list}, what);
+    if (rc) return rc;
+    if (n_live <= 0 || n_live > P.num_tiles) {
+      gs::set_error("%s: invalid number of tiles %d", what, (int)n_live);
+      return GSPLAT_ERR_INVALID_ARGUMENT;
+    }
+  }
+  hipStream_t s = static_cast<hipStream_t>(stream);
+  auto slice_of = [](const RasterParams& Q, const gsplat_slice* S) {
+    return gs::BackwardSlice{Q,            S->packed,    S->tile_offsets,
+                             S->binned_ids, S->tile_stop, S->capacity,
+                             S->render_workspace};
+  };
+  rc = gs::launch_sliced_backward(
+      slice_of(PS, front),
+      back != nullptr ? slice_of(PB, back) : gs::BackwardSlice{},
+      gs::TileSet{live_list, back != nullptr ? n_live : 0, nullptr}, final_T,
+      last, grad_rgb, grad_records, s);
+  if (!rc)
+    rc = gs::launch_grads_unpack(grad_records, g_means2d, g_conics, g_colors,
+                                 g_opacities, P.num_splats, s);
+  return rc;
 }
 
 }  // extern "C"

@@ -88,8 +88,11 @@ __device__ __forceinline__ TileCoord tile_coord_of(const RasterParams& P,
   return c;
 }
 
-__device__ __forceinline__ TileCoord tile_coord(const RasterParams& P) {
-  return tile_coord_of(P, xcd_remap((int)blockIdx.x, P.num_tiles));
+// (one workgroup per tile of the list, or per tile of the images)
+__device__ __forceinline__ TileCoord tile_coord(const RasterParams& P,
+                                                const int32_t* list) {
+  const int i = xcd_remap((int)blockIdx.x, (int)gridDim.x);
+  return tile_coord_of(P, list != nullptr ? list[i] : i);
 }
 
 __device__ __forceinline__ int slot_y(const TileCoord& c, int k) {
@@ -471,12 +474,12 @@ void render_fwd_kernel(
     const int32_t* __restrict__ binned, float* __restrict__ out_rgb,
     float* __restrict__ out_T, int32_t* __restrict__ out_last,
     int32_t* __restrict__ out_tile_stop, HeavyState H, HostReport R,
-    bool all_last) {
+    bool all_last, TileSet tiles) {
   __shared__ Staged S;
   // The binning's report reaches the host as the forward starts.
   if (R.host != nullptr && blockIdx.x == 0 && threadIdx.x == 0)
     write_host_report(R);
-  const TileCoord tc = tile_coord(P);
+  const TileCoord tc = tile_coord(P, tiles.list);
   const int x = tc.x0 + tc.lx;
   const float px = (float)x + 0.5f;
   // A pixel is alive while T > transmittance_threshold (< 1, checked on the
@@ -560,6 +563,7 @@ void render_fwd_kernel(
       if (threadIdx.x == 0) {
         H.handoff[item] = tc.tile;
         H.handoff_tail[item] = tail;
+        if (tiles.live != nullptr) tiles.live[tc.tile] = 0u;
       }
       return;
     }
@@ -581,6 +585,12 @@ void render_fwd_kernel(
 #pragma unroll
   for (int k = 0; k < kPix; ++k) stop |= valid[k] && !(T[k] > t_thr);
   const bool put_last = all_last || __builtin_amdgcn_ballot_w64(stop) != 0;
+  if (tiles.live != nullptr) {  // (pixels outside the image hold T = 0)
+    const bool alive = (T[0] > t_thr) | (T[1] > t_thr) | (T[2] > t_thr) |
+                       (T[3] > t_thr);
+    const bool any = __builtin_amdgcn_ballot_w64(alive) != 0;
+    if (threadIdx.x == 0) tiles.live[tc.tile] = any ? 1u : 0u;
+  }
 #pragma unroll
   for (int k = 0; k < kPix; ++k) {
     if (valid[k]) {
@@ -647,7 +657,8 @@ __global__ __launch_bounds__(256 / kSpW) void render_fwd_long_kernel(
     const int32_t* __restrict__ tile_offsets,
     const int32_t* __restrict__ binned, float* __restrict__ out_rgb,
     float* __restrict__ out_T, int32_t* __restrict__ out_last,
-    int32_t* __restrict__ out_tile_stop, HeavyState H) {
+    int32_t* __restrict__ out_tile_stop, HeavyState H,
+    uint32_t* __restrict__ live) {
   __shared__ Staged S;
   __shared__ int sh_slot;
   __shared__ int sh_plain;  // batch_plain of the staged batch
@@ -715,6 +726,12 @@ __global__ __launch_bounds__(256 / kSpW) void render_fwd_long_kernel(
     if (threadIdx.x == 0) sh_slot = next_segment(H, tile, seg_cur, tail);
     __syncthreads();
     last_segment<kSpW>(P, tc, out_rgb, H, sh_slot, valid, cr, cg, cb, T, t0);
+    if (live != nullptr) {
+      bool alive = false;
+#pragma unroll
+      for (int k = 0; k < kSpW; ++k) alive |= T[k] > t_thr;
+      if (__builtin_amdgcn_ballot_w64(alive) != 0 && lane == 0) live[tile] = 1u;
+    }
     int tile_max = 0;
 #pragma unroll
     for (int k = 0; k < kSpW; ++k) {
@@ -803,7 +820,7 @@ __device__ __forceinline__ void wave_lds_sync() {
 // DPP.  LDS accesses issue on their own port, so the reduction costs few
 // vector-ALU slots, the compositor's bound.
 constexpr int kGradQ = 8;
-constexpr int kAccFloats = 16;  // floats per accumulator record (64 bytes)
+constexpr int kAccFloats = GSPLAT_GRAD_RECORD_FLOATS;  // per accumulator record (64 bytes)
 struct BwdShared {
   Staged S;
   float red[kGradQ * kLanes];
@@ -1055,8 +1072,8 @@ __device__ __forceinline__ void bwd_batch(
 template <bool kCheckLast, bool kAcc>
 __device__ __forceinline__ void bwd_walk(
     const RasterParams& P, const float4* __restrict__ packed,
-    const int32_t* __restrict__ binned, int start, int lo, int hi,
-    const TileCoord& tc, BwdShared& SH, BwdPixels& Q, const GradOut& G) {
+    const int32_t* __restrict__ binned, uint32_t max_gid, int start, int lo,
+    int hi, const TileCoord& tc, BwdShared& SH, BwdPixels& Q, const GradOut& G) {
   const GradTarget target = kAcc ? GradTarget{} : grad_target(G);
   const GradTarget opac = kAcc ? GradTarget{} : opac_target(G);
   const float max_alpha = fminf(P.max_alpha, 1.0f);
@@ -1066,7 +1083,7 @@ __device__ __forceinline__ void bwd_walk(
     __syncthreads();
     const uint32_t bmask =
         stage_batch<false>(packed, binned, start + cstart, n, tc,
-                           (uint32_t)P.num_splats - 1u, SH.S);
+                           max_gid, SH.S);
     __syncthreads();
     if (batch_plain(bmask))
       bwd_batch<kCheckLast, true, kAcc>(SH, bmask, n, cstart, max_alpha,
@@ -1139,17 +1156,31 @@ __device__ __forceinline__ bool seg_item(const RasterParams& P,
 // more values spilled) for tiles of few pairs, whose time goes to the
 // per-tile set-up and the loads of the pixel state.  kAcc: G has the
 // gradient records (the workspace path).
+// The grid holds B's work items before A's: the back of a sliced scene, which
+// has few tiles, next to its front (B is empty otherwise).
+struct BwdSource {
+  const float4* packed;
+  const int32_t* tile_offsets;
+  const int32_t* binned;
+  const int32_t* tile_stop;
+  HeavyState H;
+  uint32_t max_gid;
+  const int32_t* list;  // the tiles walked, null: tile i
+  int seg_blocks, tiles;
+};
 template <int kWaves, bool kAcc>
 __global__ __launch_bounds__(kLanes)
 __attribute__((amdgpu_waves_per_eu(kWaves, 8))) void render_bwd_kernel(
-    RasterParams P, const float4* __restrict__ packed,
-    const int32_t* __restrict__ tile_offsets,
-    const int32_t* __restrict__ binned, const float* __restrict__ final_T,
-    const int32_t* __restrict__ last_in, const int32_t* __restrict__ tile_stop,
-    const float* __restrict__ grad_rgb, GradOut G, HeavyState H,
-    int seg_blocks) {
+    RasterParams P, BwdSource A, BwdSource B, int b_blocks,
+    const float* __restrict__ final_T, const int32_t* __restrict__ last_in,
+    const float* __restrict__ grad_rgb, GradOut G) {
   __shared__ BwdShared SH;
-  const int bid = (int)blockIdx.x;
+  const bool in_b = (int)blockIdx.x < b_blocks;
+  const BwdSource& W = in_b ? B : A;
+  const HeavyState& H = W.H;
+  const int32_t* __restrict__ tile_stop = W.tile_stop;
+  const int bid = (int)blockIdx.x - (in_b ? 0 : b_blocks);
+  const int seg_blocks = W.seg_blocks;
   const bool seg = bid < seg_blocks;
   const int m = bid;
   {
@@ -1158,13 +1189,16 @@ __attribute__((amdgpu_waves_per_eu(kWaves, 8))) void render_bwd_kernel(
       if (m >= min(H.counters[0], H.max_slots)) return;
       if (!seg_item(P, H, tile_stop, m, tile, kseg, nseg, lo, hi)) return;
     } else {
-      // seg_blocks is a multiple of 8, so the XCD-aware mapping is kept
-      tile = xcd_remap(bid - seg_blocks, P.num_tiles);
+      // seg_blocks and b_blocks are multiples of 8, so the XCD-aware mapping
+      // is kept
+      if (bid - seg_blocks >= W.tiles) return;
+      tile = xcd_remap(bid - seg_blocks, W.tiles);
+      if (W.list != nullptr) tile = W.list[tile];
       hi = tile_stop[tile];
     }
     // the tile's range start and pixel state are loaded before its stop is
     // waited for (an empty tile's loads are wasted: few tiles are empty)
-    const int start = tile_offsets[tile];
+    const int start = W.tile_offsets[tile];
     const TileCoord tc = tile_coord_of(P, tile);
     BwdPixels Q;
     load_bwd_pixels(P, tc, final_T, last_in, grad_rgb, Q);
@@ -1207,9 +1241,11 @@ __attribute__((amdgpu_waves_per_eu(kWaves, 8))) void render_bwd_kernel(
     // Q.Tc holds T_final, or T at the segment's end for pixels alive past it
     // (T_end > T_final > threshold), so the test sees the final state.
     if (needs_last_test(P, tc, Q))
-      bwd_walk<true, kAcc>(P, packed, binned, start, lo, hi, tc, SH, Q, G);
+      bwd_walk<true, kAcc>(P, W.packed, W.binned, W.max_gid, start, lo, hi, tc,
+                           SH, Q, G);
     else
-      bwd_walk<false, kAcc>(P, packed, binned, start, lo, hi, tc, SH, Q, G);
+      bwd_walk<false, kAcc>(P, W.packed, W.binned, W.max_gid, start, lo, hi,
+                            tc, SH, Q, G);
   }
 }
 
@@ -1315,10 +1351,12 @@ int launch_render_forward(const RasterParams& P, const float* packed,
                           float* out_T, int32_t* out_last,
                           int32_t* out_tile_stop, int64_t n_pairs,
                           void* workspace, hipStream_t stream, int flags,
-                          const HostReport* report) {
+                          const HostReport* report, const TileSet* tiles) {
   hipEvent_t t0 = nullptr, t1 = nullptr;
   take_launch_timing(kTimeForward, t0, t1);
-  if (P.num_tiles == 0)
+  const TileSet set = tiles != nullptr ? *tiles : TileSet{};
+  const int n_tiles = set.list != nullptr ? set.n : P.num_tiles;
+  if (n_tiles == 0)
     return report != nullptr ? launch_host_report(*report, stream) : GSPLAT_OK;
   const HeavyState H = forward_state(P, n_pairs, workspace, out_T);
   const float4* pk = reinterpret_cast<const float4*>(packed);
@@ -1330,16 +1368,16 @@ int launch_render_forward(const RasterParams& P, const float* packed,
   }
   // the continuation follows in this call: it ends the timed span
   const bool more = !(flags & kForwardNoLong) && workspace != nullptr;
-  launch_timed("render_fwd_kernel", render_fwd_kernel, dim3((unsigned)P.num_tiles), dim3(kLanes),
+  launch_timed("render_fwd_kernel", render_fwd_kernel, dim3((unsigned)n_tiles), dim3(kLanes),
                stream, t0, more ? nullptr : t1, P, pk, tile_offsets,
                binned_ids, out_rgb, out_T, out_last, out_tile_stop, H,
                report != nullptr ? *report : HostReport{},
-               !(flags & kForwardStoppedLast));
+               !(flags & kForwardStoppedLast), set);
   const int rc = check_launch("render_fwd_kernel");
   if (rc || !more) return rc;
   return launch_render_forward_long(P, packed, tile_offsets, binned_ids,
                                     out_rgb, out_T, out_last, out_tile_stop,
-                                    n_pairs, workspace, stream, t1);
+                                    n_pairs, workspace, stream, t1, set.live);
 }
 
 int launch_render_forward_long(const RasterParams& P, const float* packed,
@@ -1348,7 +1386,7 @@ int launch_render_forward_long(const RasterParams& P, const float* packed,
                                float* out_T, int32_t* out_last,
                                int32_t* out_tile_stop, int64_t n_pairs,
                                void* workspace, hipStream_t stream,
-                               hipEvent_t stop) {
+                               hipEvent_t stop, uint32_t* live) {
   if (P.num_tiles == 0 || workspace == nullptr) return GSPLAT_OK;
   const HeavyState H = forward_state(P, n_pairs, workspace, out_T);
   // Workgroups stride over the hand-off list (its length is on the device).
@@ -1356,9 +1394,51 @@ int launch_render_forward_long(const RasterParams& P, const float* packed,
   launch_timed("render_fwd_long_kernel", render_fwd_long_kernel<kLongStrips>, dim3(grid),
                dim3(256 / kLongStrips), stream, nullptr, stop, P,
                reinterpret_cast<const float4*>(packed), tile_offsets,
-               binned_ids, out_rgb, out_T, out_last, out_tile_stop, H);
+               binned_ids, out_rgb, out_T, out_last, out_tile_stop, H, live);
   return check_launch("render_fwd_long_kernel");
 }
+
+namespace {
+// The work of one binning in the backward's grid: one block per possible
+// segment slot, rounded to a multiple of 8 (XCD mapping), and one per tile.
+BwdSource bwd_source(const RasterParams& P, const float* packed,
+                     const int32_t* tile_offsets, const int32_t* binned_ids,
+                     const int32_t* tile_stop, const HeavyState& H,
+                     const TileSet* tiles) {
+  BwdSource W{};
+  W.packed = reinterpret_cast<const float4*>(packed);
+  W.tile_offsets = tile_offsets;
+  W.binned = binned_ids;
+  W.tile_stop = tile_stop;
+  W.H = H;
+  W.max_gid = (uint32_t)P.num_splats - 1u;
+  W.list = tiles != nullptr ? tiles->list : nullptr;
+  W.seg_blocks = H.counters ? (H.max_slots + 7) & ~7 : 0;
+  W.tiles = tiles != nullptr ? tiles->n : P.num_tiles;
+  return W;
+}
+
+int launch_backward_walk(const RasterParams& P, const BwdSource& A,
+                         const BwdSource& B, const float* final_T,
+                         const int32_t* last, const float* grad_rgb,
+                         const GradOut& G, int64_t n_pairs,
+                         hipStream_t stream) {
+  hipEvent_t t0 = nullptr, t1 = nullptr;
+  take_launch_timing(kTimeBackward, t0, t1);
+  // (the pair buffer's size stands for the pair count: up to 64 pairs per
+  // tile on average the short-tile variant is faster)
+  const bool short_tiles = n_pairs <= (int64_t)64 * P.num_tiles;
+  const int b_blocks = B.seg_blocks + ((B.tiles + 7) & ~7);
+  launch_timed("render_bwd_kernel",
+               G.acc == nullptr ? render_bwd_kernel<6, false>
+               : short_tiles    ? render_bwd_kernel<7, true>
+                                : render_bwd_kernel<6, true>,
+               dim3((unsigned)(b_blocks + A.seg_blocks + A.tiles)),
+               dim3(kLanes), stream, t0, t1, P, A, B, b_blocks, final_T, last,
+               grad_rgb, G);
+  return check_launch("render_bwd_kernel");
+}
+}  // namespace
 
 int launch_render_backward(const RasterParams& P, const float* packed,
                            const int32_t* tile_offsets,
@@ -1380,26 +1460,39 @@ int launch_render_backward(const RasterParams& P, const float* packed,
                                    P.num_splats, stream);
   if (rc) return rc;
   if (P.num_tiles == 0) return GSPLAT_OK;
-  const float4* pk = reinterpret_cast<const float4*>(packed);
-  // One block per possible slot, rounded to a multiple of 8 (XCD mapping).
-  const int seg_blocks = H.counters ? (H.max_slots + 7) & ~7 : 0;
-  hipEvent_t t0 = nullptr, t1 = nullptr;
-  take_launch_timing(kTimeBackward, t0, t1);
-  // (the pair buffer's size stands for the pair count: up to 64 pairs per
-  // tile on average the short-tile variant is faster)
-  const bool short_tiles = n_pairs <= (int64_t)64 * P.num_tiles;
-  launch_timed("render_bwd_kernel",
-               G.acc == nullptr ? render_bwd_kernel<6, false>
-               : short_tiles    ? render_bwd_kernel<7, true>
-                                : render_bwd_kernel<6, true>,
-               dim3((unsigned)(seg_blocks + P.num_tiles)), dim3(kLanes),
-               stream, t0, t1, P, pk, tile_offsets, binned_ids, final_T, last,
-               tile_stop, grad_rgb, G, H, seg_blocks);
-  rc = check_launch("render_bwd_kernel");
+  rc = launch_backward_walk(P,
+                            bwd_source(P, packed, tile_offsets, binned_ids,
+                                       tile_stop, H, nullptr),
+                            BwdSource{}, final_T, last, grad_rgb, G, n_pairs,
+                            stream);
   if (rc || G.acc == nullptr || P.num_splats <= 0) return rc;
+  return launch_grads_unpack(G.acc, g_means2d, g_conics, g_colors, g_opac,
+                             P.num_splats, stream);
+}
+
+int launch_sliced_backward(const BackwardSlice& front,
+                           const BackwardSlice& back, const TileSet& live,
+                           const float* final_T, const int32_t* last,
+                           const float* grad_rgb, float* acc,
+                           hipStream_t stream) {
+  auto source = [](const BackwardSlice& S, const TileSet* tiles) {
+    return bwd_source(S.P, S.packed, S.tile_offsets, S.binned_ids, S.tile_stop,
+                      heavy_state(S.P, S.n_pairs, S.workspace), tiles);
+  };
+  GradOut G{};
+  G.acc = acc;
+  return launch_backward_walk(
+      front.P, source(front, nullptr),
+      live.n > 0 ? source(back, &live) : BwdSource{}, final_T, last, grad_rgb,
+      G, front.n_pairs, stream);
+}
+
+int launch_grads_unpack(float* acc, float* g_means2d, float* g_conics,
+                        float* g_colors, float* g_opac, int n,
+                        hipStream_t stream) {
+  const GradOut G{g_means2d, g_conics, g_colors, g_opac, acc};
   launch_traced("render_grads_unpack_kernel", render_grads_unpack_kernel,
-                dim3((unsigned)((P.num_splats + 255) / 256)), dim3(256), 0,
-                stream, G, P.num_splats);
+                dim3((unsigned)((n + 255) / 256)), dim3(256), 0, stream, G, n);
   return check_launch("render_grads_unpack_kernel");
 }
 

@@ -27,6 +27,14 @@ struct RasterParams {
   float alpha_thr, trans_thr;
   float bg_r, bg_g, bg_b;
   float eps, max_alpha;
+  // Splats compacted from a larger set (slice.hip; null otherwise): the
+  // record of splat i carries orig_map[i] as its original index; with live
+  // only tiles whose bit is set there (tile t: word t / 32, bit t % 32) are
+  // hit, all of them in the box that boxes (SliceBuffers::box, by original
+  // index) holds.
+  const int32_t* orig_map;
+  const uint32_t* live;
+  const uint2* boxes;
 };
 
 struct ProjectParams {
@@ -137,6 +145,72 @@ int launch_depth_order_small(const float* depths, int32_t* perm, int64_t G,
 int launch_depth_ranks_small(void* buffers, int32_t* perm, int64_t G,
                              int batch, hipStream_t stream);
 
+// ---- slices of dense scenes (slice.hip)
+// The attributes of compacted splats and their original indices.
+struct SliceSplats {
+  float* means2d;
+  float* conics;
+  float* colors;
+  float* opacities;
+  float* depths;
+  int32_t* orig;
+};
+// ctl words and sums (zero before launch_slice_front, like hist, status_* and
+// back_count)
+constexpr int kSliceErr = 0, kSliceLive = 1, kSliceBackMax = 2,
+              kSliceFresh = 3;
+constexpr int kSliceTilesAll = 0, kSliceTilesBack = 1, kSliceStops = 2,
+              kSliceOpaque = 3, kSliceSums = 4;
+constexpr int kSliceBins = 2048;
+// A bin of a depth histogram and the totals before it.
+struct SliceCrossing {
+  int bin;
+  uint32_t c;
+  unsigned long long t;
+};
+struct SliceBuffers {
+  uint32_t* ctl;             // [8]
+  unsigned long long* sums;  // [kSliceSums]
+  uint32_t* back_count;      // [batch] splats that touch a live tile
+  unsigned long long* hist;  // [2][batch][kSliceBins] splats and their box
+                             // tiles per depth bin
+  uint64_t* status_front;    // [slice_status_words] look-back
+  uint64_t* status_back;
+  SliceCrossing* cross;      // [batch] where the budget ends, top 11 bits
+  uint32_t* limit;           // [batch] the front's depth key limit (22 bits)
+  uint2* box;                // [num_splats] tile boxes {x | y << 16, width |
+                             // height << 16}; of the back's splats cut down
+                             // to the live tiles
+  int32_t* back_list;        // [num_splats] those splats, per image
+  uint32_t* live_bits;       // [num_tiles / 32 + 2]
+  int32_t* live_list;        // [num_tiles]
+  SliceSplats front;         // [batch * slots]
+};
+bool slice_ok(const RasterParams& P);
+int slice_status_words(const RasterParams& P);
+// The nearest splats of each image, as many as fit slots splats and
+// max_tiles box tiles, into Q.front (the slots left over hold splats without
+// tiles), and Q.box, Q.limit.
+int launch_slice_front(const RasterParams& P, const SliceBuffers& Q,
+                       const float* means2d, const float* conics,
+                       const float* colors, const float* opacities,
+                       const float* depths, int slots, int64_t max_tiles,
+                       hipStream_t stream);
+// After the front's forward: live_bits, live_list, back_list and the host's
+// report (the words of gsplat_hip_front_render); tile_stop of a live tile
+// becomes 0.
+int launch_slice_back(const RasterParams& P, const SliceBuffers& Q,
+                      const float* depths, const uint32_t* tile_live,
+                      int32_t* tile_stop, const int32_t* bin_status,
+                      int32_t* host_words, hipStream_t stream);
+// The splats of back_list into `to` (slots per image, at least every
+// back_count).
+int launch_slice_gather(const RasterParams& P, const SliceBuffers& Q,
+                        const SliceSplats& to, int slots, const float* means2d,
+                        const float* conics, const float* colors,
+                        const float* opacities, const float* depths,
+                        hipStream_t stream);
+
 // ---- binning (binning.hip)
 // count: per-splat tile-hit counts (original order) into splat_count, the
 // per-workgroup sums into block_sums (count_blocks(P) ints) and their total
@@ -173,12 +247,19 @@ struct CountHist {
   int nparts = 0;
   uint32_t* ghist = nullptr;
 };
-int count_depth_runs_blocks(const RasterParams& P);
+// Splats per wavefront of the small-image path's two tile walks (8, 16 or
+// 32), by the pairs per splat that the buffers hold.
+int walk_splats(const RasterParams& P, int64_t capacity);
+// Largest number of emit workgroups of that path, where an emit workgroup
+// adds at most 4096 totals (16 per thread).
+constexpr int kScanEmitMaxBlocks = 4096;
+int count_depth_runs_blocks(const RasterParams& P, int walk);
 int launch_count_depth_runs(const RasterParams& P, const float* means2d,
                             const float* conics, const float* opacities,
                             int32_t* splat_count, uint32_t* zero_words,
                             int64_t n_zero_words, const float* depths,
-                            void* depth_buffers, hipStream_t stream,
+                            void* depth_buffers, int walk,
+                            hipStream_t stream,
                             const CountHist& H = CountHist{});
 // pack: packed records in gid order and splat_offsets[0..BG] (exclusive scan
 // of splat_count[perm]) via a look-back scan whose status
@@ -212,7 +293,7 @@ struct ZeroSpan {
 // the tile), atomically or via per-workgroup partials
 // (emit_blocks(P) * 4 * 256 words) and a reduction launch.  Only the first min(N, capacity) pairs are written and counted,
 // N = splat_offsets[num_splats] (-1 when N overflowed: nothing is written).
-int emit_blocks(const RasterParams& P);
+int emit_blocks(const RasterParams& P, int walk);
 // With scan, the emit scans the per-gid counts itself, each workgroup from
 // the sum of block_totals (emit_blocks(P) words: per emit workgroup the sum
 // of its gids' counts, as launch_rank_pack adds them) over the workgroups
@@ -222,6 +303,7 @@ struct EmitScanArgs {
   const int32_t* gid_count;
   int32_t* splat_offsets;
   const uint32_t* block_totals;
+  int walk;  // splats per wavefront (walk_splats)
 };
 // With orig (not with scan), the emit walks the splats in original order,
 // as the count did: from the count's records (rec_orig, launch_count's),
@@ -275,7 +357,7 @@ int launch_rank_pack(const RasterParams& P, const float* means2d,
                      const float* conics, const float* colors,
                      const float* opacities, void* depth_buffers,
                      const int32_t* splat_count, int32_t* perm, float* packed,
-                     int32_t* gid_count, uint32_t* block_totals,
+                     int32_t* gid_count, uint32_t* block_totals, int walk,
                      hipStream_t stream, const CountHist& H = CountHist{});
 // Tile ranges longer than this many pairs are walked by the forward's first
 // launch only up to here and continued by its second (render_fwd_long).
@@ -388,20 +470,30 @@ constexpr int kForwardStoppedLast = 4;
 // report (may be null): the binning's host report, written by the forward's
 // first workgroup as it starts (or by launch_host_report if the forward has
 // no workgroup).
+// T (may be null): tiles of a slice.  With list only the n tiles it names
+// are composited; with live, live[tile] becomes 1 where a pixel stayed above
+// the transmittance threshold, else 0.
+struct TileSet {
+  const int32_t* list;
+  int n;
+  uint32_t* live;
+};
 int launch_render_forward(const RasterParams& P, const float* packed,
                           const int32_t* tile_offsets,
                           const int32_t* binned_ids, float* out_rgb,
                           float* out_T, int32_t* out_last,
                           int32_t* out_tile_stop, int64_t n_pairs,
                           void* workspace, hipStream_t stream, int flags = 0,
-                          const HostReport* report = nullptr);
+                          const HostReport* report = nullptr,
+                          const TileSet* tiles = nullptr);
 int launch_render_forward_long(const RasterParams& P, const float* packed,
                                const int32_t* tile_offsets,
                                const int32_t* binned_ids, float* out_rgb,
                                float* out_T, int32_t* out_last,
                                int32_t* out_tile_stop, int64_t n_pairs,
                                void* workspace, hipStream_t stream,
-                               hipEvent_t stop = nullptr);
+                               hipEvent_t stop = nullptr,
+                               uint32_t* live = nullptr);
 // The workspace words a forward needs zero before it starts (hand-off
 // counters; with the state outputs also the backward's gradient records).
 void render_forward_zero_spans(const RasterParams& P, int64_t n_pairs,
@@ -415,6 +507,28 @@ int launch_render_backward(const RasterParams& P, const float* packed,
                            float* g_conics, float* g_colors, float* g_opac,
                            int64_t n_pairs, void* workspace,
                            hipStream_t stream);
+// The backward of a sliced forward, one launch: the front's tiles (a live
+// tile's stop is 0 there) and the live tiles of the back (live.n = 0: no
+// back).  Adds to the gradient records at acc ([splats of the whole scene],
+// zero on entry).
+struct BackwardSlice {
+  RasterParams P;
+  const float* packed;
+  const int32_t* tile_offsets;
+  const int32_t* binned_ids;
+  const int32_t* tile_stop;
+  int64_t n_pairs;
+  void* workspace;
+};
+int launch_sliced_backward(const BackwardSlice& front,
+                           const BackwardSlice& back, const TileSet& live,
+                           const float* final_T, const int32_t* last,
+                           const float* grad_rgb, float* acc,
+                           hipStream_t stream);
+// The records at acc scaled into the gradient arrays and zeroed.
+int launch_grads_unpack(float* acc, float* g_means2d, float* g_conics,
+                        float* g_colors, float* g_opac, int n,
+                        hipStream_t stream);
 
 // ---- projection (project.hip)
 int launch_project_forward(const ProjectParams& P, const float* means3d,

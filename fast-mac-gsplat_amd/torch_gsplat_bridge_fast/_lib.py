@@ -20,6 +20,7 @@ LIB_PATH = os.environ.get("GSPLAT_HIP_LIB", os.path.join(_HERE, "lib", "libgspla
 ABI_VERSION = 15
 TILE_SIZE = 16
 RECORD_FLOATS = 16
+GRAD_RECORD_FLOATS = 16                   # GSPLAT_GRAD_RECORD_FLOATS
 PROJECT_NOALLOC_SCRATCH_BYTES = 1 << 20   # GSPLAT_PROJECT_NOALLOC_SCRATCH_BYTES
 STATUS_LOOKBACK_TIMEOUT = 1               # GSPLAT_STATUS_LOOKBACK_TIMEOUT
 HANDOFF_PAIRS = 128                       # GSPLAT_HANDOFF_PAIRS
@@ -59,8 +60,16 @@ class ProjectMeta(ctypes.Structure):
     ]
 
 
+class Slice(ctypes.Structure):
+    """gsplat_slice of the C ABI."""
+    _fields_ = [("capacity", _i64), ("packed", _vp), ("binned_ids", _vp), ("tile_offsets", _vp), ("tile_stop", _vp),
+                ("splats", _vp), ("splats_bytes", _sz), ("bin_workspace", _vp), ("bin_workspace_bytes", _sz),
+                ("render_workspace", _vp), ("render_workspace_bytes", _sz), ("slots", _i32)]
+
+
 _PM = ctypes.POINTER(RasterMeta)
 _PP = ctypes.POINTER(ProjectMeta)
+_PS = ctypes.POINTER(Slice)
 
 # name -> (restype, argtypes); every name here is declared in gsplat_hip.h.
 SIGNATURES = {
@@ -87,6 +96,14 @@ SIGNATURES = {
         [_PM] + [_vp] * 5 + [_i64] + [_vp] * 7 + [_sz] + [_vp] * 5 + [_sz] + [_vp] * 5,
     ),
     "gsplat_hip_render_backward": (ctypes.c_int, [_PM] + [_vp] * 11 + [_i64, _vp, _sz, _vp]),
+    "gsplat_hip_slice_workspace_bytes": (_sz, [_PM]),
+    "gsplat_hip_slice_splats_bytes": (_sz, [_i32, _i32]),
+    "gsplat_hip_front_render": (ctypes.c_int, [_PM] + [_vp] * 5 + [_PS] + [_vp] * 6 + [_sz, _vp, _vp]),
+    "gsplat_hip_back_render": (
+        ctypes.c_int,
+        [_PM] + [_vp] * 5 + [_PS] + [_vp] * 4 + [_i32, _vp, _sz, _vp] + [_vp] * 4,
+    ),
+    "gsplat_hip_sliced_backward": (ctypes.c_int, [_PM, _PS, _PS, _vp, _i32] + [_vp] * 9),
     "gsplat_hip_project_forward": (ctypes.c_int, [_PP] + [_vp] * 10 + [_vp]),
     "gsplat_hip_project_backward_workspace_bytes": (_sz, [_PP]),
     "gsplat_hip_project_backward": (ctypes.c_int, [_PP] + [_vp] * 16 + [_vp, _sz, _vp]),

@@ -38,7 +38,7 @@ from typing import Any, Dict, List, Tuple
 import torch
 from torch import Tensor
 
-from . import _lib, _ops
+from . import _lib, _ops, _slices
 
 
 @dataclass(frozen=True)
@@ -295,9 +295,18 @@ class _RasterizeProjectedGaussians(torch.autograd.Function):
                      depths_b.detach())
         # the first backward's outputs, allocated before the host waits on the binning
         ctx.grad_bufs = _ops.gradient_buffers(B, G, means2d_b.device)
-        st, (img, final_T, last, tile_stop, ws) = _ops.bin_and_render(meta, flat, save_state=True)
-        _check_overflow(config, st)
-        ctx.save_for_backward(st.packed, st.tile_offsets, st.pairs, final_T, last, tile_stop, ws)
+        # (a check of the tiles' pair counts needs the whole binning)
+        sliced = _slices.render(meta, flat, save_state=True) if config.enable_overflow_fallback else None
+        if sliced is not None:
+            st, (img, final_T, last) = sliced
+            ctx.save_for_backward(final_T, last, *st.tensors())
+            ctx.sliced = st.plain()
+            st.release()
+        else:
+            st, (img, final_T, last, tile_stop, ws) = _ops.bin_and_render(meta, flat, save_state=True)
+            _check_overflow(config, st)
+            ctx.save_for_backward(st.packed, st.tile_offsets, st.pairs, final_T, last, tile_stop, ws)
+            ctx.sliced = None
         # the binning's status is read before the backward (by then the GPU is done with it)
         ctx.check_status = st.check_status
         ctx.meta = meta
@@ -308,11 +317,18 @@ class _RasterizeProjectedGaussians(torch.autograd.Function):
 
     @staticmethod
     def backward(ctx, grad_out):
-        packed, tile_offsets, pairs, final_T, last, tile_stop, ws = ctx.saved_tensors
+        saved = ctx.saved_tensors
         ctx.check_status()
-        st = _ops.BinState(None, packed, None, tile_offsets, pairs, pairs.numel())
         bufs, ctx.grad_bufs = ctx.grad_bufs, None   # a second backward (retain_graph) allocates anew
-        g_m, g_q, g_c, g_o = _ops.render_backward(ctx.meta, st, final_T, last, tile_stop, grad_out, ws, out=bufs)
+        if ctx.sliced is not None:
+            final_T, last, *tensors = saved
+            g_m, g_q, g_c, g_o = _slices.backward(
+                ctx.meta, tensors, ctx.sliced, final_T, last, grad_out,
+                bufs if bufs is not None else _ops.gradient_buffers(*ctx.shape, grad_out.device))
+        else:
+            packed, tile_offsets, pairs, final_T, last, tile_stop, ws = saved
+            st = _ops.BinState(None, packed, None, tile_offsets, pairs, pairs.numel())
+            g_m, g_q, g_c, g_o = _ops.render_backward(ctx.meta, st, final_T, last, tile_stop, grad_out, ws, out=bufs)
         need = ctx.needs_input_grad
         # The depth gradient is zero (the reference returns zeros, v8 rasterize.py:680).  For depths
         # computed by the projection (depth_grad False) it is returned as None, which autograd
@@ -330,9 +346,13 @@ def _rasterize_chunk_eval(means2d_b, conics_b, colors_b, opacities_b, depths_b, 
     """Eval path (reference v8 rasterize.py:684-786): no saved state."""
     B, G = means2d_b.shape[:2]
     meta = _meta(config, B, G)
-    st, out = _ops.bin_and_render(meta, _flat(means2d_b, conics_b, colors_b, opacities_b, depths_b),
-                                  save_state=False)
-    _check_overflow(config, st)
+    flat = _flat(means2d_b, conics_b, colors_b, opacities_b, depths_b)
+    sliced = _slices.render(meta, flat, save_state=False) if config.enable_overflow_fallback else None
+    if sliced is not None:
+        st, out = sliced
+    else:
+        st, out = _ops.bin_and_render(meta, flat, save_state=False)
+        _check_overflow(config, st)
     st.check_status()
     return out[0]
 

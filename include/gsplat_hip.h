@@ -491,6 +491,93 @@ int gsplat_hip_radix_sort_pairs_u32(const uint32_t* keys_in,
                                     int32_t* status, void* workspace,
                                     size_t workspace_bytes, void* stream);
 
+/* ---- Sliced rendering of dense scenes -------------------------------------
+ * Where most of a tile's list lies behind the splat that makes it opaque, the
+ * one-call forward is done in two parts, with the image, stops and gradients
+ * of gsplat_hip_bin_render_forward.  The front bins and composites the
+ * nearest splats of each image, as many as fit the slice's slots and
+ * capacity; it lists the live tiles, those with a pixel above the
+ * transmittance threshold.  The back bins every splat whose tile box holds a
+ * live tile, in live tiles only, and composites those tiles again from their
+ * whole lists.  It has no counterpart in the reference. */
+
+/* Floats of one splat's gradient sums (grad_records: [B*G] of them). */
+#define GSPLAT_GRAD_RECORD_FLOATS 16
+
+/* One slice: its splats per image and pair capacity, its outputs (packed
+ * float [B*slots*16], binned_ids int32 [capacity], tile_offsets int32 [T+1],
+ * tile_stop int32 [T]) and workspaces, sized with a meta of
+ * gaussians_per_batch = slots: bin_workspace by gsplat_hip_bin_workspace_bytes
+ * and render_workspace by gsplat_hip_render_workspace_bytes (capacity, or 0
+ * without state outputs), splats by gsplat_hip_slice_splats_bytes.  The
+ * backward reads packed, binned_ids, tile_offsets, tile_stop and
+ * render_workspace. */
+typedef struct gsplat_slice {
+  int64_t capacity;
+  float* packed;
+  int32_t* binned_ids;
+  int32_t* tile_offsets;
+  int32_t* tile_stop;
+  void* splats;
+  size_t splats_bytes;
+  void* bin_workspace;
+  size_t bin_workspace_bytes;
+  void* render_workspace;
+  size_t render_workspace_bytes;
+  int32_t slots;
+} gsplat_slice;
+
+/* 0 where the scene cannot be sliced (more than 64 images, or images of more
+ * than 2^18 tiles or of 2^22 splats or more). */
+size_t gsplat_hip_slice_workspace_bytes(const gsplat_raster_meta* meta);
+size_t gsplat_hip_slice_splats_bytes(int32_t batch, int32_t slots);
+
+/* The front: each image gets capacity / B pairs.  out_final_T, out_last and
+ * grad_records (float [B*G*16], zeroed here) are all given or all NULL.
+ * live_list int32 [T].  host_words: pinned int32 [16], written when the front
+ * is done, the ready word last: {0: status (GSPLAT_STATUS_*), 1: live tiles,
+ * 2: most splats of an image whose box holds a live tile, 3: 1 if one of
+ * those is not in the front, 4-5: box tiles of all splats (64 bits), 6-7: live
+ * tiles in the boxes of those splats (at least the back's pairs), 8-9: sum of
+ * the opaque tiles' stops, 10-11: their number, 15: 1}.  Without live tiles,
+ * or with word 3 = 0, the front is the whole result. */
+int gsplat_hip_front_render(const gsplat_raster_meta* meta,
+                            const float* means2d, const float* conics,
+                            const float* colors, const float* opacities,
+                            const float* depths, const gsplat_slice* front,
+                            float* out_rgb, float* out_final_T,
+                            int32_t* out_last, float* grad_records,
+                            int32_t* live_list, void* workspace,
+                            size_t workspace_bytes, int32_t* host_words,
+                            void* stream);
+
+/* The back, after the front of the same inputs, outputs and workspace: slots
+ * at least word 2 and capacity at least words 6-7 of its report, n_live its
+ * word 1.  host_words: pinned int32 [4], as gsplat_hip_bin's.  count_stream
+ * and the events as there. */
+int gsplat_hip_back_render(const gsplat_raster_meta* meta,
+                           const float* means2d, const float* conics,
+                           const float* colors, const float* opacities,
+                           const float* depths, const gsplat_slice* back,
+                           float* out_rgb, float* out_final_T,
+                           int32_t* out_last, int32_t* live_list,
+                           int32_t n_live, void* workspace,
+                           size_t workspace_bytes, int32_t* host_words,
+                           void* stream, void* count_stream,
+                           void* inputs_event, void* count_event);
+
+/* gsplat_hip_render_backward of a sliced forward (back NULL where there was
+ * none).  grad_records: the front's, zero again afterwards. */
+int gsplat_hip_sliced_backward(const gsplat_raster_meta* meta,
+                               const gsplat_slice* front,
+                               const gsplat_slice* back,
+                               const int32_t* live_list, int32_t n_live,
+                               const float* final_T, const int32_t* last,
+                               const float* grad_rgb, float* grad_records,
+                               float* g_means2d, float* g_conics,
+                               float* g_colors, float* g_opacities,
+                               void* stream);
+
 #ifdef __cplusplus
 }
 #endif

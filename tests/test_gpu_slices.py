@@ -1,0 +1,167 @@
+"""The sliced forward and backward of dense scenes against the unsliced path:
+the image bit for bit (both walk the same splats of every tile in the same
+order), the gradients up to the order of their atomic sums."""
+import pytest
+import torch
+
+from torch_gsplat_bridge_fast import RasterConfig, _lib, _ops, _slices, rasterize_projected_gaussians
+
+pytestmark = pytest.mark.gpu
+
+
+def _scene(B, G, H, W, seed, sigma=(4.0, 20.0), logit=0.0, depth="uniform", cover=1.0):
+    """Splats over the left `cover` of the image; depth ties with depth="planes"."""
+    g = torch.Generator().manual_seed(seed)
+    means = torch.rand(B, G, 2, generator=g) * torch.tensor([W * cover, float(H)])
+    sig = sigma[0] + torch.rand(B, G, 2, generator=g) * (sigma[1] - sigma[0])
+    th = torch.rand(B, G, generator=g) * 3.14159
+    c, s = torch.cos(th), torch.sin(th)
+    ix, iy = sig[..., 0] ** -2, sig[..., 1] ** -2
+    conics = torch.stack([c * c * ix + s * s * iy, c * s * (ix - iy), s * s * ix + c * c * iy], -1)
+    depths = torch.rand(B, G, generator=g) * 10 if depth == "uniform" else \
+        torch.randint(0, 40, (B, G), generator=g).float()
+    if depth == "one":
+        depths = torch.ones(B, G)
+    opac = torch.sigmoid(logit + torch.randn(B, G, generator=g))
+    if depth == "veil":  # the left 45% nearly transparent: most of its splats touch live tiles
+        opac = torch.where(means[..., 0] < 0.45 * W, 0.02 * opac, opac)
+        depths = torch.rand(B, G, generator=g) * 10
+    t = [means, conics, torch.rand(B, G, 3, generator=g), opac, depths]
+    return [x.cuda().contiguous() for x in t]
+
+
+def _flat(ts):
+    return [t.reshape(-1, t.shape[-1]) if t.ndim == 3 else t.reshape(-1) for t in ts]
+
+
+def _unsliced(meta, ts, w):
+    st = _ops.bin_gaussians(meta, *_flat(ts))
+    img, T, last, stop, ws = _ops.render_forward(meta, st, save_state=True)
+    grads = _ops.render_backward(meta, st, T, last, stop, w, ws)
+    return st, img, T, stop, grads
+
+
+def _sliced(monkeypatch, meta, ts, w, budget, cap, save_state=True):
+    key = (0, meta.batch, meta.gaussians_per_batch, meta.height, meta.width)
+    monkeypatch.setattr(_slices, "MIN_PAIRS", 0)
+    monkeypatch.setattr(_slices, "MIN_PAIRS_PER_TILE", 0)
+    monkeypatch.setitem(_ops._capacity, key, cap)
+    plan = _slices._Plan(cap)
+    plan.budget = budget
+    monkeypatch.setitem(_slices._plans, key, plan)
+    got = _slices.render(meta, _flat(ts), save_state=save_state)
+    if got is None or not save_state:
+        return got, None
+    st, (img, T, last) = got
+    out = _ops.gradient_buffers(meta.batch, meta.gaussians_per_batch, img.device)
+    grads = _slices.backward(meta, st.tensors(), st.plain(), T, last, w, out)
+    st.check_status()
+    return got, grads
+
+
+CASES = [
+    # B, G, H, W, sigma, logit, depth, cover, budget
+    (1, 20000, 200, 300, (4.0, 20.0), 0.0, "uniform", 1.0, 256),    # opaque but for some edges
+    (1, 20000, 200, 300, (4.0, 20.0), 0.0, "planes", 0.6, 400),     # depth ties, an empty side
+    (2, 9001, 203, 341, (4.0, 20.0), 0.0, "uniform", 0.9, 220),     # ragged, two images
+    (3, 5000, 64, 80, (2.0, 9.0), 0.0, "planes", 1.0, 300),         # tiles of three images in one bitmap word
+    (1, 30000, 160, 160, (4.0, 30.0), -1.0, "uniform", 0.8, 900),   # lists over 128: continuation, segments
+    (1, 350000, 512, 512, (1.0, 6.0), 0.5, "veil", 1.0, 400),       # a back of over 131,072 splats
+    (1, 20000, 200, 300, (4.0, 20.0), 0.0, "uniform", 1.0, 100000),  # the front holds every splat
+]
+
+
+@pytest.mark.parametrize("B,G,H,W,sigma,logit,depth,cover,budget", CASES)
+def test_sliced_matches_unsliced(monkeypatch, B, G, H, W, sigma, logit, depth, cover, budget):
+    ts = _scene(B, G, H, W, 3, sigma, logit, depth, cover)
+    meta = _lib.make_raster_meta(H, W, B, G, 1 / 255, 1e-4, (0.1, 0.2, 0.3))
+    w = torch.rand(B, H, W, 3, generator=torch.Generator().manual_seed(1)).cuda()
+    st, img, T, stop, ref = _unsliced(meta, ts, w)
+    cap = max(st.n_pairs, 2 * budget * st.num_tiles)
+    got, grads = _sliced(monkeypatch, meta, ts, w, budget, cap)
+    key = (0, B, G, H, W)
+    assert got is not None, f"the scene was meant to be sliced (budget now {_slices._plans[key].budget})"
+    state, (img2, T2, last2) = got
+    assert torch.equal(img, img2) and torch.equal(T, T2)
+    if budget >= 100000:
+        assert not state.has_back
+    if depth == "veil":
+        assert state.plain()[1][1][1] > 131072  # the back's slots
+    for a, b in zip(grads, ref):
+        torch.testing.assert_close(a, b, rtol=1e-4, atol=1e-5 * float(b.abs().max()))
+    # a second backward on the same state: the gradient records are zero again
+    again = _slices.backward(meta, state.tensors(), state.plain(), T2, last2, w,
+                             _ops.gradient_buffers(B, G, img.device))
+    for a, b in zip(again, ref):
+        torch.testing.assert_close(a, b, rtol=1e-4, atol=1e-5 * float(b.abs().max()))
+    # the eval forward
+    got, _ = _sliced(monkeypatch, meta, ts, w, budget, cap, save_state=False)
+    assert torch.equal(got[1][0], img)
+
+
+def test_fronts_that_do_not_suit_return_none(monkeypatch):
+    """One depth for all (no front can be chosen) and a translucent scene: the caller is sent to the
+    unsliced path and the shape's budget is raised or given up."""
+    for kw in (dict(depth="one"), dict(logit=-4.0)):
+        ts = _scene(1, 20000, 200, 300, 5, **kw)
+        meta = _lib.make_raster_meta(200, 300, 1, 20000, 1 / 255, 1e-4, (0, 0, 0))
+        st = _ops.bin_gaussians(meta, *_flat(ts))
+        got, _ = _sliced(monkeypatch, meta, ts, None, 32, max(st.n_pairs, 64 * st.num_tiles), save_state=False)
+        assert got is None
+        assert _slices._plans[(0, 1, 20000, 200, 300)].budget in (0, 64)
+
+
+def test_public_calls_take_the_slices(monkeypatch):
+    """rasterize_projected_gaussians on a dense scene: the second and later calls of the shape are
+    sliced and give the first call's image, through autograd too."""
+    monkeypatch.setattr(_slices, "MIN_PAIRS", 1 << 18)
+    monkeypatch.setattr(_slices, "FIRST_BUDGET", 96)
+    seen = []
+    orig = _slices.render
+    monkeypatch.setattr(_slices, "render", lambda *a, **k: seen.append(orig(*a, **k)) or seen[-1])
+    B, G, H, W = 1, 40001, 190, 310
+    ts = _scene(B, G, H, W, 11)
+    cfg = RasterConfig(height=H, width=W, background=(0.1, 0.2, 0.3))
+    imgs, grads = [], []
+    for k in range(4):
+        leaves = [t[0].clone().requires_grad_(True) for t in ts]
+        img = rasterize_projected_gaussians(*leaves, cfg)
+        img.square().mean().backward()
+        imgs.append(img.detach())
+        grads.append([t.grad for t in leaves])
+    with torch.no_grad():
+        imgs.append(rasterize_projected_gaussians(*[t[0] for t in ts], cfg))
+    assert any(s is not None for s in seen)
+    for img in imgs[1:]:
+        assert torch.equal(img, imgs[0])
+    for g in grads[1:]:
+        for a, b in zip(g, grads[0]):
+            torch.testing.assert_close(a, b, rtol=1e-4, atol=1e-5 * float(b.abs().max()))
+
+
+@pytest.mark.parametrize("B,G,H,W,sigma", [
+    (1, 2999, 300, 500, (6.0, 20.0)),     # 8 splats per wavefront: dozens of pairs per splat
+    (2, 70001, 400, 500, (8.0, 16.0)),    # 16: as dense, over 131,072 splats in the batch
+    (1, 16384, 300, 500, (0.5, 2.0)),     # 16: few splats
+    (1, 16385, 300, 500, (0.5, 2.0)),     # 32
+])
+def test_walk_widths(monkeypatch, B, G, H, W, sigma):
+    """The one-call binning at each number of splats per wavefront against the staged calls (always
+    32): the same offsets, tile ranges and lists."""
+    ts = _scene(B, G, H, W, 7, sigma)
+    meta = _lib.make_raster_meta(H, W, B, G, 1 / 255, 1e-4, (0, 0, 0))
+    key = (0, B, G, H, W)
+    monkeypatch.delitem(_ops._capacity, key, raising=False)
+    ref = _ops.bin_gaussians(meta, *_flat(ts))   # staged: the shape's first binning
+    n = ref.n_pairs
+    if sigma[0] > 1:
+        assert n >= 24 * B * G
+    for cap in (n, n + 1, n + n // 4):
+        got = _ops._bin_fast(meta, *_flat(ts), cap, key)
+        assert got.n_pairs == n
+        got.check_status()
+        assert torch.equal(got.perm, ref.perm)
+        assert torch.equal(got.splat_offsets, ref.splat_offsets)
+        assert torch.equal(got.tile_offsets, ref.tile_offsets)
+        assert torch.equal(got.binned_ids, ref.binned_ids)
+        assert torch.equal(got.packed, ref.packed)
