@@ -1454,7 +1454,7 @@ int gsplat_hip_front_render(const gsplat_raster_meta* meta,
   if (!rc)
     rc = slice_render(ms, PS, front, C, view, SL, out_rgb, out_final_T,
                       out_last, acc, host_words, stream, nullptr, nullptr,
-                      nullptr, gs::TileSet{nullptr, 0, tile_live}, &report,
+                      nullptr, gs::TileSet{nullptr, 0, tile_live, nullptr}, &report,
                       false);
   if (!rc)
     rc = gs::launch_slice_back(P, Q, depths, tile_live, front->tile_stop,
@@ -1508,7 +1508,7 @@ int gsplat_hip_back_render(const gsplat_raster_meta* meta,
     rc = slice_render(ms, PS, back, C, view, SL, out_rgb, out_final_T, out_last,
                       gs::ZeroSpan{nullptr, 0}, host_words, stream,
                       count_stream, inputs_event, count_event,
-                      gs::TileSet{live_list, n_live, nullptr}, &report, true);
+                      gs::TileSet{live_list, n_live, nullptr, nullptr}, &report, true);
   return rc;
 }
 
@@ -1549,12 +1549,95 @@ int gsplat_hip_sliced_backward(const gsplat_raster_meta* meta,
   rc = gs::launch_sliced_backward(
       slice_of(PS, front),
       back != nullptr ? slice_of(PB, back) : gs::BackwardSlice{},
-      gs::TileSet{live_list, back != nullptr ? n_live : 0, nullptr}, final_T,
+      gs::TileSet{live_list, back != nullptr ? n_live : 0, nullptr, nullptr}, final_T,
       last, grad_rgb, grad_records, s);
   if (!rc)
     rc = gs::launch_grads_unpack(grad_records, g_means2d, g_conics, g_colors,
                                  g_opacities, P.num_splats, s);
   return rc;
+}
+
+}  // extern "C"
+
+namespace {
+// The direct path's workspace: the splats' boxes and tests, and the tiles'
+// ends.
+struct DirectLayout {
+  size_t box, test, ends, total;
+};
+DirectLayout direct_layout(const RasterParams& P) {
+  DirectLayout L{};
+  L.box = 0;
+  L.test = gs::align_up((size_t)P.num_splats * sizeof(uint2), 256);
+  L.ends = L.test + gs::align_up((size_t)P.num_splats * sizeof(float4), 256);
+  L.total = L.ends + gs::align_up((size_t)P.num_tiles * sizeof(int32_t), 256);
+  return L;
+}
+}  // namespace
+
+extern "C" {
+
+size_t gsplat_hip_direct_workspace_bytes(const gsplat_raster_meta* meta) {
+  RasterParams P;
+  if (make_params(meta, P) || !gs::direct_ok(P)) return 0;
+  return direct_layout(P).total;
+}
+
+int gsplat_hip_direct_render(const gsplat_raster_meta* meta,
+                             const float* means2d, const float* conics,
+                             const float* colors, const float* opacities,
+                             const float* depths, float* packed,
+                             int32_t* tile_starts, int32_t* binned_ids,
+                             float* out_rgb, float* out_final_T,
+                             int32_t* out_last, int32_t* out_tile_stop,
+                             void* workspace, size_t workspace_bytes,
+                             void* render_workspace,
+                             size_t render_workspace_bytes, void* stream) {
+  const char* what = "gsplat_hip_direct_render";
+  RasterParams P;
+  int rc = make_params(meta, P);
+  if (rc) return rc;
+  if (!gs::direct_ok(P)) {
+    gs::set_error("%s: needs at most %d splats per image and %lld tiles x "
+                  "splats", what, gs::kDirectMaxSplats,
+                  (long long)gs::kDirectMaxTests);
+    return GSPLAT_ERR_INVALID_ARGUMENT;
+  }
+  const int64_t n_pairs = (int64_t)P.num_tiles * P.gpb;
+  rc = null_check({means2d, conics, colors, opacities, depths, binned_ids,
+                   workspace, render_workspace},
+                  what);
+  if (!rc)
+    rc = check_forward(P, packed, tile_starts, binned_ids, out_rgb, out_final_T,
+                       out_last, out_tile_stop, n_pairs, render_workspace,
+                       render_workspace_bytes, what);
+  if (rc) return rc;
+  const DirectLayout L = direct_layout(P);
+  if (workspace_bytes < L.total) {
+    gs::set_error("%s: workspace too small (%zu < %zu)", what, workspace_bytes,
+                  L.total);
+    return GSPLAT_ERR_WORKSPACE;
+  }
+  char* b = static_cast<char*>(workspace);
+  const gs::DirectSplats D{reinterpret_cast<uint2*>(b + L.box),
+                           reinterpret_cast<float4*>(b + L.test)};
+  int32_t* ends = reinterpret_cast<int32_t*>(b + L.ends);
+  hipStream_t s = static_cast<hipStream_t>(stream);
+  gs::ZeroSpan zero[2];
+  gs::render_forward_zero_spans(P, n_pairs, render_workspace,
+                                out_final_T != nullptr, zero);
+  rc = gs::launch_direct_lists(P, means2d, conics, colors, opacities, depths,
+                               packed, D, binned_ids, tile_starts, ends, zero,
+                               s);
+  if (rc) return rc;
+  // (no list is longer than the image's splats)
+  const int flags = gs::kForwardPreZeroed | gs::kForwardStoppedLast |
+                    (P.gpb <= gs::kHandoffPairs ? gs::kForwardNoLong : 0);
+  const gs::TileSet tiles{nullptr, 0, nullptr, ends};
+  return gs::launch_render_forward(P, packed, tile_starts, binned_ids, out_rgb,
+                                   out_final_T, out_last, out_tile_stop,
+                                   n_pairs, render_workspace, s, flags, nullptr,
+                                   &tiles);
 }
 
 }  // extern "C"

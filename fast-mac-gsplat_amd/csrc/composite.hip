@@ -499,7 +499,7 @@ void render_fwd_kernel(
     last[k] = 0;
   }
   const int start = tile_offsets[tc.tile];
-  const int end = tile_offsets[tc.tile + 1];
+  const int end = tiles.ends[tc.tile];
   if (H.rec != nullptr && threadIdx.x == 0) H.tile_slot[tc.tile] = -1;
   // The workspace's layout follows n_pairs: the backward uses the segment
   // records only if it was given the same n_pairs (same max_slots).
@@ -657,8 +657,7 @@ __global__ __launch_bounds__(256 / kSpW) void render_fwd_long_kernel(
     const int32_t* __restrict__ tile_offsets,
     const int32_t* __restrict__ binned, float* __restrict__ out_rgb,
     float* __restrict__ out_T, int32_t* __restrict__ out_last,
-    int32_t* __restrict__ out_tile_stop, HeavyState H,
-    uint32_t* __restrict__ live) {
+    int32_t* __restrict__ out_tile_stop, HeavyState H, TileSet tiles) {
   __shared__ Staged S;
   __shared__ int sh_slot;
   __shared__ int sh_plain;  // batch_plain of the staged batch
@@ -690,7 +689,7 @@ __global__ __launch_bounds__(256 / kSpW) void render_fwd_long_kernel(
       cr[k] = cg[k] = cb[k] = 0.0f;
     }
     const int start = tile_offsets[tile];
-    const int end = tile_offsets[tile + 1];
+    const int end = tiles.ends[tile];
     int seg_cur = kHandoff / kSegSplats;
     for (int base = start + kHandoff; base < end; base += kBatch) {
       bool alive = false;
@@ -726,11 +725,12 @@ __global__ __launch_bounds__(256 / kSpW) void render_fwd_long_kernel(
     if (threadIdx.x == 0) sh_slot = next_segment(H, tile, seg_cur, tail);
     __syncthreads();
     last_segment<kSpW>(P, tc, out_rgb, H, sh_slot, valid, cr, cg, cb, T, t0);
-    if (live != nullptr) {
+    if (tiles.live != nullptr) {
       bool alive = false;
 #pragma unroll
       for (int k = 0; k < kSpW; ++k) alive |= T[k] > t_thr;
-      if (__builtin_amdgcn_ballot_w64(alive) != 0 && lane == 0) live[tile] = 1u;
+      if (__builtin_amdgcn_ballot_w64(alive) != 0 && lane == 0)
+        tiles.live[tile] = 1u;
     }
     int tile_max = 0;
 #pragma unroll
@@ -1332,6 +1332,13 @@ HeavyState forward_state(const RasterParams& P, int64_t n_pairs,
 }
 }  // namespace
 
+// The kernels' tile set: ends given, or the offsets' own.
+static TileSet tile_set(const TileSet* tiles, const int32_t* tile_offsets) {
+  TileSet s = tiles != nullptr ? *tiles : TileSet{};
+  if (s.ends == nullptr) s.ends = tile_offsets + 1;
+  return s;
+}
+
 // A launch with the one-shot timing events start/stop (gsplat_hip_time_next_
 // launch; either may be null), else a traced launch.
 template <typename... KArgs, typename... Args>
@@ -1354,7 +1361,7 @@ int launch_render_forward(const RasterParams& P, const float* packed,
                           const HostReport* report, const TileSet* tiles) {
   hipEvent_t t0 = nullptr, t1 = nullptr;
   take_launch_timing(kTimeForward, t0, t1);
-  const TileSet set = tiles != nullptr ? *tiles : TileSet{};
+  const TileSet set = tile_set(tiles, tile_offsets);
   const int n_tiles = set.list != nullptr ? set.n : P.num_tiles;
   if (n_tiles == 0)
     return report != nullptr ? launch_host_report(*report, stream) : GSPLAT_OK;
@@ -1377,7 +1384,7 @@ int launch_render_forward(const RasterParams& P, const float* packed,
   if (rc || !more) return rc;
   return launch_render_forward_long(P, packed, tile_offsets, binned_ids,
                                     out_rgb, out_T, out_last, out_tile_stop,
-                                    n_pairs, workspace, stream, t1, set.live);
+                                    n_pairs, workspace, stream, t1, tiles);
 }
 
 int launch_render_forward_long(const RasterParams& P, const float* packed,
@@ -1386,7 +1393,7 @@ int launch_render_forward_long(const RasterParams& P, const float* packed,
                                float* out_T, int32_t* out_last,
                                int32_t* out_tile_stop, int64_t n_pairs,
                                void* workspace, hipStream_t stream,
-                               hipEvent_t stop, uint32_t* live) {
+                               hipEvent_t stop, const TileSet* tiles) {
   if (P.num_tiles == 0 || workspace == nullptr) return GSPLAT_OK;
   const HeavyState H = forward_state(P, n_pairs, workspace, out_T);
   // Workgroups stride over the hand-off list (its length is on the device).
@@ -1394,7 +1401,8 @@ int launch_render_forward_long(const RasterParams& P, const float* packed,
   launch_timed("render_fwd_long_kernel", render_fwd_long_kernel<kLongStrips>, dim3(grid),
                dim3(256 / kLongStrips), stream, nullptr, stop, P,
                reinterpret_cast<const float4*>(packed), tile_offsets,
-               binned_ids, out_rgb, out_T, out_last, out_tile_stop, H, live);
+               binned_ids, out_rgb, out_T, out_last, out_tile_stop, H,
+               tile_set(tiles, tile_offsets));
   return check_launch("render_fwd_long_kernel");
 }
 

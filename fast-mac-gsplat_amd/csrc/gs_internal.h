@@ -452,6 +452,25 @@ inline void launch_traced(const char* name, void (*kernel)(KArgs...),
                        static_cast<KArgs>(args)...);
 }
 
+// ---- small scenes (direct.hip)
+constexpr int kDirectMaxSplats = 4096;            // per image
+constexpr int64_t kDirectMaxTests = 12 << 20;     // tiles x splats per image
+// Per gid: the tile box and the constants of its exact test.
+struct DirectSplats {
+  uint2* box;    // [num_splats]
+  float4* test;  // [num_splats]
+};
+bool direct_ok(const RasterParams& P);
+// Depth order, records and tile lists: tile t's gids, ascending, at
+// pairs[tile_starts[t] .. tile_ends[t]) with tile_starts[t] = t * gpb.  The
+// first launch zeroes the two spans.
+int launch_direct_lists(const RasterParams& P, const float* means2d,
+                        const float* conics, const float* colors,
+                        const float* opacities, const float* depths,
+                        float* packed, const DirectSplats& D, int32_t* pairs,
+                        int32_t* tile_starts, int32_t* tile_ends,
+                        const ZeroSpan zero[2], hipStream_t stream);
+
 // ---- compositing (composite.hip)
 // workspace (render_workspace_bytes, may be null): heavy-tile segment state,
 // written by the forward and read by the backward of the same binning.
@@ -470,13 +489,15 @@ constexpr int kForwardStoppedLast = 4;
 // report (may be null): the binning's host report, written by the forward's
 // first workgroup as it starts (or by launch_host_report if the forward has
 // no workgroup).
-// T (may be null): tiles of a slice.  With list only the n tiles it names
-// are composited; with live, live[tile] becomes 1 where a pixel stayed above
-// the transmittance threshold, else 0.
+// tiles (may be null): with list only the n tiles it names are composited;
+// with live, live[tile] becomes 1 where a pixel stayed above the
+// transmittance threshold, else 0; with ends, tile t's range ends at ends[t]
+// (else at tile_offsets[t + 1]).
 struct TileSet {
   const int32_t* list;
   int n;
   uint32_t* live;
+  const int32_t* ends;
 };
 int launch_render_forward(const RasterParams& P, const float* packed,
                           const int32_t* tile_offsets,
@@ -493,7 +514,7 @@ int launch_render_forward_long(const RasterParams& P, const float* packed,
                                int32_t* out_tile_stop, int64_t n_pairs,
                                void* workspace, hipStream_t stream,
                                hipEvent_t stop = nullptr,
-                               uint32_t* live = nullptr);
+                               const TileSet* tiles = nullptr);
 // The workspace words a forward needs zero before it starts (hand-off
 // counters; with the state outputs also the backward's gradient records).
 void render_forward_zero_spans(const RasterParams& P, int64_t n_pairs,

@@ -104,6 +104,8 @@ SIGNATURES = {
         [_PM] + [_vp] * 5 + [_PS] + [_vp] * 4 + [_i32, _vp, _sz, _vp] + [_vp] * 4,
     ),
     "gsplat_hip_sliced_backward": (ctypes.c_int, [_PM, _PS, _PS, _vp, _i32] + [_vp] * 9),
+    "gsplat_hip_direct_workspace_bytes": (_sz, [_PM]),
+    "gsplat_hip_direct_render": (ctypes.c_int, [_PM] + [_vp] * 13 + [_sz, _vp, _sz, _vp]),
     "gsplat_hip_project_forward": (ctypes.c_int, [_PP] + [_vp] * 10 + [_vp]),
     "gsplat_hip_project_backward_workspace_bytes": (_sz, [_PP]),
     "gsplat_hip_project_backward": (ctypes.c_int, [_PP] + [_vp] * 16 + [_vp, _sz, _vp]),

@@ -319,6 +319,52 @@ def bin_and_render(meta: _lib.RasterMeta, flat, *, save_state: bool):
     return st, out
 
 
+_direct_bytes: dict = {}
+
+
+def direct_render(meta: _lib.RasterMeta, flat, *, save_state: bool):
+    """(BinState, render_forward outputs) of a small scene by gsplat_hip_direct_render, where every tile
+    scans its image's splats: no pair count, so the host waits for nothing and nothing can overflow.
+    None for scenes above its limits.  The state's lists start at tile_offsets[t] = t * G."""
+    means2d, conics, colors, opacities, depths = flat
+    dev = means2d.device
+    B, G, H, W = meta.batch, meta.gaussians_per_batch, meta.height, meta.width
+    if G > 4096 or _staged():
+        return None
+    key = (B, G, H, W, save_state)
+    sizes = _direct_bytes.get(key)
+    if sizes is None:
+        L = _lib.lib()
+        ws_bytes = L.gsplat_hip_direct_workspace_bytes(meta)
+        tiles = B * ((H + 15) // 16) * ((W + 15) // 16)
+        n = tiles * G if ws_bytes else 0
+        sizes = (ws_bytes, L.gsplat_hip_render_workspace_bytes(meta, n if save_state else 0) if ws_bytes else 0,
+                 tiles, n)
+        if len(_direct_bytes) > 256:
+            _direct_bytes.clear()
+        _direct_bytes[key] = sizes
+    ws_bytes, rws_bytes, tiles, n = sizes
+    if ws_bytes == 0:
+        return None
+    packed = torch.empty((B * G, _lib.RECORD_FLOATS), dtype=torch.float32, device=dev)
+    starts = _empty(tiles + 1, torch.int32, dev)
+    pairs = _empty(n, torch.int32, dev)
+    ws = _empty(ws_bytes, torch.uint8, dev)
+    rws = _empty(rws_bytes, torch.uint8, dev)
+    img = torch.empty((B, H, W, 3), dtype=torch.float32, device=dev)
+    final_T = last = tile_stop = None
+    if save_state:
+        final_T = torch.empty((B, H, W), dtype=torch.float32, device=dev)
+        last = torch.empty((B, H, W), dtype=torch.int32, device=dev)
+        tile_stop = _empty(tiles, torch.int32, dev)
+    check(_lib.lib().gsplat_hip_direct_render(
+        meta, ptr(means2d), ptr(conics), ptr(colors), ptr(opacities), ptr(depths), ptr(packed), ptr(starts), ptr(pairs),
+        ptr(img), ptr(final_T), ptr(last), ptr(tile_stop), ptr(ws), ws_bytes, ptr(rws), rws_bytes,
+        torch.cuda.current_stream(dev).cuda_stream), "gsplat_hip_direct_render")
+    return (BinState(None, packed, None, starts, pairs, n),
+            (img, final_T, last, tile_stop, (rws if save_state else None)))
+
+
 def _staged() -> bool:
     """True while per-stage timing of the binning or the forward is on: those calls then run one
     by one, each bracketed by its events."""

@@ -279,6 +279,21 @@ def _check_overflow(config: RasterConfig, st: _ops.BinState) -> None:
         )
 
 
+def _render(config: RasterConfig, meta: _lib.RasterMeta, flat, *, save_state: bool) -> tuple:
+    """(sliced result, None) or (None, whole result) of binning and forward: the direct path for small
+    scenes, slices for dense ones, else the one-call binning."""
+    if config.enable_overflow_fallback:  # (else the tiles' pair counts are checked: the whole binning)
+        whole = _ops.direct_render(meta, flat, save_state=save_state)
+        if whole is not None:
+            return None, whole
+        sliced = _slices.render(meta, flat, save_state=save_state)
+        if sliced is not None:
+            return sliced, None
+    whole = _ops.bin_and_render(meta, flat, save_state=save_state)
+    _check_overflow(config, whole[0])
+    return None, whole
+
+
 class _RasterizeProjectedGaussians(torch.autograd.Function):
     """Training path (reference _RasterizeProjectedGaussiansV8, v8 rasterize.py:444-681).
 
@@ -295,16 +310,14 @@ class _RasterizeProjectedGaussians(torch.autograd.Function):
                      depths_b.detach())
         # the first backward's outputs, allocated before the host waits on the binning
         ctx.grad_bufs = _ops.gradient_buffers(B, G, means2d_b.device)
-        # (a check of the tiles' pair counts needs the whole binning)
-        sliced = _slices.render(meta, flat, save_state=True) if config.enable_overflow_fallback else None
+        sliced, whole = _render(config, meta, flat, save_state=True)
         if sliced is not None:
             st, (img, final_T, last) = sliced
             ctx.save_for_backward(final_T, last, *st.tensors())
             ctx.sliced = st.plain()
             st.release()
         else:
-            st, (img, final_T, last, tile_stop, ws) = _ops.bin_and_render(meta, flat, save_state=True)
-            _check_overflow(config, st)
+            st, (img, final_T, last, tile_stop, ws) = whole
             ctx.save_for_backward(st.packed, st.tile_offsets, st.pairs, final_T, last, tile_stop, ws)
             ctx.sliced = None
         # the binning's status is read before the backward (by then the GPU is done with it)
@@ -347,12 +360,8 @@ def _rasterize_chunk_eval(means2d_b, conics_b, colors_b, opacities_b, depths_b, 
     B, G = means2d_b.shape[:2]
     meta = _meta(config, B, G)
     flat = _flat(means2d_b, conics_b, colors_b, opacities_b, depths_b)
-    sliced = _slices.render(meta, flat, save_state=False) if config.enable_overflow_fallback else None
-    if sliced is not None:
-        st, out = sliced
-    else:
-        st, out = _ops.bin_and_render(meta, flat, save_state=False)
-        _check_overflow(config, st)
+    sliced, whole = _render(config, meta, flat, save_state=False)
+    st, out = sliced if sliced is not None else whole
     st.check_status()
     return out[0]
 

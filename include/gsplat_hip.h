@@ -578,6 +578,32 @@ int gsplat_hip_sliced_backward(const gsplat_raster_meta* meta,
                                float* g_colors, float* g_opacities,
                                void* stream);
 
+/* ---- Small scenes ---------------------------------------------------------
+ * gsplat_hip_bin_render_forward for scenes of a few thousand splats at most,
+ * in fewer launches and without a pair count: every tile scans its image's
+ * splats.  Same image, stops and gradients.  It has no counterpart in the
+ * reference. */
+
+/* 0 where the scene is too large (4096 splats per image, 12 * 2^20 tiles x
+ * splats per image). */
+size_t gsplat_hip_direct_workspace_bytes(const gsplat_raster_meta* meta);
+
+/* packed float [B*G*16]; tile_starts int32 [T], binned_ids int32 [T*G]: tile
+ * t's gids in depth order from tile_starts[t] = t*G on; the outputs and the
+ * render workspace as gsplat_hip_render_forward's with n_pairs = T*G, out_last
+ * as gsplat_hip_bin_render_forward's.  gsplat_hip_render_backward takes
+ * tile_starts as its tile_offsets and n_pairs = T*G. */
+int gsplat_hip_direct_render(const gsplat_raster_meta* meta,
+                             const float* means2d, const float* conics,
+                             const float* colors, const float* opacities,
+                             const float* depths, float* packed,
+                             int32_t* tile_starts, int32_t* binned_ids,
+                             float* out_rgb, float* out_final_T,
+                             int32_t* out_last, int32_t* out_tile_stop,
+                             void* workspace, size_t workspace_bytes,
+                             void* render_workspace,
+                             size_t render_workspace_bytes, void* stream);
+
 #ifdef __cplusplus
 }
 #endif
