@@ -276,6 +276,15 @@ constexpr int kSegSplats = 128;     // multiple of kBatch
 constexpr int kHandoff = kHandoffPairs;  // multiple of kSegSplats
 static_assert(kHandoff % kSegSplats == 0, "hand-off at a segment boundary");
 constexpr int kLongStrips = 1;      // strips per wavefront of the long kernel
+// Images of up to this many tiles are composited with a wavefront per strip
+// instead of one per tile, and walked back with one per two strips: one per
+// tile would leave most of the chip's 8192 wavefronts idle and each with four
+// strips in a row.  Forward with its continuation, backward: 54 tiles of 300
+// splats 20 -> 10 us; 1430 tiles of 100 pairs 31 -> 23 us, 49 -> 41 us (one
+// per strip, which reduces every splat four times, 44); 1024 tiles of 10 pairs
+// 8.8 -> 6.4 us, 9.2 -> 7.9 us (10.6).
+constexpr int kStripTiles = 2048;
+constexpr int kFewTilesPix = 2;  // strips per wavefront of their backward
 
 struct HeavyState {      // all null: every tile is walked whole by one wave
   int32_t* counters;     // [0] slots handed out, [1] tiles handed off
@@ -651,26 +660,46 @@ __device__ __forceinline__ void long_batch(const Staged& S, int n, int idx1,
 // saved state with the same per-pixel operations, so the result is bit for
 // bit the one-wavefront walk's.  Workgroup b takes hand-off items b,
 // b + gridDim.x, ...
-template <int kSpW>
+// kWhole: the whole forward of images of few tiles, whose one wavefront per
+// tile would leave most of the chip idle (launch_render_forward): workgroup b
+// walks tile b from its start, with render_fwd_kernel's duties (report,
+// all_last).
+template <int kSpW, bool kWhole>
 __global__ __launch_bounds__(256 / kSpW) void render_fwd_long_kernel(
     RasterParams P, const float4* __restrict__ packed,
     const int32_t* __restrict__ tile_offsets,
     const int32_t* __restrict__ binned, float* __restrict__ out_rgb,
     float* __restrict__ out_T, int32_t* __restrict__ out_last,
-    int32_t* __restrict__ out_tile_stop, HeavyState H, TileSet tiles) {
+    int32_t* __restrict__ out_tile_stop, HeavyState H, TileSet tiles,
+    HostReport R, bool all_last) {
   __shared__ Staged S;
   __shared__ int sh_slot;
   __shared__ int sh_plain;  // batch_plain of the staged batch
+  __shared__ int sh_stop, sh_live;
   const int lane = (int)threadIdx.x & 63;
   const int s0 = __builtin_amdgcn_readfirstlane(((int)threadIdx.x >> 6) * kSpW);
   const int t0 = 64 * s0 + lane;  // in-tile index of the first strip's pixel
-  const int n_items = H.counters[1];
+  const int n_items = kWhole ? (int)gridDim.x : H.counters[1];
   const float t_thr = P.trans_thr;
   const float max_alpha = fminf(P.max_alpha, 1.0f);
+  if (kWhole && blockIdx.x == 0 && threadIdx.x == 0) {
+    if (R.host != nullptr) write_host_report(R);
+    H.counters[2] = H.rec != nullptr ? H.max_slots : -1;
+  }
   for (int item = blockIdx.x; item < n_items; item += gridDim.x) {
     __syncthreads();  // the previous tile's reads of S and sh_slot are done
-    const int tile = H.handoff[item];
-    int tail = H.handoff_tail[item];  // used by thread 0
+    int tile, tail = -1;  // tail: used by thread 0
+    if (kWhole) {
+      tile = xcd_remap(item, n_items);
+      if (tiles.list != nullptr) tile = tiles.list[tile];
+      if (threadIdx.x == 0) {
+        sh_stop = sh_live = 0;
+        if (H.rec != nullptr) H.tile_slot[tile] = -1;
+      }
+    } else {
+      tile = H.handoff[item];
+      tail = H.handoff_tail[item];
+    }
     const TileCoord tc = tile_coord_of(P, tile);
     const int x = tc.x0 + (lane & 15);
     const float px = (float)x + 0.5f;
@@ -684,20 +713,26 @@ __global__ __launch_bounds__(256 / kSpW) void render_fwd_long_kernel(
       valid[k] = (x < P.width) && (y < P.height);
       py[k] = (float)y + 0.5f;
       pix[k] = ((int64_t)tc.batch * P.height + y) * P.width + x;
-      T[k] = H.hand_T[(int64_t)item * 256 + t0 + 64 * k];
-      last[k] = (valid[k] && out_last != nullptr) ? out_last[pix[k]] : 0;
+      if (kWhole) {
+        T[k] = valid[k] ? 1.0f : 0.0f;
+        last[k] = 0;
+      } else {
+        T[k] = H.hand_T[(int64_t)item * 256 + t0 + 64 * k];
+        last[k] = (valid[k] && out_last != nullptr) ? out_last[pix[k]] : 0;
+      }
       cr[k] = cg[k] = cb[k] = 0.0f;
     }
     const int start = tile_offsets[tile];
     const int end = tiles.ends[tile];
-    int seg_cur = kHandoff / kSegSplats;
-    for (int base = start + kHandoff; base < end; base += kBatch) {
+    constexpr int kFrom = kWhole ? 0 : kHandoff;
+    int seg_cur = kFrom / kSegSplats;
+    for (int base = start + kFrom; base < end; base += kBatch) {
       bool alive = false;
 #pragma unroll
       for (int k = 0; k < kSpW; ++k) alive |= T[k] > t_thr;
       if (!__syncthreads_or(alive)) break;  // uniform; frees S
       // (the boundary at kHandoff was closed by render_fwd_kernel)
-      if (base > start + kHandoff && (base - start) % kSegSplats == 0) {
+      if (base > start + kFrom && (base - start) % kSegSplats == 0) {
         if (threadIdx.x == 0) sh_slot = next_segment(H, tile, seg_cur, tail);
         __syncthreads();
         end_segment<kSpW>(P, tc, out_rgb, H, sh_slot, seg_cur, valid, cr, cg,
@@ -722,15 +757,29 @@ __global__ __launch_bounds__(256 / kSpW) void render_fwd_long_kernel(
                                 max_alpha, T, cr, cg, cb, last);
     }
     __syncthreads();  // sh_slot of the last boundary has been read
-    if (threadIdx.x == 0) sh_slot = next_segment(H, tile, seg_cur, tail);
-    __syncthreads();
-    last_segment<kSpW>(P, tc, out_rgb, H, sh_slot, valid, cr, cg, cb, T, t0);
+    if (!kWhole || seg_cur > 0) {
+      if (threadIdx.x == 0) sh_slot = next_segment(H, tile, seg_cur, tail);
+      __syncthreads();
+      last_segment<kSpW>(P, tc, out_rgb, H, sh_slot, valid, cr, cg, cb, T, t0);
+    }
+    // (kWhole: last for the strips where a pixel stopped, or for all)
+    bool put_last = true;
+    if (kWhole && !all_last) {
+      bool stop = false;
+#pragma unroll
+      for (int k = 0; k < kSpW; ++k) stop |= valid[k] && !(T[k] > t_thr);
+      put_last = __builtin_amdgcn_ballot_w64(stop) != 0;
+    }
     if (tiles.live != nullptr) {
       bool alive = false;
 #pragma unroll
       for (int k = 0; k < kSpW; ++k) alive |= T[k] > t_thr;
-      if (__builtin_amdgcn_ballot_w64(alive) != 0 && lane == 0)
-        tiles.live[tile] = 1u;
+      if (__builtin_amdgcn_ballot_w64(alive) != 0 && lane == 0) {
+        if (kWhole)
+          atomicOr(&sh_live, 1);
+        else
+          tiles.live[tile] = 1u;
+      }
     }
     int tile_max = 0;
 #pragma unroll
@@ -742,14 +791,26 @@ __global__ __launch_bounds__(256 / kSpW) void render_fwd_long_kernel(
         out_rgb[3 * pix[k] + 2] = cb[k] + T[k] * P.bg_b;
         if (out_T != nullptr) {
           out_T[pix[k]] = T[k];
-          out_last[pix[k]] = last[k];
+          if (put_last) out_last[pix[k]] = last[k];
         }
         tile_max = max(tile_max, last[k]);
       }
     }
     if (out_tile_stop != nullptr) {
       tile_max = wave_max_row3(tile_max);
-      if (lane == kLanes - 1) atomicMax(out_tile_stop + tile, tile_max);
+      if (lane == kLanes - 1) {
+        if (kWhole)
+          atomicMax(&sh_stop, tile_max);
+        else
+          atomicMax(out_tile_stop + tile, tile_max);
+      }
+    }
+    if (kWhole) {
+      __syncthreads();
+      if (threadIdx.x == 0) {
+        if (out_tile_stop != nullptr) out_tile_stop[tile] = sh_stop;
+        if (tiles.live != nullptr) tiles.live[tile] = (uint32_t)sh_live;
+      }
     }
   }
 }
@@ -873,11 +934,13 @@ __device__ __forceinline__ GradTarget opac_target(const GradOut& G) {
   return {G.g_opac, 4, 1.0f};
 }
 
-// Per-pixel state of the backward walk (4 pixels per lane).
+// Per-pixel state of the backward walk (kN pixels per lane, in the strips
+// strip0 .. strip0 + kN - 1).
+template <int kN>
 struct BwdPixels {
   float px;
-  float py[kPix], Tc[kPix], gr[kPix], gg[kPix], gb[kPix], gT[kPix];
-  int lk[kPix];
+  float py[kN], Tc[kN], gr[kN], gg[kN], gb[kN], gT[kN];
+  int lk[kN];
 };
 
 // Loads grad and saved state; T and gT start at final_T and the background
@@ -886,20 +949,21 @@ struct BwdPixels {
 // wavefronts that have one: a pixel above the threshold composited its whole
 // tile range (lk = 2^31 - 1), and the one-call forward stores last only for
 // the pixels that stopped.
+template <int kN>
 __device__ __forceinline__ void load_bwd_pixels(
-    const RasterParams& P, const TileCoord& tc,
+    const RasterParams& P, const TileCoord& tc, int strip0,
     const float* __restrict__ final_T, const int32_t* __restrict__ last_in,
-    const float* __restrict__ grad_rgb, BwdPixels& Q) {
+    const float* __restrict__ grad_rgb, BwdPixels<kN>& Q) {
   const int x = tc.x0 + tc.lx;
   Q.px = (float)x + 0.5f;
   // The lane's pixels are 4 rows apart: one 64-bit index, then increments.
   const int64_t pix0 = opaque64(
-      ((int64_t)tc.batch * P.height + slot_y(tc, 0)) * P.width + x);
+      ((int64_t)tc.batch * P.height + slot_y(tc, strip0)) * P.width + x);
   const int64_t strip = (int64_t)4 * P.width;
-  bool stopped[kPix];
+  bool stopped[kN];
 #pragma unroll
-  for (int k = 0; k < kPix; ++k) {
-    const int y = slot_y(tc, k);
+  for (int k = 0; k < kN; ++k) {
+    const int y = slot_y(tc, strip0 + k);
     const bool valid = (x < P.width) && (y < P.height);
     Q.py[k] = (float)y + 0.5f;
     if (valid) {
@@ -919,10 +983,10 @@ __device__ __forceinline__ void load_bwd_pixels(
   }
   bool any = false;
 #pragma unroll
-  for (int k = 0; k < kPix; ++k) any |= stopped[k];
+  for (int k = 0; k < kN; ++k) any |= stopped[k];
   if (__builtin_amdgcn_ballot_w64(any) != 0) {
 #pragma unroll
-    for (int k = 0; k < kPix; ++k)
+    for (int k = 0; k < kN; ++k)
       if (stopped[k])
         Q.lk[k] = __builtin_nontemporal_load(last_in + pix0 + k * strip);
   }
@@ -932,14 +996,16 @@ __device__ __forceinline__ void load_bwd_pixels(
 // early in the forward (T <= transmittance threshold).  Otherwise every pixel
 // composited every splat visible to it, so a splat at index >= last is
 // invisible there and the walk can skip the index test (kCheckLast = false).
+template <int kN>
 __device__ __forceinline__ bool needs_last_test(const RasterParams& P,
                                                 const TileCoord& tc,
-                                                const BwdPixels& Q) {
+                                                int strip0,
+                                                const BwdPixels<kN>& Q) {
   const int x = tc.x0 + tc.lx;
   bool need = false;
 #pragma unroll
-  for (int k = 0; k < kPix; ++k)
-    need |= (x >= P.width) | (slot_y(tc, k) >= P.height) |
+  for (int k = 0; k < kN; ++k)
+    need |= (x >= P.width) | (slot_y(tc, strip0 + k) >= P.height) |
             !(Q.Tc[k] > P.trans_thr);
   return __builtin_amdgcn_ballot_w64(need) != 0;
 }
@@ -952,11 +1018,11 @@ __device__ __forceinline__ bool needs_last_test(const RasterParams& P,
 // kPlain: every record has kPlainBit, so e <= 0 and the max_alpha gate are
 // not tested (they always pass).  kAcc: the totals go to the records at acc,
 // else to target and opac.
-template <bool kCheckLast, bool kPlain, bool kAcc>
+template <bool kCheckLast, bool kPlain, bool kAcc, int kN>
 __device__ __forceinline__ void bwd_batch(
     BwdShared& SH, uint32_t bmask, int n, int cstart, float max_alpha,
-    float* acc, const GradTarget& target, const GradTarget& opac,
-    BwdPixels& Q) {
+    float* acc, const GradTarget& target, const GradTarget& opac, int strip0,
+    BwdPixels<kN>& Q) {
   const Staged& S = SH.S;
   const int lane = threadIdx.x;
   const bool group_head = (lane & 7) == 0;
@@ -974,7 +1040,8 @@ __device__ __forceinline__ void bwd_batch(
   float S0 = 0.f, S1 = 0.f, S2 = 0.f;
   float acc_r = 0.f, acc_g = 0.f, acc_b = 0.f;
   for (int j = n - 1; j >= 0; --j) {
-    const uint32_t mask = __builtin_amdgcn_readlane(bmask, j);
+    uint32_t mask = __builtin_amdgcn_readlane(bmask, j);
+    if (kN < kPix) mask = (mask >> strip0) & ((1u << kN) - 1u);
     if (mask == 0u) continue;
     const float4 a2 = S.s2[j];
     const int i = cstart + j;
@@ -986,7 +1053,7 @@ __device__ __forceinline__ void bwd_batch(
     // (uniform; a ballot of the combined test would be materialised per lane)
     uint64_t hits = 0;
 #pragma unroll
-    for (int k = 0; k < kPix; ++k) {
+    for (int k = 0; k < kN; ++k) {
       if (!((mask >> k) & 1u)) continue;  // scalar branch
       // one combined test: composited in the forward (i < last) and visible
       const float dy = Q.py[k] - a0.y;
@@ -1069,11 +1136,12 @@ __device__ __forceinline__ void bwd_batch(
 
 // Reverse walk over the tile-range indices [lo, hi), one staged batch of 64
 // records at a time.
-template <bool kCheckLast, bool kAcc>
+template <bool kCheckLast, bool kAcc, int kN>
 __device__ __forceinline__ void bwd_walk(
     const RasterParams& P, const float4* __restrict__ packed,
     const int32_t* __restrict__ binned, uint32_t max_gid, int start, int lo,
-    int hi, const TileCoord& tc, BwdShared& SH, BwdPixels& Q, const GradOut& G) {
+    int hi, const TileCoord& tc, int strip0, BwdShared& SH, BwdPixels<kN>& Q,
+    const GradOut& G) {
   const GradTarget target = kAcc ? GradTarget{} : grad_target(G);
   const GradTarget opac = kAcc ? GradTarget{} : opac_target(G);
   const float max_alpha = fminf(P.max_alpha, 1.0f);
@@ -1086,11 +1154,11 @@ __device__ __forceinline__ void bwd_walk(
                            max_gid, SH.S);
     __syncthreads();
     if (batch_plain(bmask))
-      bwd_batch<kCheckLast, true, kAcc>(SH, bmask, n, cstart, max_alpha,
-                                        G.acc, target, opac, Q);
+      bwd_batch<kCheckLast, true, kAcc, kN>(SH, bmask, n, cstart, max_alpha,
+                                            G.acc, target, opac, strip0, Q);
     else
-      bwd_batch<kCheckLast, false, kAcc>(SH, bmask, n, cstart, max_alpha,
-                                         G.acc, target, opac, Q);
+      bwd_batch<kCheckLast, false, kAcc, kN>(SH, bmask, n, cstart, max_alpha,
+                                             G.acc, target, opac, strip0, Q);
   }
 }
 
@@ -1168,18 +1236,24 @@ struct BwdSource {
   const int32_t* list;  // the tiles walked, null: tile i
   int seg_blocks, tiles;
 };
-template <int kWaves, bool kAcc>
+// kN < 4: kN strips per work item, the item's 4 / kN blocks 8 apart (on one
+// XCD).
+template <int kWaves, bool kAcc, int kN>
 __global__ __launch_bounds__(kLanes)
 __attribute__((amdgpu_waves_per_eu(kWaves, 8))) void render_bwd_kernel(
     RasterParams P, BwdSource A, BwdSource B, int b_blocks,
     const float* __restrict__ final_T, const int32_t* __restrict__ last_in,
     const float* __restrict__ grad_rgb, GradOut G) {
   __shared__ BwdShared SH;
-  const bool in_b = (int)blockIdx.x < b_blocks;
+  constexpr int kParts = kPix / kN;
+  const int slot = (int)blockIdx.x >> 3;
+  const int strip0 = kN * (slot % kParts);
+  const int block = (slot / kParts) * 8 + ((int)blockIdx.x & 7);
+  const bool in_b = block < b_blocks;
   const BwdSource& W = in_b ? B : A;
   const HeavyState& H = W.H;
   const int32_t* __restrict__ tile_stop = W.tile_stop;
-  const int bid = (int)blockIdx.x - (in_b ? 0 : b_blocks);
+  const int bid = block - (in_b ? 0 : b_blocks);
   const int seg_blocks = W.seg_blocks;
   const bool seg = bid < seg_blocks;
   const int m = bid;
@@ -1200,24 +1274,24 @@ __attribute__((amdgpu_waves_per_eu(kWaves, 8))) void render_bwd_kernel(
     // waited for (an empty tile's loads are wasted: few tiles are empty)
     const int start = W.tile_offsets[tile];
     const TileCoord tc = tile_coord_of(P, tile);
-    BwdPixels Q;
-    load_bwd_pixels(P, tc, final_T, last_in, grad_rgb, Q);
+    BwdPixels<kN> Q;
+    load_bwd_pixels(P, tc, strip0, final_T, last_in, grad_rgb, Q);
     // (a tile walked as segments returns here)
     if (!seg && (hi <= 0 || heavy_backward(H, tile, hi))) return;
     {
       if (kseg < nseg - 1) {
         // Pixels composited past this segment: T and gT at its end from the
         // forward's segment records (Q.gT holds <g, bg>, Q.Tc T_final).
-        float cr[kPix], cg[kPix], cb[kPix];
+        float cr[kN], cg[kN], cb[kN];
 #pragma unroll
-        for (int k = 0; k < kPix; ++k) cr[k] = cg[k] = cb[k] = 0.0f;
-        const int t = opaque((int)threadIdx.x);
+        for (int k = 0; k < kN; ++k) cr[k] = cg[k] = cb[k] = 0.0f;
+        const int t = opaque((int)threadIdx.x + 64 * strip0);
         int sl = H.slot_next[m];
         for (int j = kseg + 1;
              j < nseg && (unsigned)sl < (unsigned)H.max_slots; ++j) {
           const float4* rj = H.rec + (int64_t)sl * 256 + t;
 #pragma unroll
-          for (int k = 0; k < kPix; ++k) {
+          for (int k = 0; k < kN; ++k) {
             const float4 v = rj[64 * k];
             cr[k] += v.x;
             cg[k] += v.y;
@@ -1227,7 +1301,7 @@ __attribute__((amdgpu_waves_per_eu(kWaves, 8))) void render_bwd_kernel(
         }
         const float4* rm = H.rec + (int64_t)m * 256 + t;
 #pragma unroll
-        for (int k = 0; k < kPix; ++k) {
+        for (int k = 0; k < kN; ++k) {
           if (Q.lk[k] > hi) {
             const float Te = rm[64 * k].w;  // > 0: the pixel was alive
             const float num = Q.gr[k] * cr[k] + Q.gg[k] * cg[k] +
@@ -1240,12 +1314,12 @@ __attribute__((amdgpu_waves_per_eu(kWaves, 8))) void render_bwd_kernel(
     }
     // Q.Tc holds T_final, or T at the segment's end for pixels alive past it
     // (T_end > T_final > threshold), so the test sees the final state.
-    if (needs_last_test(P, tc, Q))
-      bwd_walk<true, kAcc>(P, W.packed, W.binned, W.max_gid, start, lo, hi, tc,
-                           SH, Q, G);
+    if (needs_last_test(P, tc, strip0, Q))
+      bwd_walk<true, kAcc, kN>(P, W.packed, W.binned, W.max_gid, start, lo, hi,
+                               tc, strip0, SH, Q, G);
     else
-      bwd_walk<false, kAcc>(P, W.packed, W.binned, W.max_gid, start, lo, hi,
-                            tc, SH, Q, G);
+      bwd_walk<false, kAcc, kN>(P, W.packed, W.binned, W.max_gid, start, lo, hi,
+                                tc, strip0, SH, Q, G);
   }
 }
 
@@ -1373,6 +1447,18 @@ int launch_render_forward(const RasterParams& P, const float* packed,
     const int rc = launch_zero2(z[0].p, z[0].n, z[1].p, z[1].n, stream);
     if (rc) return rc;
   }
+  // Few tiles: four wavefronts a tile from the start (one would leave the
+  // chip's 8192 wavefronts mostly idle and walk four strips in a row); no
+  // tile is handed off then.
+  if (H.counters != nullptr && n_tiles <= kStripTiles) {
+    launch_timed("render_fwd_kernel", render_fwd_long_kernel<kLongStrips, true>,
+                 dim3((unsigned)n_tiles), dim3(256 / kLongStrips), stream, t0,
+                 t1, P, pk, tile_offsets, binned_ids, out_rgb, out_T, out_last,
+                 out_tile_stop, H, set,
+                 report != nullptr ? *report : HostReport{},
+                 !(flags & kForwardStoppedLast));
+    return check_launch("render_fwd_kernel");
+  }
   // the continuation follows in this call: it ends the timed span
   const bool more = !(flags & kForwardNoLong) && workspace != nullptr;
   launch_timed("render_fwd_kernel", render_fwd_kernel, dim3((unsigned)n_tiles), dim3(kLanes),
@@ -1398,11 +1484,11 @@ int launch_render_forward_long(const RasterParams& P, const float* packed,
   const HeavyState H = forward_state(P, n_pairs, workspace, out_T);
   // Workgroups stride over the hand-off list (its length is on the device).
   const unsigned grid = (unsigned)std::min<int64_t>(P.num_tiles, 2048);
-  launch_timed("render_fwd_long_kernel", render_fwd_long_kernel<kLongStrips>, dim3(grid),
+  launch_timed("render_fwd_long_kernel", render_fwd_long_kernel<kLongStrips, false>, dim3(grid),
                dim3(256 / kLongStrips), stream, nullptr, stop, P,
                reinterpret_cast<const float4*>(packed), tile_offsets,
                binned_ids, out_rgb, out_T, out_last, out_tile_stop, H,
-               tile_set(tiles, tile_offsets));
+               tile_set(tiles, tile_offsets), HostReport{}, true);
   return check_launch("render_fwd_long_kernel");
 }
 
@@ -1437,11 +1523,16 @@ int launch_backward_walk(const RasterParams& P, const BwdSource& A,
   // tile on average the short-tile variant is faster)
   const bool short_tiles = n_pairs <= (int64_t)64 * P.num_tiles;
   const int b_blocks = B.seg_blocks + ((B.tiles + 7) & ~7);
+  const int blocks = b_blocks + A.seg_blocks + ((A.tiles + 7) & ~7);
+  // few tiles: more wavefronts a tile, as in the forward
+  const bool strips = G.acc != nullptr && A.tiles + B.tiles <= kStripTiles;
   launch_timed("render_bwd_kernel",
-               G.acc == nullptr ? render_bwd_kernel<6, false>
-               : short_tiles    ? render_bwd_kernel<7, true>
-                                : render_bwd_kernel<6, true>,
-               dim3((unsigned)(b_blocks + A.seg_blocks + A.tiles)),
+               strips           ? render_bwd_kernel<6, true, kFewTilesPix>
+               : G.acc == nullptr ? render_bwd_kernel<6, false, kPix>
+               : short_tiles    ? render_bwd_kernel<7, true, kPix>
+                                : render_bwd_kernel<6, true, kPix>,
+               dim3((unsigned)(strips ? kPix / kFewTilesPix * blocks
+                                       : blocks)),
                dim3(kLanes), stream, t0, t1, P, A, B, b_blocks, final_T, last,
                grad_rgb, G);
   return check_launch("render_bwd_kernel");

@@ -16,7 +16,7 @@
 //   whose box holds the tile compacted in LDS, then tested exactly 64 at a
 //   time.  Bound by the tiles x splats box tests: 4.5 us at 1024 tiles x
 //   512 splats, 14 at 1430 x 4001.
-// Both together: 512 splats at 512 x 512 34 -> 10 us, five images of 4001
+// Both together: 512 splats at 512 x 512 41 -> 10 us, five images of 4001
 // splats 46 -> 33 us, and the forward's caller no longer waits.
 //
 // Compiled with -ffp-contract=off, like binning.hip: the lists are those of

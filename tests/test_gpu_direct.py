@@ -78,3 +78,33 @@ def test_direct_limits():
         sc = make_scene_2d(0, seed=1, G=G, H=H, W=W)
         meta = _lib.make_raster_meta(H, W, 1, G, 1 / 255, 1e-4, (0, 0, 0))
         assert _ops.direct_render(meta, _flat(sc, 1, G), save_state=False) is None
+
+
+@pytest.mark.parametrize("G,H,W", [
+    (3000, 16, 16),        # one tile
+    (20000, 511, 1009),    # 2048 tiles, the most that are composited by several wavefronts each
+    (20000, 513, 990),     # 2046 tiles of 33 rows, the last cut
+    (20000, 512, 1025),    # 2080 tiles: one wavefront each
+])
+def test_wavefronts_per_tile(G, H, W):
+    """Image, stops and gradients with the workspace (several wavefronts per tile in images of few
+    tiles, continuation in others) against those without it (one wavefront per tile throughout)."""
+    L = _lib.lib()
+    sc = make_scene_2d(0, seed=3, G=G, B=1, H=H, W=W)
+    sc["opacities"] = 0.3 * sc["opacities"]
+    flat = _flat(sc, 1, G)
+    meta = _lib.make_raster_meta(H, W, 1, G, 1 / 255, 1e-4, (0.1, 0.2, 0.3))
+    _ops._capacity.pop((0, 1, G, H, W), None)
+    st = _ops.bin_gaussians(meta, *flat)
+    out = _ops.render_forward(meta, st, save_state=True)
+    one = [torch.empty_like(t) for t in out[:4]]
+    p = _lib.ptr
+    _lib.check(L.gsplat_hip_render_forward(meta, p(st.packed), p(st.tile_offsets), p(st.pairs), *map(p, one),
+                                           st.capacity, None, 0, _lib.stream_of(one[0])), "render_forward")
+    for a, b in zip(out[:4], one):
+        assert torch.equal(a, b)
+    w = torch.rand(1, H, W, 3, generator=torch.Generator().manual_seed(2)).cuda()
+    got = _ops.render_backward(meta, st, *out[1:4], w, out[4])
+    want = _ops.render_backward(meta, st, *one[1:], w, None)
+    for a, b in zip(got, want):
+        torch.testing.assert_close(a, b, rtol=1e-4, atol=1e-5 * float(b.abs().max()))
