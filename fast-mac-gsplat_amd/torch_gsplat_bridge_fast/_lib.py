@@ -144,6 +144,24 @@ def load(path: str = LIB_PATH) -> ctypes.CDLL:
     return lib
 
 
+_host_module = None
+
+
+def host():
+    """The extension module with the host path (csrc/host.cpp), bound to the loaded library."""
+    global _host_module
+    if _host_module is None:
+        load()
+        try:
+            from . import _host
+        except ImportError as e:
+            raise RuntimeError("_host.so (the host path) is missing or was built for another torch; build it with "
+                               "`make -C fast-mac-gsplat_amd/csrc`") from e
+        _host.bind(LIB_PATH)
+        _host_module = _host
+    return _host_module
+
+
 def lib() -> ctypes.CDLL:
     return _lib if _lib is not None else load()
 

@@ -48,6 +48,7 @@ def set_timing(enabled: bool, ops=None, pool: int = 0, every: int = 1) -> None:
     global _timing, _timing_ops, _pool, _every, _seen
     _timing = [] if enabled else None
     _timing_ops = set(ops) if ops is not None else None
+    _lib.host().set_timed(enabled)
     _every, _seen = max(1, int(every)), 0
     _pool = []
     if enabled and pool:
@@ -67,6 +68,7 @@ def pop_timing() -> list:
     global _timing
     out = _timing or []
     _timing = None
+    _lib.host().set_timed(False)
     return out
 
 
@@ -161,6 +163,15 @@ def _headroom(n: int) -> int:
     return min(cap, MAX_PAIRS) if n <= MAX_PAIRS else cap
 
 
+def note_pairs(key: tuple, n: int) -> int:
+    """Remembers a binning of n pairs for a shape: the capacity follows when n is above it or far
+    below.  Returns the capacity."""
+    cap = _capacity.get(key, 0)
+    if n > cap or 2 * _headroom(n) < cap:
+        _capacity[key] = _headroom(n)
+    return _capacity.get(key, cap)
+
+
 @dataclass
 class BinState:
     perm: Optional[Tensor]          # int32 [BG]  depth rank -> original index within image
@@ -204,9 +215,7 @@ class BinState:
         if n < 0:
             raise RuntimeError("pair count overflowed int32")
         if self._key is not None:
-            cap = _capacity.get(self._key, 0)
-            if n > cap or 2 * _headroom(n) < cap:
-                _capacity[self._key] = _headroom(n)
+            note_pairs(self._key, n)
         return n <= self.capacity
 
     @property

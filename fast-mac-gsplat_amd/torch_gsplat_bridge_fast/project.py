@@ -18,7 +18,7 @@ import torch
 from torch import Tensor
 
 from . import _lib, _ops
-from .rasterize import RasterConfig, _rasterize_batched, _runtime_validate
+from .rasterize import RasterConfig, _make_plan, _plan, _rasterize_batched, _runtime_validate
 
 
 def _normalize_3d_inputs(means3d, scales, quats, opacities):
@@ -160,9 +160,25 @@ def _project_pinhole_gaussians_batched(means3d_b, scales_b, quats_b, opacities_b
                                           float(near_plane))
 
 
+def _project_plain(means3d, scales, quats, opacities, fx, fy, cx, cy, camera_to_world, near_plane):
+    """project_pinhole_gaussians by the host path (csrc/host.cpp), None where its inputs are not plain
+    tensors of the right shapes."""
+    h = _lib.host()
+    B = h.project_images(means3d, scales, quats, opacities)
+    if B == 0:
+        return None
+    dev, dt = means3d.device, means3d.dtype
+    return h.project(means3d, scales, quats, opacities,
+                     _camera_to_world_batch(camera_to_world, B, dev, dt),
+                     _camera_params(fx, fy, cx, cy, B, dev, dt), float(near_plane))
+
+
 def project_pinhole_gaussians(means3d: Tensor, scales: Tensor, quats: Tensor, opacities: Tensor, fx, fy, cx, cy,
                               camera_to_world=None, near_plane: float = 1e-4):
     """Returns (means2d, conics, projected_opacities, depths)."""
+    out = _project_plain(means3d, scales, quats, opacities, fx, fy, cx, cy, camera_to_world, near_plane)
+    if out is not None:
+        return out
     _check_3d_inputs(means3d, scales, quats, opacities)
     m_b, s_b, q_b, o_b, was_batched = _normalize_3d_inputs(means3d, scales, quats, opacities)
     out = _project_pinhole_gaussians_batched(m_b.contiguous(), s_b.contiguous(), q_b.contiguous(), o_b.contiguous(),
@@ -178,17 +194,41 @@ def rasterize_pinhole_gaussians(means3d: Tensor, scales: Tensor, quats: Tensor, 
                                 config: RasterConfig | None = None) -> Tensor:
     if config is None:
         raise ValueError("config is required")
+    plan = _plan(config)
+    if plan is not None:
+        flat = _project_plain(means3d, scales, quats, opacities, fx, fy, cx, cy, camera_to_world, near_plane)
+        if flat is not None:
+            means2d, conics, opac, depths = flat
+            out = plan.run(means2d, conics, colors, opac, depths, False)
+            if out is not None:
+                return out
+            was_batched = means3d.ndim == 3
+            if not was_batched:
+                means2d, conics, opac, depths = (t.unsqueeze(0) for t in flat)
+            return _rasterize_colored(means2d, conics, colors, opac, depths, was_batched, config)
     _check_3d_inputs(means3d, scales, quats, opacities)
     m_b, s_b, q_b, o_b, was_batched = _normalize_3d_inputs(means3d, scales, quats, opacities)
+    _check_colors(colors, m_b, was_batched)
+    _runtime_validate(config)
+    _make_plan(config)
+    means2d, conics, opac, depths = _project_pinhole_gaussians_batched(
+        m_b.contiguous(), s_b.contiguous(), q_b.contiguous(), o_b.contiguous(), fx, fy, cx, cy, camera_to_world,
+        near_plane)
+    return _rasterize_colored(means2d, conics, colors, opac, depths, was_batched, config)
+
+
+def _check_colors(colors, m_b, was_batched) -> Tensor:
     B, G = m_b.shape[:2]
     colors_b = _normalize_colors(colors, B, G, was_batched)
     if colors_b.device != m_b.device:
         raise ValueError("colors must be on the same device as means3d")
     if colors_b.dtype != torch.float32:
         raise ValueError("colors must be float32")
-    _runtime_validate(config)
-    means2d, conics, opac, depths = _project_pinhole_gaussians_batched(
-        m_b.contiguous(), s_b.contiguous(), q_b.contiguous(), o_b.contiguous(), fx, fy, cx, cy, camera_to_world,
-        near_plane)
+    return colors_b
+
+
+def _rasterize_colored(means2d, conics, colors, opac, depths, was_batched, config) -> Tensor:
+    """The rasterizer on batched projected splats."""
+    colors_b = _check_colors(colors, means2d, was_batched)
     out = _rasterize_batched(means2d, conics, colors_b.contiguous(), opac, depths, config, depth_grad=False)
     return out if was_batched else out.squeeze(0)

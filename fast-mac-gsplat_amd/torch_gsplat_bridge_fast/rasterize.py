@@ -428,12 +428,56 @@ def _rasterize_batched(means2d_b, conics_b, colors_b, opacities_b, depths_b, con
     return torch.cat(outs, dim=0) if len(outs) > 1 else outs[0]
 
 
+# Configs whose first call has gone through the checks below: the host path's plan of each (None: not
+# for this config).
+_plans: dict = {}
+
+
+def _plan(config: RasterConfig):
+    """The host path (csrc/host.cpp) of a config that an earlier call has validated, else None."""
+    if _ops._timing is not None and _ops._staged():
+        return None
+    try:
+        return _plans.get((config, os.environ.get("GSP_TILE_SIZE"), os.environ.get("GSP_CHUNK"),
+                           os.environ.get("GSP_FAST_CAP")))
+    except TypeError:   # a field that is not hashable (e.g. a list background)
+        return None
+
+
+def _make_plan(config: RasterConfig) -> None:
+    """Remembers the plan of a config that a whole call has just used."""
+    key = (config, os.environ.get("GSP_TILE_SIZE"), os.environ.get("GSP_CHUNK"), os.environ.get("GSP_FAST_CAP"))
+    try:
+        if key in _plans:
+            return
+    except TypeError:
+        return
+    plan = None
+    if config.enable_overflow_fallback:   # (else the tiles' pair counts are checked)
+        plan = _lib.host().Plan(
+            int(config.height), int(config.width), float(config.alpha_threshold),
+            float(config.transmittance_threshold), [float(v) for v in config.background], _EPS, _MAX_ALPHA,
+            ("auto", "flatten", "serial").index(config.batch_strategy), int(config.batch_launch_limit_tiles),
+            int(config.batch_launch_limit_gaussians),
+            config.batch_strategy == "auto" and config.max_pairs_per_launch > 0, _ops._capacity, _ops.note_pairs,
+            _slices.MIN_PAIRS, _slices.MIN_PAIRS_PER_TILE)
+    if len(_plans) > 256:
+        _plans.clear()
+    _plans[key] = plan
+
+
 def rasterize_projected_gaussians(means2d: Tensor, conics: Tensor, colors: Tensor, opacities: Tensor,
                                   depths: Tensor, config: RasterConfig) -> Tensor:
+    plan = _plan(config)
+    if plan is not None:
+        out = plan.run(means2d, conics, colors, opacities, depths, True)
+        if out is not None:
+            return out
     _check_inputs(means2d, conics, colors, opacities, depths)
     means2d_b, conics_b, colors_b, opacities_b, depths_b, was_batched = _normalize_inputs(
         means2d, conics, colors, opacities, depths)
     _runtime_validate(config)
+    _make_plan(config)
     out = _rasterize_batched(means2d_b, conics_b, colors_b, opacities_b, depths_b, config)
     # squeeze, not out[0]: the backward of an index zero-fills an image and copies the gradient into
     # it (26 + 91 us at 4096 x 4096), that of squeeze is a view

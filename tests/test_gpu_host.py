@@ -1,0 +1,215 @@
+"""The host path in C++ (csrc/host.cpp) against the Python path that takes every
+call it leaves: same results, gradients and refusals, and it does leave what is
+not the plain case."""
+import threading
+
+import pytest
+import torch
+
+from torch_gsplat_bridge_fast import (RasterConfig, project_pinhole_gaussians, rasterize_pinhole_gaussians,
+                                      rasterize_projected_gaussians)
+from torch_gsplat_bridge_fast import project as project_mod
+from torch_gsplat_bridge_fast import rasterize as rasterize_mod
+from torch_gsplat_bridge_fast.scenes import make_scene_2d, make_scene_3d
+
+pytestmark = pytest.mark.gpu
+
+KEYS = ("means2d", "conics", "colors", "opacities", "depths")
+SIZES = [(1, 300, 96, 131), (2, 5000, 130, 170)]   # the direct path, the one-call binning
+
+
+def _scene(B, G, H, W, batched=True, seed=1):
+    sc = make_scene_2d(0, seed=seed, G=G, B=B, H=H, W=W)
+    ts = [sc[k].cuda() for k in KEYS]
+    return ts if batched else [t[0].contiguous() for t in ts]
+
+
+def _plan(cfg, ts):
+    """The config's plan (a first call makes it, and the shape's capacity)."""
+    with torch.no_grad():
+        rasterize_projected_gaussians(*ts, cfg)
+        rasterize_projected_gaussians(*ts, cfg)
+    plan = rasterize_mod._plan(cfg)
+    assert plan is not None
+    return plan
+
+
+def _python(ts, cfg):
+    if ts[0].ndim == 2:
+        return rasterize_mod._rasterize_batched(*(t.unsqueeze(0) for t in ts), cfg).squeeze(0)
+    return rasterize_mod._rasterize_batched(*ts, cfg)
+
+
+def _leaves(ts, need):
+    return [t.clone().requires_grad_(bool(n)) for t, n in zip(ts, need)]
+
+
+@pytest.mark.parametrize("B,G,H,W", SIZES)
+@pytest.mark.parametrize("need", [(1, 1, 1, 1, 1), (1, 1, 1, 1, 0), (0, 1, 0, 0, 0), (0, 0, 0, 1, 1)])
+def test_matches_python(B, G, H, W, need):
+    batched = B > 1
+    ts = _scene(B, G, H, W, batched)
+    cfg = RasterConfig(height=H, width=W, background=(0.1, 0.2, 0.3))
+    plan = _plan(cfg, ts)
+    w = torch.rand((B, H, W, 3) if batched else (H, W, 3), generator=torch.Generator().manual_seed(2)).cuda()
+    a, b = _leaves(ts, need), _leaves(ts, need)
+    img = plan.run(*a, True)
+    ref = _python(b, cfg)
+    assert img is not None and img.shape == ref.shape and torch.equal(img, ref) and img.requires_grad
+    img.backward(w, retain_graph=True)
+    img.backward(w)
+    ref.backward(w, retain_graph=True)
+    ref.backward(w)
+    for x, y in zip(a, b):
+        assert (x.grad is None) == (y.grad is None)
+        if x.grad is not None:
+            assert x.grad.shape == x.shape
+            torch.testing.assert_close(x.grad, y.grad, rtol=1e-4, atol=1e-5 * float(y.grad.abs().max()) + 1e-7)
+    with pytest.raises(RuntimeError, match="second time"):
+        img.backward(w)
+    with torch.no_grad():
+        out = plan.run(*a, True)
+    assert torch.equal(out, ref) and not out.requires_grad
+
+
+@pytest.mark.parametrize("B,G,H,W", SIZES)
+def test_strides_hooks_and_streams(B, G, H, W):
+    """Strided inputs, saved-tensor hooks (the buffers go to host memory and back), another stream and
+    an upstream graph give the plain call's gradients."""
+    ts = _scene(B, G, H, W)
+    cfg = RasterConfig(height=H, width=W)
+    _plan(cfg, ts)
+    w = torch.rand(B, H, W, 3, generator=torch.Generator().manual_seed(2)).cuda()
+
+    def step(leaves, args, grad=w):
+        img = rasterize_projected_gaussians(*args, cfg)
+        img.backward(grad)
+        return img.detach(), [x.grad for x in leaves[:4]]
+
+    leaves = _leaves(ts, (1, 1, 1, 1, 0))
+    want = step(leaves, leaves)
+
+    def close(got):
+        assert torch.equal(got[0], want[0])
+        for x, y in zip(got[1], want[1]):
+            torch.testing.assert_close(x, y, rtol=1e-4, atol=1e-5 * float(y.abs().max()))
+
+    wide = [torch.stack([t, t], dim=-1)[..., 0].detach().requires_grad_(k < 4) for k, t in enumerate(ts)]
+    assert not any(t.is_contiguous() for t in wide)
+    close(step(wide, wide))
+    x = _leaves(ts, (1, 1, 1, 1, 0))
+    close(step(x, [t * 1.0 for t in x[:4]] + [x[4]], w.transpose(1, 2).contiguous().transpose(1, 2)))
+    x = _leaves(ts, (1, 1, 1, 1, 0))
+    packed = []
+    with torch.autograd.graph.saved_tensors_hooks(lambda t: packed.append(t.shape) or t.cpu(), lambda t: t.cuda()):
+        close(step(x, x))
+    assert packed
+    x = _leaves(ts, (1, 1, 1, 1, 0))
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        got = step(x, x)
+    torch.cuda.current_stream().wait_stream(side)
+    close(got)
+
+
+def test_threads_share_a_plan():
+    """Threads with streams of their own, one config, different scenes."""
+    B, G, H, W = SIZES[1]
+    cfg = RasterConfig(height=H, width=W)
+    scenes = [_scene(B, G, H, W, seed=s) for s in range(4)]
+    _plan(cfg, scenes[0])
+    want = [_python(s, cfg) for s in scenes]
+    torch.cuda.synchronize()
+    bad = []
+
+    def work(k):
+        stream = torch.cuda.Stream()
+        with torch.cuda.stream(stream), torch.no_grad():
+            for _ in range(20):
+                img = rasterize_projected_gaussians(*scenes[k], cfg)
+                stream.synchronize()
+                if not torch.equal(img, want[k]):
+                    bad.append(k)
+
+    threads = [threading.Thread(target=work, args=(k,)) for k in range(4)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not bad
+
+
+def test_refusals_stay():
+    """With the config's plan known, inputs that were refused are refused with the same errors."""
+    B, G, H, W = SIZES[0]
+    ts = _scene(B, G, H, W)
+    cfg = RasterConfig(height=H, width=W)
+    _plan(cfg, ts)
+
+    def bad(k, t, match, err=ValueError):
+        args = list(ts)
+        args[k] = t
+        with pytest.raises(err, match=match):
+            rasterize_projected_gaussians(*args, cfg)
+
+    bad(0, ts[0].double(), "must be float32")
+    bad(1, ts[1].cpu(), "same device")
+    bad(1, ts[1][:, :-1], "dimensions must match")
+    bad(2, ts[2][..., :2], "last dim = 3")
+    bad(3, ts[3][0], "rank")
+    with pytest.raises(ValueError, match="ROCm device"):
+        rasterize_projected_gaussians(*(t.cpu() for t in ts), cfg)
+    with pytest.raises(ValueError, match="at least one Gaussian"):
+        rasterize_projected_gaussians(*(t[:, :0] for t in ts), cfg)
+    with pytest.raises(RuntimeError):   # no vmap rule
+        torch.vmap(lambda m: rasterize_projected_gaussians(m, *ts[1:], cfg))(torch.stack([ts[0]] * 2))
+    with pytest.raises(Exception):      # no jvp
+        torch.func.jvp(lambda m: rasterize_projected_gaussians(m, *ts[1:], cfg), (ts[0],), (ts[0],))
+    # vmap used in this thread before does not keep later calls off the host path
+    assert rasterize_mod._plan(cfg).run(*ts, True) is not None
+
+
+@pytest.mark.parametrize("batched", [False, True])
+def test_projection_matches_python(batched):
+    G = 3000
+    sc = make_scene_3d(seed=4, G=G, H=200, W=300)
+    ts = [sc[k].cuda() for k in ("means3d", "scales", "quats", "opacities", "colors")]
+    ts = [torch.cat([t, t.flip(1)]) if batched else t[0].contiguous() for t in ts]
+    ts[3] = ts[3].unsqueeze(-1)   # [.., 1] opacities
+    c2w = sc["camera_to_world"].cuda()
+    cfg = RasterConfig(height=200, width=300)
+    cam = (250.0, 250.0, 150.0, 100.0)
+
+    def run(native):
+        if not native:
+            project_mod._project_plain, keep = (lambda *a: None), project_mod._project_plain
+        try:
+            x = [t.clone().requires_grad_(True) for t in ts]
+            pose = c2w.clone().requires_grad_(True)
+            out = project_pinhole_gaussians(*x[:4], *cam, camera_to_world=pose)
+            (out[0].sum() * 1e-3 + out[1].square().sum() + out[2].sum() + 0.1 * out[3].sum()).backward()
+            g1 = [t.grad.clone() for t in x[:4]] + [pose.grad.clone()]
+            for t in (*x, pose):
+                t.grad = None
+            imgs = []
+            for _ in range(3):
+                img = rasterize_pinhole_gaussians(*x, *cam, camera_to_world=pose, config=cfg)
+                imgs.append(img.detach())
+            img.square().mean().backward()
+            return out, g1, imgs[-1], [t.grad for t in x] + [pose.grad]
+        finally:
+            if not native:
+                project_mod._project_plain = keep
+
+    a, b = run(True), run(False)
+    for x, y in zip(a[0], b[0]):
+        assert x.shape == y.shape and torch.equal(x, y)
+    assert torch.equal(a[2], b[2])
+    for x, y in zip(a[1] + a[3], b[1] + b[3]):
+        assert x.shape == y.shape
+        torch.testing.assert_close(x, y, rtol=1e-4, atol=1e-5 * float(y.abs().max()))
+    with pytest.raises(ValueError, match="quats must have shape"):
+        project_pinhole_gaussians(ts[0], ts[1], ts[2][..., :3], ts[3], *cam)
+    with pytest.raises(ValueError, match="must be float32"):
+        project_pinhole_gaussians(ts[0].double(), *ts[1:4], *cam)
