@@ -1326,6 +1326,297 @@ __global__ __launch_bounds__(kBucketThreads) void bucket_sort_kernel(
     *A.long_flag = 1;
 }
 
+// ---- The tile-sorted binning (launch_tile_sorted): three launches instead of
+// five for scenes of up to 128K splats.  Latency bounds them: a chain of
+// dependent loads and LDS steps each, 3 to 9 MB moved.  The splats keep their
+// original order, so there is no depth order to wait for (run sort and ranks,
+// 30 us of serial chains at 64K splats); instead each pair carries its splat's depth
+// key, and the workgroup that groups a bucket's pairs by tile also sorts each
+// tile's list by (depth, index), which is the stable depth order.  The pairs
+// go straight to their bucket: the count's per-block digit counts, which the
+// one-call binning reduces to one histogram, give each emit block its place
+// in every bucket, so there is no pass over the pairs and no look-back either.
+//
+// tile_count_kernel  records in original order, each block's pairs per bucket
+// tile_emit_kernel   every block sums the counts of the blocks before it (256
+//   buckets x at most 256 blocks), walks again and writes {depth key, tile in
+//   the bucket << 24 | index} at its places, in any order inside them
+// tile_sort_kernel   a workgroup per bucket: tile counts, grouping and ranks
+//   in LDS, the ids and the tile ranges
+//
+// Measured against the one-call binning (us for count, emit and sort; the five
+// launches): 64K splats at 1080p 11.9 + 13.1 + 6.5 against 60 in all, at 4096 x
+// 4096 14.3 + 17.8 + 7.3 against 68; 128K splats at 1080p 15.0 + 15.2 + 11.8
+// against 83; 5000 splats at 1080p 8.1 + 8.4 + 4.2 against 43; 16K splats at
+// 512 x 512 8.7 + 8.7 + 6.1 against 45; two images of 32K splats at 600 x 800
+// 10.0 + 12.4 + 8.7 against 55.
+constexpr int kTileWaves = 16;
+constexpr int kTileThreads = 64 * kTileWaves;
+// A bucket that the sort's LDS does not hold (64 KB of pairs, 8 in registers
+// per thread), or a tile list so long that ranking its entries against each
+// other (its length per entry: a full bucket of lists of 512 takes 8 x 512
+// steps) costs more than the depth order, sets kTileSkewed in the long-range
+// flag and leaves its tiles empty; the caller bins such a scene by the other
+// path.
+constexpr int kTileRounds = 8;
+constexpr int kTileBucket = kTileRounds * kTileThreads;
+constexpr int kTileList = 512;
+
+// The wavefront's splats staged for the walk, in original order.
+template <int kS>
+__device__ __forceinline__ int tile_walk_setup(
+    const RasterParams& P, const float* __restrict__ means2d,
+    const float* __restrict__ conics, const float* __restrict__ opacities,
+    int orig, bool valid, WalkSlots<kS>& W, int& n_inner) {
+  const int o = valid ? orig : P.num_splats - 1;
+  SplatGeom s;
+  s.mx = means2d[2 * o + 0];
+  s.my = means2d[2 * o + 1];
+  s.a = conics[3 * o + 0];
+  s.b = conics[3 * o + 1];
+  s.c = conics[3 * o + 2];
+  s.o = opacities[o];
+  return walk_setup(P, valid, s, o / P.gpb, o, W, n_inner);
+}
+
+template <int kS>
+__global__ __launch_bounds__(kTileThreads) void tile_count_kernel(
+    RasterParams P, const float* __restrict__ means2d,
+    const float* __restrict__ conics, const float* __restrict__ colors,
+    const float* __restrict__ opacities, float4* __restrict__ packed,
+    uint32_t* __restrict__ parts, int shift, int32_t* __restrict__ ctl,
+    ZeroSpan z0, ZeroSpan z1) {
+  __shared__ WalkSlots<kS> walk[kTileWaves];
+  __shared__ uint32_t hist[2 * 257];
+  const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
+  const int64_t stride = (int64_t)gridDim.x * kTileThreads;
+  const int64_t first = (int64_t)blockIdx.x * kTileThreads + t;
+  for (int64_t i = first; i < z0.n; i += stride) z0.p[i] = 0u;
+  for (int64_t i = first; i < z1.n; i += stride) z1.p[i] = 0u;
+  if (first < 4) ctl[first] = 0;
+  for (int i = t; i < 2 * 257; i += kTileThreads) hist[i] = 0u;
+  __syncthreads();
+  const int orig = ((int)blockIdx.x * kTileWaves + wave) * kS + lane;
+  const bool valid = lane < kS && orig < P.num_splats;
+  WalkSlots<kS>& W = walk[wave];
+  int n_inner;
+  const int total = tile_walk_setup(P, means2d, conics, opacities, orig, valid,
+                                    W, n_inner);
+  walk_candidates(P, W, total, nullptr,
+                  [&](uint64_t, bool hit, int, int tile, int) {
+                    if (hit)
+                      atomicAdd(&hist[(lane & 1) * 257 +
+                                      (((uint32_t)tile >> shift) & 255u)],
+                                1u);
+                  });
+  if (lane < kS && n_inner > 0) {
+    const int4 in = W.inner[lane];
+    const int4 bx = W.box[lane];
+    for (int r = 0; r < in.w; ++r) {
+      uint32_t t0 = (uint32_t)(bx.w + (bx.y + in.y + r) * P.tiles_x + bx.x + in.x);
+      const uint32_t t1 = t0 + (uint32_t)in.z;
+      while (t0 < t1) {
+        const uint32_t seg = min(t1, ((t0 >> shift) + 1u) << shift);
+        atomicAdd(&hist[(lane & 1) * 257 + ((t0 >> shift) & 255u)], seg - t0);
+        t0 = seg;
+      }
+    }
+  }
+  if (valid)
+    store_record(packed, orig,
+                 record_of(P, means2d, conics, colors, opacities, orig,
+                           (uint32_t)orig));
+  __syncthreads();
+  if (t < 256) parts[(int64_t)blockIdx.x * 256 + t] = hist[t] + hist[257 + t];
+}
+
+template <int kS>
+__global__ __launch_bounds__(kTileThreads) void tile_emit_kernel(
+    RasterParams P, const float* __restrict__ means2d,
+    const float* __restrict__ conics, const float* __restrict__ opacities,
+    const float* __restrict__ depths, const uint32_t* __restrict__ parts,
+    int shift, int64_t capacity, uint2* __restrict__ pairs,
+    uint32_t* __restrict__ bucket_start, int32_t* __restrict__ ctl) {
+  __shared__ WalkSlots<kS> walk[kTileWaves];
+  __shared__ uint32_t dkey[kTileWaves][kS];
+  __shared__ uint32_t cursor[256];
+  __shared__ uint32_t red[2][kTileThreads];
+  __shared__ unsigned long long wsum[4];
+  const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
+  const int vb = (int)blockIdx.x, nblk = (int)gridDim.x;
+  const int orig0 = (vb * kTileWaves + wave) * kS;
+  const int orig = orig0 + lane;
+  const bool valid = lane < kS && orig < P.num_splats;
+  {  // bucket t % 256 in a quarter of the blocks: all, and those before this
+    const int d = t & 255, g = t >> 8;
+    uint32_t all = 0u, before = 0u;
+    for (int r = g; r < nblk; r += 64) {  // sixteen loads in flight
+      uint32_t v[16];
+#pragma unroll
+      for (int u = 0; u < 16; ++u)
+        v[u] = parts[(int64_t)min(r + 4 * u, nblk - 1) * 256 + d];
+#pragma unroll
+      for (int u = 0; u < 16; ++u) {
+        const uint32_t x = r + 4 * u < nblk ? v[u] : 0u;
+        all += x;
+        before += r + 4 * u < vb ? x : 0u;
+      }
+    }
+    red[0][t] = all;
+    red[1][t] = before;
+  }
+  WalkSlots<kS>& W = walk[wave];
+  int n_inner;
+  const int total = tile_walk_setup(P, means2d, conics, opacities, orig, valid,
+                                    W, n_inner);
+  if (lane < kS) dkey[wave][lane] = valid ? depth_key(depths[orig]) : 0u;
+  __syncthreads();
+  unsigned long long inc = 0;
+  uint32_t all = 0u, before = 0u;
+  if (t < 256) {
+#pragma unroll
+    for (int g = 0; g < 4; ++g) {
+      all += red[0][g * 256 + t];
+      before += red[1][g * 256 + t];
+    }
+    inc = all;
+  }
+#pragma unroll
+  for (int off = 1; off < 64; off <<= 1) {
+    const unsigned long long y = __shfl_up(inc, off, 64);
+    if (lane >= off) inc += y;
+  }
+  if (t < 256 && lane == 63) wsum[wave] = inc;
+  __syncthreads();
+  if (t < 256) {
+    for (int w = 0; w < wave; ++w) inc += wsum[w];
+    // (positions at or above the capacity, below 2^31, are not written)
+    const unsigned long long start = inc - all;
+    const unsigned long long top = 0x7fffffffull;
+    cursor[t] = (uint32_t)min(start + before, top);
+    if (vb == 0) {
+      bucket_start[t] = (uint32_t)min(start, top);
+      if (t == 255) {
+        bucket_start[256] = (uint32_t)min(inc, top);
+        ctl[0] = inc > top ? -1 : (int32_t)inc;
+      }
+    }
+  }
+  __syncthreads();
+  const uint32_t low = (1u << shift) - 1u;
+  auto put = [&](uint32_t tile, int sl) {
+    const uint32_t pos = atomicAdd(&cursor[(tile >> shift) & 255u], 1u);
+    if (pos < (uint32_t)capacity)
+      pairs[pos] = make_uint2(dkey[wave][sl],
+                              (tile & low) << 24 | (uint32_t)(orig0 + sl));
+  };
+  walk_candidates(P, W, total, nullptr,
+                  [&](uint64_t, bool hit, int sl, int tile, int) {
+                    if (hit) put((uint32_t)tile, sl);
+                  });
+  uint64_t with_inner = __ballot(lane < kS && n_inner > 0);
+  for (; with_inner != 0ull; with_inner &= with_inner - 1ull) {
+    const int sl = (int)__builtin_ctzll(with_inner);
+    const int4 in = W.inner[sl];
+    const int4 bx = W.box[sl];
+    for (int i = lane; i < in.z * in.w; i += 64) {
+      const int dy = div_small(i, in.z);
+      put((uint32_t)(bx.w + (bx.y + in.y + dy) * P.tiles_x +
+                     (bx.x + in.x + (i - dy * in.z))),
+          sl);
+    }
+  }
+}
+
+__global__ __launch_bounds__(kTileThreads) void tile_sort_kernel(
+    const uint2* __restrict__ pairs, const uint32_t* __restrict__ bucket_start,
+    int64_t capacity, int num_tiles, int low_bits,
+    uint32_t* __restrict__ binned_ids, int32_t* __restrict__ tile_offsets,
+    int32_t* __restrict__ ctl) {
+  __shared__ uint64_t list[kTileBucket];  // depth key << 32 | tile << 24 | index
+  __shared__ uint32_t cnt[256], start[256];
+  __shared__ uint32_t wsum[4];
+  __shared__ int skewed;
+  const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
+  const int b = (int)blockIdx.x;
+  const int tile0 = b << low_bits, ndig = 1 << low_bits;
+  const uint32_t cap = (uint32_t)capacity;
+  const uint32_t base = min(bucket_start[b], cap);
+  const uint32_t end = min(bucket_start[b + 1], cap);
+  const uint32_t size = end - base;
+  if (t < 256) cnt[t] = 0u;
+  if (t == 0) skewed = size > (uint32_t)kTileBucket;
+  if (b == (int)gridDim.x - 1 && t == 0) tile_offsets[num_tiles] = (int32_t)end;
+  __syncthreads();
+  const bool fits = size <= (uint32_t)kTileBucket;
+  uint2 v[kTileRounds];
+  uint32_t slot[kTileRounds];
+  if (fits) {
+#pragma unroll
+    for (int r = 0; r < kTileRounds; ++r) {
+      const uint32_t i = (uint32_t)(t + kTileThreads * r);
+      if (i < size) v[r] = pairs[base + i];
+    }
+#pragma unroll
+    for (int r = 0; r < kTileRounds; ++r) {
+      const uint32_t i = (uint32_t)(t + kTileThreads * r);
+      if (i < size) slot[r] = atomicAdd(&cnt[v[r].y >> 24], 1u);
+    }
+  }
+  __syncthreads();
+  const uint32_t n = t < 256 ? cnt[t] : 0u;
+  uint32_t inc = n;
+#pragma unroll
+  for (int off = 1; off < 64; off <<= 1) {
+    const uint32_t y = __shfl_up(inc, off, 64);
+    if (lane >= off) inc += y;
+  }
+  if (t < 256) {
+    if (lane == 63) wsum[wave] = inc;
+    if (n > (uint32_t)kTileList) skewed = 1;
+  }
+  __syncthreads();
+  const bool skip = skewed != 0;  // uniform
+  if (t < 256) {
+    for (int w = 0; w < wave; ++w) inc += wsum[w];
+    start[t] = inc - n;
+    // (a skewed bucket's tiles are empty, at its end)
+    if (t < ndig && tile0 + t < num_tiles)
+      tile_offsets[tile0 + t] = (int32_t)(skip ? end : base + inc - n);
+    const bool is_long = n > (uint32_t)kHandoffPairs;
+    if (__ballot(is_long) != 0ull && lane == 0) atomicOr(ctl + 2, 1);
+  }
+  if (skip) {
+    if (t == 0) atomicOr(ctl + 2, kTileSkewed);
+    return;
+  }
+  __syncthreads();
+#pragma unroll
+  for (int r = 0; r < kTileRounds; ++r) {
+    const uint32_t i = (uint32_t)(t + kTileThreads * r);
+    if (i < size)
+      list[start[v[r].y >> 24] + slot[r]] = (uint64_t)v[r].x << 32 | v[r].y;
+  }
+  __syncthreads();
+  // Each entry's rank in its tile (the entries' tiles agree, so the low words
+  // compare by index); neighbouring threads mostly share a tile, and read
+  // the same words.
+  for (uint32_t i = t; i < size; i += kTileThreads) {
+    const uint64_t own = list[i];
+    const uint32_t d = (uint32_t)own >> 24;
+    const uint32_t s0 = start[d], s1 = s0 + cnt[d];
+    uint32_t rank = 0u, j = s0;
+    for (; j + 4 <= s1; j += 4) {
+      rank += (uint32_t)(list[j] < own);
+      rank += (uint32_t)(list[j + 1] < own);
+      rank += (uint32_t)(list[j + 2] < own);
+      rank += (uint32_t)(list[j + 3] < own);
+    }
+    for (; j < s1; ++j) rank += (uint32_t)(list[j] < own);
+    binned_ids[base + s0 + rank] = (uint32_t)own & 0xffffffu;
+  }
+}
+
 __global__ __launch_bounds__(kThreads) void counts_kernel(
     const int32_t* __restrict__ tile_offsets, int num_tiles,
     int32_t* __restrict__ tile_counts) {
@@ -1634,6 +1925,51 @@ int launch_bucket_sort(const BucketSortArgs& A, hipStream_t stream) {
   launch_traced("bucket_sort_kernel", bucket_sort_kernel,
                 dim3((unsigned)buckets), dim3(kBucketThreads), 0, stream, A);
   return check_launch("bucket_sort_kernel");
+}
+
+// Splats per wavefront: 16 up to 64K splats (a block per CU: count + emit at
+// 64K splats 25.0 us at 1080p, 32.1 at 4096 x 4096, with 32 25.5 and 35.7), 32
+// above (each emit block reads every block's counts).
+static int tile_walk(const RasterParams& P) {
+  return P.num_splats <= (1 << 16) ? 16 : 32;
+}
+
+int tile_blocks(const RasterParams& P) {
+  const int splats = kTileWaves * tile_walk(P);
+  return (P.num_splats + splats - 1) / splats;
+}
+
+int launch_tile_sorted(const RasterParams& P, const float* means2d,
+                       const float* conics, const float* colors,
+                       const float* opacities, const float* depths,
+                       int low_bits, int64_t capacity, float* packed,
+                       uint32_t* parts, uint32_t* bucket_start, int32_t* ctl,
+                       void* pairs, int32_t* binned_ids, int32_t* tile_offsets,
+                       const ZeroSpan zero[2], hipStream_t stream) {
+  const unsigned blocks = (unsigned)tile_blocks(P);
+  const bool narrow = tile_walk(P) == 16;
+  launch_traced("tile_count_kernel",
+                narrow ? tile_count_kernel<16> : tile_count_kernel<32>,
+                dim3(blocks), dim3(kTileThreads), 0, stream, P, means2d,
+                conics, colors, opacities, reinterpret_cast<float4*>(packed),
+                parts, low_bits, ctl, zero[0], zero[1]);
+  int rc = check_launch("tile_count_kernel");
+  if (rc) return rc;
+  launch_traced("tile_emit_kernel",
+                narrow ? tile_emit_kernel<16> : tile_emit_kernel<32>,
+                dim3(blocks), dim3(kTileThreads), 0, stream, P, means2d,
+                conics, opacities, depths, parts, low_bits, capacity,
+                reinterpret_cast<uint2*>(pairs), bucket_start, ctl);
+  rc = check_launch("tile_emit_kernel");
+  if (rc) return rc;
+  launch_traced("tile_sort_kernel", tile_sort_kernel,
+                dim3((unsigned)(((int64_t)P.num_tiles + (1 << low_bits) - 1) >>
+                                low_bits)),
+                dim3(kTileThreads), 0, stream,
+                reinterpret_cast<const uint2*>(pairs), bucket_start, capacity,
+                P.num_tiles, low_bits, reinterpret_cast<uint32_t*>(binned_ids),
+                tile_offsets, ctl);
+  return check_launch("tile_sort_kernel");
 }
 
 int launch_host_report(const HostReport& R, hipStream_t stream) {

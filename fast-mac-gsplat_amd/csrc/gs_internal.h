@@ -347,6 +347,23 @@ struct BucketSortArgs {
   ZeroSpan zero[2];
 };
 int launch_bucket_sort(const BucketSortArgs& A, hipStream_t stream);
+// The tile-sorted binning of at most kTileMaxSplats splats, low_bits as the
+// bucket form's: records in original order, binned_ids original indices in
+// depth order per tile, tile_offsets.  Scratch: parts (tile_blocks(P) * 256
+// words), bucket_start (257), pairs (capacity * 8 bytes).  ctl[0] = N (-1
+// above int32), ctl[1] = 0, ctl[2]: bit 0 a list longer than kHandoffPairs,
+// kTileSkewed a bucket or list too long (its tiles are then empty, and the
+// binning is to be done otherwise).  The first launch zeroes the two spans.
+constexpr int kTileMaxSplats = 1 << 17;
+constexpr int kTileSkewed = GSPLAT_TILE_SKEWED;
+int tile_blocks(const RasterParams& P);
+int launch_tile_sorted(const RasterParams& P, const float* means2d,
+                       const float* conics, const float* colors,
+                       const float* opacities, const float* depths,
+                       int low_bits, int64_t capacity, float* packed,
+                       uint32_t* parts, uint32_t* bucket_start, int32_t* ctl,
+                       void* pairs, int32_t* binned_ids, int32_t* tile_offsets,
+                       const ZeroSpan zero[2], hipStream_t stream);
 // rank_pack: the second launch of the small-image depth order (runs in
 // depth_buffers, as launch_count_depth_runs leaves them) with the records
 // packed at the ranks: perm, packed, gid_count[gid] = splat_count[orig], and

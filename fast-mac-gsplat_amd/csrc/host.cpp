@@ -50,6 +50,8 @@ using torch::autograd::variable_list;
   F(render_backward)                    \
   F(direct_workspace_bytes)             \
   F(direct_render)                      \
+  F(tile_workspace_bytes)               \
+  F(tile_render)                        \
   F(project_forward)                    \
   F(project_backward)                   \
   F(project_backward_workspace_bytes)
@@ -197,7 +199,7 @@ struct Saved : torch::CustomClassHolder {
   bool depth_grad = true;
 };
 
-enum class Mode { kDirect, kBinned };
+enum class Mode { kDirect, kTiled, kBinned };
 
 struct Call {
   gsplat_raster_meta meta;
@@ -210,6 +212,7 @@ struct Call {
 struct Result {
   Tensor img, final_T, last, kept;
   int32_t n = 0;  // N of a binned call
+  bool skewed = false;  // a tiled call that is to be done by kBinned
 };
 
 Tensor bytes(int64_t n, const Tensor& like) {
@@ -262,7 +265,14 @@ Result render(const Call& c, const std::array<Tensor, 5>& in, bool train) {
     return r;
   }
   int32_t* row = rows_of(like.device().index()).next();
-  check(api.bin_render_forward(
+  if (c.mode == Mode::kTiled)
+    check(api.tile_render(&c.meta, f32(t[0]), f32(t[1]), f32(t[2]), f32(t[3]),
+                          f32(t[4]), c.n_pairs, packed, offsets, pairs, row,
+                          r.img.data_ptr<float>(), T, last, stop, u + uo[2],
+                          (size_t)(uo[3] - uo[2]), rws, rws_bytes, s),
+          "gsplat_hip_tile_render");
+  else
+    check(api.bin_render_forward(
             &c.meta, f32(t[0]), f32(t[1]), f32(t[2]), f32(t[3]), f32(t[4]),
             c.n_pairs, reinterpret_cast<int32_t*>(u + uo[0]), packed,
             reinterpret_cast<int32_t*>(u + uo[1]), pairs, offsets, row,
@@ -283,7 +293,8 @@ Result render(const Call& c, const std::array<Tensor, 5>& in, bool train) {
   TORCH_CHECK(status == 0, "binning failed with device status ", status);
   r.n = row[0];
   TORCH_CHECK(r.n >= 0, "pair count overflowed int32");
-  if (r.n <= c.n_pairs && row[2] != 0)
+  r.skewed = c.mode == Mode::kTiled && (row[2] & GSPLAT_TILE_SKEWED) != 0;
+  if (r.n <= c.n_pairs && !r.skewed && row[2] != 0)
     check(api.render_forward_long(&c.meta, packed, offsets, pairs,
                                   r.img.data_ptr<float>(), T, last, stop,
                                   c.n_pairs, rws, rws_bytes, s),
@@ -293,12 +304,17 @@ Result render(const Call& c, const std::array<Tensor, 5>& in, bool train) {
 
 class Plan;
 Call grown(Plan& plan, const Call& c, const Tensor& like, int32_t n, bool train);
+Call unskewed(Plan& plan, const Call& c, const Tensor&, bool train);
 
 // The forward with the pairs it found room for: binned again, once, when N was
 // above the capacity of the shape's earlier calls.
 Result render_all(Plan& plan, Call& c, const std::array<Tensor, 5>& in, bool train) {
   Result r = render(c, in, train);
   if (c.mode == Mode::kDirect) return r;
+  if (r.skewed) {  // (remembered: the shape's next calls are binned at once)
+    c = unskewed(plan, c, in[0], train);
+    r = render(c, in, train);
+  }
   const int32_t n = r.n;
   Call next = grown(plan, c, in[0], n, train);
   if (n <= c.n_pairs) return r;
@@ -437,9 +453,24 @@ class Plan {
     const int64_t cap = note_pairs_(key(c, like), n).cast<int64_t>();
     Call next = c;
     if (n > c.n_pairs) {
+      next.mode = Mode::kBinned;
       next.n_pairs = cap;
       next.sizes = sizes_of(c.meta, Mode::kBinned, cap, train);
     }
+    return next;
+  }
+
+  // The call of a skewed scene by the one-call binning; the shape's later
+  // calls go there at once.
+  Call binned(const Call& c, bool train) {
+    {
+      std::lock_guard<std::mutex> lock(mu_);
+      if (skewed_.size() >= 64) skewed_.erase(skewed_.begin());
+      skewed_.emplace_back(c.meta.batch, c.meta.gaussians_per_batch);
+    }
+    Call next = c;
+    next.mode = Mode::kBinned;
+    next.sizes = sizes_of(c.meta, Mode::kBinned, c.n_pairs, train);
     return next;
   }
 
@@ -479,6 +510,17 @@ class Plan {
     if (c.n_pairs <= 0 || c.n_pairs > 0x7fffffff ||
         4 * c.n_pairs >= 5 * (sliced_pairs_ + sliced_pairs_per_tile_ * tiles_ * B))
       return false;
+    bool skewed = false;
+    {
+      std::lock_guard<std::mutex> lock(mu_);
+      for (const auto& e : skewed_)
+        skewed |= e.first == c.meta.batch && e.second == c.meta.gaussians_per_batch;
+    }
+    if (!skewed) {
+      c.mode = Mode::kTiled;
+      c.sizes = sizes_of(c.meta, Mode::kTiled, c.n_pairs, train);
+      if (c.sizes.keep[5] > 0) return true;
+    }
     c.mode = Mode::kBinned;
     c.sizes = sizes_of(c.meta, Mode::kBinned, c.n_pairs, train);
     return true;
@@ -492,13 +534,14 @@ class Plan {
       if (e.first == k) return e.second;
     Sizes s{};
     const int64_t BG = (int64_t)m.batch * m.gaussians_per_batch, T = tiles_ * m.batch;
-    const int64_t work = mode == Mode::kDirect ? (int64_t)api.direct_workspace_bytes(&m)
-                                               : (int64_t)api.bin_workspace_bytes(&m, n);
+    const int64_t work = mode == Mode::kDirect  ? (int64_t)api.direct_workspace_bytes(&m)
+                         : mode == Mode::kTiled ? (int64_t)api.tile_workspace_bytes(&m, n)
+                                                : (int64_t)api.bin_workspace_bytes(&m, n);
     if (work > 0) {
       const int64_t part[5] = {BG * GSPLAT_RECORD_FLOATS * 4, n * 4, (T + 1) * 4, train ? T * 4 : 0,
                                (int64_t)api.render_workspace_bytes(&m, train ? n : 0)};
       for (int i = 0; i < 5; ++i) s.keep[i + 1] = s.keep[i] + align256(part[i]);
-      const bool direct = mode == Mode::kDirect;
+      const bool direct = mode != Mode::kBinned;  // (no depth order or offsets)
       s.use[1] = direct ? 0 : align256(BG * 4);
       s.use[2] = s.use[1] + (direct ? 0 : align256((BG + 1) * 4));
       s.use[3] = s.use[2] + align256(work);
@@ -518,10 +561,15 @@ class Plan {
   py::function note_pairs_;
   std::mutex mu_;
   std::vector<std::pair<std::array<int64_t, 5>, Sizes>> sizes_;
+  std::vector<std::pair<int32_t, int32_t>> skewed_;  // (B, G) of skewed scenes
 };
 
 Call grown(Plan& plan, const Call& c, const Tensor& like, int32_t n, bool train) {
   return plan.after(c, like, n, train);
+}
+
+Call unskewed(Plan& plan, const Call& c, const Tensor&, bool train) {
+  return plan.binned(c, train);
 }
 
 // ---- projection

@@ -604,6 +604,39 @@ int gsplat_hip_direct_render(const gsplat_raster_meta* meta,
                              void* render_workspace,
                              size_t render_workspace_bytes, void* stream);
 
+/* ---- Tile-sorted rendering ------------------------------------------------
+ * gsplat_hip_bin_render_forward in fewer launches for scenes of up to 128K
+ * splats in all, of at least 16K splats or 2048 tiles: no depth order of the splats, each tile's list is sorted by
+ * depth instead.  Same image, stops and gradients.  It has no counterpart in
+ * the reference. */
+
+/* Set in host_words[2] where a scene has tiles or groups of tiles with too
+ * many pairs for it: the image is then incomplete, and the scene is to be
+ * rendered by gsplat_hip_bin_render_forward. */
+#define GSPLAT_TILE_SKEWED 2
+
+/* 0 where the path does not apply to the shape and capacity. */
+size_t gsplat_hip_tile_workspace_bytes(const gsplat_raster_meta* meta,
+                                       int64_t capacity);
+
+/* packed float [B*G*16] in original order; binned_ids int32 [capacity]:
+ * original indices per tile in depth order; tile_offsets int32 [T+1].
+ * host_words as gsplat_hip_bin's, written as the forward starts, word 2 with
+ * GSPLAT_TILE_SKEWED beside the long-range flag (bit 0).  The outputs and
+ * the render workspace as gsplat_hip_bin_render_forward's with n_pairs =
+ * capacity; the continuation of long tiles is the caller's, as there. */
+int gsplat_hip_tile_render(const gsplat_raster_meta* meta,
+                           const float* means2d, const float* conics,
+                           const float* colors, const float* opacities,
+                           const float* depths, int64_t capacity,
+                           float* packed, int32_t* tile_offsets,
+                           int32_t* binned_ids, int32_t* host_words,
+                           float* out_rgb, float* out_final_T,
+                           int32_t* out_last, int32_t* out_tile_stop,
+                           void* workspace, size_t workspace_bytes,
+                           void* render_workspace,
+                           size_t render_workspace_bytes, void* stream);
+
 #ifdef __cplusplus
 }
 #endif

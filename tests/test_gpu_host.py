@@ -8,6 +8,7 @@ import torch
 
 from torch_gsplat_bridge_fast import (RasterConfig, project_pinhole_gaussians, rasterize_pinhole_gaussians,
                                       rasterize_projected_gaussians)
+from torch_gsplat_bridge_fast import _lib, _ops
 from torch_gsplat_bridge_fast import project as project_mod
 from torch_gsplat_bridge_fast import rasterize as rasterize_mod
 from torch_gsplat_bridge_fast.scenes import make_scene_2d, make_scene_3d
@@ -15,7 +16,8 @@ from torch_gsplat_bridge_fast.scenes import make_scene_2d, make_scene_3d
 pytestmark = pytest.mark.gpu
 
 KEYS = ("means2d", "conics", "colors", "opacities", "depths")
-SIZES = [(1, 300, 96, 131), (2, 5000, 130, 170)]   # the direct path, the one-call binning
+# the direct path, the one-call binning, the tile-sorted binning
+SIZES = [(1, 300, 96, 131), (2, 5000, 130, 170), (2, 9000, 260, 530)]
 
 
 def _scene(B, G, H, W, batched=True, seed=1):
@@ -111,6 +113,64 @@ def test_strides_hooks_and_streams(B, G, H, W):
         got = step(x, x)
     torch.cuda.current_stream().wait_stream(side)
     close(got)
+
+
+@pytest.mark.parametrize("kind,B,G,H,W", [
+    ("uniform", 1, 16384, 512, 272),     # the fewest splats, 2^9 + 32 tiles
+    ("ties", 1, 4999, 512, 1024),        # the fewest tiles
+    ("uniform", 1, 131072, 1080, 1920),  # the most
+    ("ties", 3, 21845, 300, 400),        # depth ties, three images
+    ("special", 2, 20001, 333, 517),     # NaN, infinite and signed zero depths
+    ("uniform", 1, 70001, 4096, 4096),   # 2^16 tiles, 256 a bucket
+    ("long", 1, 30000, 400, 400),        # lists above the hand-off length, below the limit
+    ("hot tile", 1, 20000, 600, 600),    # a tile above the limit: binned by the other path
+    ("hot bucket", 1, 60000, 600, 600),  # a bucket above the limit
+    ("culled", 1, 20000, 600, 600),
+])
+def test_tile_sorted_matches_python(kind, B, G, H, W):
+    g = torch.Generator().manual_seed(5)
+    sc = make_scene_2d(1, seed=3, G=G, B=B, H=H, W=W)
+    if kind == "ties":
+        sc["depths"] = torch.randint(0, 9, (B, G), generator=g).float()
+    if kind == "special":
+        for k, v in enumerate((float("nan"), float("inf"), -float("inf"), -0.0, 0.0)):
+            sc["depths"][:, k::7] = v
+    if kind == "long":
+        sc["conics"] = sc["conics"] * 0.3
+        sc["opacities"] = 0.05 + 0.0 * sc["opacities"]
+    if kind == "hot tile":
+        sc["means2d"][:, :900] = 300.0 + 2.0 * torch.rand(B, 900, 2, generator=g)
+        sc["opacities"] = 0.3 * sc["opacities"]
+    if kind == "hot bucket":
+        sc["means2d"][:, :40000] = torch.rand(B, 40000, 2, generator=g) * torch.tensor([600.0, 20.0])
+        sc["opacities"] = 0.3 * sc["opacities"]
+    if kind == "culled":
+        sc["opacities"] = 0.0 * sc["opacities"]
+    ts = [sc[k].cuda() for k in KEYS]
+    cfg = RasterConfig(height=H, width=W, background=(0.1, 0.2, 0.3))
+    plan = _plan(cfg, ts)
+    L = _lib.lib()
+    meta = rasterize_mod._meta(cfg, B, G)
+    key = (0, B, G, H, W)
+    cap = _ops._capacity.get(key, 0)
+    if kind == "culled":
+        cap = _ops._capacity[key] = 10000
+    assert L.gsplat_hip_tile_workspace_bytes(meta, cap) > 0
+    w = torch.rand(B, H, W, 3, generator=g).cuda()
+    b = _leaves(ts, (1, 1, 1, 1, 0))
+    ref = _python(b, cfg)
+    ref.backward(w)
+    n = _ops.bin_gaussians(meta, *[t.reshape(B * G, -1).squeeze(-1) for t in ts]).n_pairs
+    for cap in (cap, cap, max(1, n), max(1, n // 2)):   # the last: too small, binned again
+        _ops._capacity[key] = cap
+        a = _leaves(ts, (1, 1, 1, 1, 0))
+        img = plan.run(*a, True)
+        assert torch.equal(img, ref)
+        img.backward(w)
+        for x, y in zip(a[:4], b[:4]):
+            torch.testing.assert_close(x.grad, y.grad, rtol=1e-4, atol=1e-5 * float(y.grad.abs().max()) + 1e-7)
+        with torch.no_grad():
+            assert torch.equal(plan.run(*ts, True), ref)
 
 
 def test_threads_share_a_plan():
