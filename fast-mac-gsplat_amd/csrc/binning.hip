@@ -4,16 +4,22 @@
 // This translation unit is compiled with -ffp-contract=off: the predicate
 // results must match the CPU oracle bit for bit.
 //
-// Tile walk (count_kernel and emit_kernel).  The candidate tiles of a splat
-// are the tiles of its snug pixel bbox, row-major; a candidate is a hit when
-// the tile's pixel-centre rectangle meets the splat's alpha >= threshold
-// ellipse (reference count_tiles / emit_binned_ids,
+// Row walk (the count and emit kernels).  The candidate tiles of a splat are
+// the tiles of its snug pixel bbox; a candidate is a hit when the tile's
+// pixel-centre rectangle meets the splat's alpha >= threshold ellipse
+// (reference count_tiles / emit_binned_ids,
 // variants/v8/csrc/metal/gsplat_v8_kernels.metal:244-327).  A wavefront takes
-// kWalkSplats (32) splats, prefix-sums their candidate counts in registers
-// and then tests 64 candidates per step whatever splats they belong to (each
-// lane finds its candidate's splat from LDS marks of the splats that start
-// inside the step, spread by a DPP prefix maximum; see walk_candidates), so a
-// splat with thousands of candidate tiles does not serialise one lane.
+// kWalkSplats (32) splats, prefix-sums the rows of their tile boxes and takes
+// 64 rows per step whatever splats they belong to; each lane finds its row's
+// span of hits from the ellipse (span_constants) and tests exactly only the
+// tiles that the span's bounds leave open.  The walk is bound by the vector
+// instructions it issues, and testing every candidate tile took them: a 3D
+// scene's splats have 45 candidates in 7 rows.  The counts add up spans; the
+// emits lay a step's spans end to end and write 64 pairs at a time.  Measured
+// (us, every tile tested -> spans): two images of 100K 3D splats at 29 pairs
+// each, count 61 -> 19, emit 69 -> 45; 200K at 40 pairs, count 78 -> 18, emit
+// 82 -> 54 (from the count's recorded hits before); 64K 2D splats of 4.5
+// pairs, count 11.9 -> 11.2, emit 13.1 -> 13.8.
 //
 // Staged path (one launch per step, also the separate C-ABI steps):
 // count_kernel  original order: per-splat hit counts and per-workgroup sums
@@ -47,12 +53,10 @@
 // host_report_kernel  the binning's report to host memory where the
 //   forward compositor does not write it.
 //
-// Larger images in one call: count_kernel also keeps each wavefront's first
-// kHitSlab step ballots and the splats' records in original order;
-// pack_kernel gives each original index its pair offset and gid; and
-// emit_kernel<false, true> walks the splats in the count's original order,
-// taking the hits of the recorded steps from the ballots instead of testing
-// them again.
+// Larger images in one call: count_kernel also keeps the splats' records in
+// original order; pack_kernel gives each original index its pair offset and
+// gid; and emit_kernel<false, true> walks the splats in the count's original
+// order.
 #include <algorithm>
 
 #include "gs_internal.h"
@@ -72,8 +76,8 @@ struct SplatGeom {
 
 constexpr int kWaves = kThreads / 64;
 
-// Splats per wavefront in the tile walk.  A wavefront's 64 lanes test the
-// candidates of kS splats together; fewer splats per wavefront
+// Splats per wavefront in the row walk.  A wavefront's 64 lanes take the
+// rows of kS splats together; fewer splats per wavefront
 // than lanes gives each launch more wavefronts (the walk is latency bound)
 // and a shorter slot search.  kS is kWalkSplats, or fewer in the small-image
 // path where few splats have many candidates each (walk_splats).
@@ -85,19 +89,18 @@ constexpr int kDirectHistBlocks = 1024;
 // Copies of the emit's digit histograms (see emit_kernel).
 constexpr int kHistCopies = 2;
 
-// One wavefront's kS splats, staged for the cooperative tile walk.
+// One wavefront's kS splats, staged for the cooperative row walk.
 template <int kS>
 struct WalkSlots {
-  float4 g0[kS];  // mx, my, a, b
-  float4 g1[kS];  // c, tau, kc, ka
-  int4 box[kS];   // tx0, ty0, tiles per bbox row, first tile of the image
-  int4 inner[kS]; // the certain hits (inner_tiles): x, y relative to
-                           // the box corner, width, height
-  int flags[kS];  // bit 0: use_c, bit 1: use_a
-  int cend[kS];   // inclusive prefix sum of candidate counts
-  int first[kS];  // exclusive prefix sum: the splat's first candidate
-  int ni_incl[kS];  // inclusive prefix sum of the certain hits
-  uint32_t own[64];        // per walk step: splats starting at each position
+  float4 g0[kS];   // mx, my, a, b
+  float4 g1[kS];   // c, tau, kc, ka
+  float4 span[kS]; // SpanConst
+  int4 box[kS];    // tx0, ty0, tx1, first tile of the image
+  float margin[kS];  // of the spans' ends (pixels); < 0: no certain spans
+  int flags[kS];   // bit 0: use_c, bit 1: use_a
+  int cend[kS];    // inclusive prefix sum of the boxes' rows
+  int first[kS];   // exclusive prefix sum: the splat's first row
+  uint32_t own[64];  // per walk step: items starting at each position
 };
 
 // Inclusive prefix maximum over the wavefront's 64 lanes (DPP: row shifts by
@@ -118,259 +121,320 @@ __device__ __forceinline__ uint32_t wave_prefix_max(uint32_t x) {
   return x;
 }
 
-// k / w for 0 <= k and 1 <= w, both below 2^24: the float quotient is
-// within a few units of the truth for such operands, and the remainder
-// corrects it exactly.
-__device__ __forceinline__ int div_small(int k, int w) {
-  int q = (int)((float)k * __builtin_amdgcn_rcpf((float)w));
-  int r = k - q * w;
-  while (r < 0) {
-    --q;
-    r += w;
-  }
-  while (r >= w) {
-    ++q;
-    r -= w;
-  }
-  return q;
+// Inclusive prefix sum over the wavefront's 64 lanes, the same way.
+__device__ __forceinline__ int wave_prefix_sum(int v) {
+  uint32_t x = (uint32_t)v;
+  x += dpp_or_zero<0x111>(x);
+  x += dpp_or_zero<0x112>(x);
+  x += dpp_or_zero<0x114>(x);
+  x += dpp_or_zero<0x118>(x);
+  x += dpp_or_zero<0x142, 0xA>(x);
+  x += dpp_or_zero<0x143, 0xC>(x);
+  return (int)x;
 }
 
-// A 64-bit value of lane l (l uniform).
-__device__ __forceinline__ uint64_t readlane64(uint64_t v, int l) {
-  const uint32_t lo = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)v, l);
-  const uint32_t hi =
-      (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(v >> 32), l);
-  return ((uint64_t)hi << 32) | lo;
-}
+// The rows of a splat's tile box hold its hits in one span each, and a row's
+// span is found from the ellipse itself instead of testing every tile: for
+// dy in the row's [dy0, dy1] the points with q(dx, dy) <= t reach to
+//   dx = ka dy +- sqrt(t/a - (det/a^2) dy^2),  ka = -b/a,
+// which is largest at the ellipse's rightmost point dy = kc hx (kc = -b/c,
+// hx = sqrt(t c/det)), or at the end of the row next to it.  Evaluated for
+// t = tau (1 + d) and t = tau (1 - d), d = 2^-10, this gives a span outside
+// which no tile passes ellipse_hits_rect and one inside which every tile
+// does; the tiles between the two (almost always none) are tested exactly.
+//
+// Why d suffices: the predicate's rounded quadratics (operands dx, dy of one
+// rounded subtraction each, relative error 2^-24) differ from the exact ones
+// by less than 16 2^-24 S, S = a dx^2 + c dy^2, and S <= q / (1 - r) with
+// r^2 = b^2 / (a c).  Spans are used where 1 - r^2 = det / (a c) >= 2^-7, so
+// 1 - r >= 2^-8 and the difference is below 2^-12 q.  A tile whose exact
+// minimum is at most tau (1 - d) is thus found by the predicate (which
+// evaluates each edge's own minimum, off by a rounded slope: second order),
+// and one whose exact minimum is above tau (1 + d) has every evaluated term
+// above tau.  det's own relative error, below 2^-22 2^7, moves t/a -
+// (det/a^2) dy^2 by 2^-15 of t/a, far below d, and the clamped dy by an
+// amount whose effect at the maximum is second order (below 2^-23 hx).  The
+// rounding of mx + dx is covered by a margin of 2^-20 (|mx| + hx) + 2^-20.
+// Rows of other splats (thin ones, c or a at most 1e-8, anything not finite)
+// have no certain span: every tile is tested.
+constexpr float kSpanUp = 1.0f + 0x1p-10f;
+constexpr float kSpanDown = 1.0f - 0x1p-10f;
 
-// Smallest number of certain hits (inner_tiles) taken out of the walk: the
-// emit writes a splat's certain hits with the wavefront's 64 lanes.
-constexpr int kMinCertainHits = 64;
-
-// Tiles of the box [tx0, tx1] x [ty0, ty1] that certainly pass
-// ellipse_hits_rect: those whose pixel-centre rectangle lies in the
-// rectangle |dx| <= u, |dy| <= v around the centre, with u = k s hx,
-// v = k s hy, s^2 = tau / (a hx^2 + c hy^2 + 2|b| hx hy) and k = 1 - 2^-10.
-// The quadratic q = a dx^2 + 2b dx dy + c dy^2 is convex, so on that
-// rectangle it is at most its largest corner value a u^2 + c v^2 + 2|b| u v
-// = k^2 s^2 (...) <= tau (1 - 2^-9) (s rounded within a few ulp).  A tile
-// there has its centre inside (a hit at once) or its nearest corner inside
-// the rectangle, where the predicate's rounded q, whose operands dx, dy are
-// each one rounded subtraction (relative error 2^-24) and whose three
-// terms sum to at most 2 (a dx^2 + c dy^2) <= 2 tau in magnitude (b^2 < ac),
-// exceeds the exact one by less than 16 2^-24 tau: below tau.  The tile
-// range is computed from u and v less an absolute margin far above the
-// rounding of mx +- u and my +- v.  Returns {x, y relative to (tx0, ty0),
-// width, height}, all 0 when there is no such tile or any quantity is not
-// finite, or when they are fewer than kMinCertainHits.  hx, hy only shape
-// the rectangle (the box's half extents).
-__device__ __forceinline__ int4 inner_tiles(float mx, float my, float a,
-                                            float b, float c, float tau,
-                                            int tx0, int ty0, int tx1,
-                                            int ty1) {
+// {tau (1 + d) / a, tau (1 - d) / a, det / a^2, kc hx at tau (1 + d)}; margin
+// < 0 where spans are not used.
+__device__ __forceinline__ float4 span_constants(const SplatGeom& s, float tau,
+                                                 const ConicSlopes& k,
+                                                 float& margin) {
 #pragma clang fp contract(off)
-  const float det = a * c - b * b;
-  if (!(a > 0.0f && c > 0.0f && det > 0.0f)) return make_int4(0, 0, 0, 0);
-  const float hx = __builtin_sqrtf(tau * c / det);
-  const float hy = __builtin_sqrtf(tau * a / det);
-  const float den = a * hx * hx + c * hy * hy + 2.0f * fabsf(b) * hx * hy;
-  const float sk = __builtin_sqrtf(tau / den) * (1.0f - 0x1p-10f);
-  const float margin =
-      (fabsf(mx) + fabsf(my) + hx + hy) * 0x1p-20f + 0x1p-20f;
-  const float u = sk * hx - margin, v = sk * hy - margin;
-  if (!(u > 0.0f && v > 0.0f && u < 0x1p30f && v < 0x1p30f &&
-        fabsf(mx) < 0x1p30f && fabsf(my) < 0x1p30f))
-    return make_int4(0, 0, 0, 0);
-  // tiles t with 16 t + 0.5 >= mx - u and 16 t + 15.5 <= mx + u
-  const float fx0 = fmaxf(ceilf((mx - u - 0.5f) * 0.0625f), (float)tx0);
-  const float fx1 = fminf(floorf((mx + u - 15.5f) * 0.0625f), (float)tx1);
-  const float fy0 = fmaxf(ceilf((my - v - 0.5f) * 0.0625f), (float)ty0);
-  const float fy1 = fminf(floorf((my + v - 15.5f) * 0.0625f), (float)ty1);
-  if (!(fx0 <= fx1 && fy0 <= fy1)) return make_int4(0, 0, 0, 0);
-  const int ix0 = (int)fx0, iy0 = (int)fy0;
-  const int iw = (int)fx1 - ix0 + 1, ih = (int)fy1 - iy0 + 1;
-  // (fewer tiles are cheaper to walk than to write in a loop of their own)
-  if (iw * ih < kMinCertainHits) return make_int4(0, 0, 0, 0);
-  return make_int4(ix0 - tx0, iy0 - ty0, iw, ih);
+  margin = -1.0f;
+  const float det = s.a * s.c - s.b * s.b;
+  if (!(k.use_a && k.use_c && s.a < 0x1p60f && s.c < 0x1p60f &&
+        det >= 0x1p-7f * (s.a * s.c) && fabsf(s.mx) < 0x1p30f &&
+        fabsf(s.my) < 0x1p30f))
+    return make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+  const float hx = __builtin_sqrtf(tau * kSpanUp * s.c / det);
+  if (!(hx < 0x1p30f)) return make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+  margin = (fabsf(s.mx) + hx) * 0x1p-20f + 0x1p-20f;
+  return make_float4(tau * kSpanUp / s.a, tau * kSpanDown / s.a,
+                     det / s.a / s.a, k.kc * hx);
 }
 
-// Stages this lane's splat (lanes below kS) and returns the
-// wavefront's candidate total: the tiles of each splat's box outside its
-// certain hits (inner_tiles), whose count goes to n_inner.  With P.live the
-// box is P.boxes[source], whole: it holds the live tiles, few of which are
-// certain hits.  Candidate
-// counts fit in int32: tiles per image are limited to 2^24 on the host, so
-// a wavefront has at most 2^28 candidates.
+// A row's tiles [m0, m1] that may hit and, of those, [c0, c1] that certainly
+// do (c0 > m1 when none).
+struct RowSpan {
+  int m0, m1, c0, c1;
+};
+
+template <int kS>
+__device__ __forceinline__ RowSpan row_span(const RasterParams& P,
+                                            const WalkSlots<kS>& W, int sl,
+                                            int ty) {
+#pragma clang fp contract(off)
+  const int4 bx = W.box[sl];
+  const float margin = W.margin[sl];
+  RowSpan r{bx.x, bx.z, 0x7fffffff, 0x7fffffff};
+  if (margin < 0.0f) return r;
+  const float4 g0 = W.g0[sl], sc = W.span[sl];
+  const float ka = W.g1[sl].w;
+  const float dy0 = (float)(ty * 16) + 0.5f - g0.y;
+  const float dy1 =
+      fminf((float)(P.height - 1) + 0.5f, (float)(ty * 16 + 15) + 0.5f) - g0.y;
+  const float yr = fminf(fmaxf(sc.w, dy0), dy1);
+  const float yl = fminf(fmaxf(-sc.w, dy0), dy1);
+  const float dr = sc.x - sc.z * yr * yr, dl = sc.x - sc.z * yl * yl;
+  const float lo = (float)bx.x, hi = (float)bx.z;
+  if (dr < 0.0f || dl < 0.0f) {  // the row lies beyond the ellipse
+    r.m1 = r.m0 - 1;
+    return r;
+  }
+  const float xr = g0.x + (ka * yr + __builtin_amdgcn_sqrtf(dr));
+  const float xl = g0.x + (ka * yl - __builtin_amdgcn_sqrtf(dl));
+  // tiles t with 16 t + 0.5 <= xr and 16 t + 15.5 >= xl
+  r.m0 = (int)fminf(fmaxf(ceilf((xl - margin - 15.5f) * 0.0625f), lo), hi + 1.0f);
+  r.m1 = (int)fmaxf(fminf(floorf((xr + margin - 0.5f) * 0.0625f), hi), lo - 1.0f);
+  const float inw = sc.w * kSpanDown;
+  const float zr = fminf(fmaxf(inw, dy0), dy1);
+  const float zl = fminf(fmaxf(-inw, dy0), dy1);
+  const float er = sc.y - sc.z * zr * zr, el = sc.y - sc.z * zl * zl;
+  if (er < 0.0f || el < 0.0f) return r;
+  const float ur = g0.x + (ka * zr + __builtin_amdgcn_sqrtf(er));
+  const float ul = g0.x + (ka * zl - __builtin_amdgcn_sqrtf(el)) + margin;
+  const int c0 = (int)fminf(fmaxf(ceilf((ul - 15.5f) * 0.0625f), lo), hi + 1.0f);
+  int c1 = (int)fmaxf(fminf(floorf((ur - margin - 0.5f) * 0.0625f), hi), lo - 1.0f);
+  // (the image's last column of tiles may end before 16 t + 15.5)
+  if (c1 == P.tiles_x - 1 && !((float)(P.width - 1) + 0.5f >= ul)) --c1;
+  if (c0 <= c1 && c0 >= r.m0 && c1 <= r.m1) {
+    r.c0 = c0;
+    r.c1 = c1;
+  }
+  return r;
+}
+
+// The exact test of one tile of the slot's splat.
+template <int kS>
+__device__ __forceinline__ bool tile_hit(const RasterParams& P,
+                                         const WalkSlots<kS>& W, int sl,
+                                         int tx, int ty) {
+  const float4 g0 = W.g0[sl], g1 = W.g1[sl];
+  const int fl = W.flags[sl];
+  ConicSlopes ks;
+  ks.kc = g1.z;
+  ks.ka = g1.w;
+  ks.use_c = (fl & 1) != 0;
+  ks.use_a = (fl & 2) != 0;
+  float rx0, ry0, rx1, ry1;
+  tile_rect(tx, ty, P.width, P.height, rx0, ry0, rx1, ry1);
+  return ellipse_hits_rect(g0.x, g0.y, g0.z, g0.w, g1.x, ks, g1.y, rx0, ry0,
+                           rx1, ry1);
+}
+
+// Stages this lane's splat (lanes below kS) and returns the rows of the
+// wavefront's boxes.  With P.live the box is P.boxes[source], which holds
+// the live tiles.  Rows fit in int32: tiles per image are limited to 2^24 on
+// the host.
 template <int kS>
 __device__ __forceinline__ int walk_setup(const RasterParams& P, bool valid,
                                           const SplatGeom& s, int batch,
-                                          int source,
-                                          WalkSlots<kS>& W, int& n_inner) {
+                                          int source, WalkSlots<kS>& W) {
 #pragma clang fp contract(off)
   const int lane = threadIdx.x & 63;
-  int ncand = 0;
-  int4 box = make_int4(0, 0, 1, 0);
-  int4 inner = make_int4(0, 0, 0, 0);
-  n_inner = 0;
-  float4 g1 = make_float4(s.c, 0.0f, 0.0f, 0.0f);
-  int flags = 0;
-  float tau;
-  if (valid && P.live != nullptr) {
-    const uint2 lb = P.boxes[source];
-    if (alpha_support(s.o, P.alpha_thr, P.eps, tau) && lb.y != 0u) {
-      box = make_int4((int)(lb.x & 0xffffu), (int)(lb.x >> 16),
-                      (int)(lb.y & 0xffffu), batch * P.tiles_per_image);
-      ncand = box.z * (int)(lb.y >> 16);
-      const ConicSlopes k = conic_slopes(s.a, s.b, s.c);
-      g1 = make_float4(s.c, tau, k.kc, k.ka);
-      flags = (k.use_c ? 1 : 0) | (k.use_a ? 2 : 0);
-    }
-  } else if (valid && alpha_support(s.o, P.alpha_thr, P.eps, tau)) {
-    const PixBox bb =
-        snugbox(s.mx, s.my, s.a, s.b, s.c, tau, P.width, P.height, P.eps);
-    if (bb.x0 <= bb.x1 && bb.y0 <= bb.y1) {
-      const int tx0 = bb.x0 >> 4, tx1 = bb.x1 >> 4;
-      const int ty0 = bb.y0 >> 4, ty1 = bb.y1 >> 4;
-      box = make_int4(tx0, ty0, tx1 - tx0 + 1, batch * P.tiles_per_image);
-      // (the inscribed rectangle is at most 2/pi of the ellipse's box)
-      if (box.z * (ty1 - ty0 + 1) >= 2 * kMinCertainHits) {
-        inner =
-            inner_tiles(s.mx, s.my, s.a, s.b, s.c, tau, tx0, ty0, tx1, ty1);
-        n_inner = inner.z * inner.w;
+  int rows = 0;
+  int4 box = make_int4(0, 0, -1, 0);
+  float tau = 0.0f;
+  if (valid && alpha_support(s.o, P.alpha_thr, P.eps, tau)) {
+    if (P.live != nullptr) {
+      const uint2 lb = P.boxes[source];
+      if (lb.y != 0u) {
+        box = make_int4((int)(lb.x & 0xffffu), (int)(lb.x >> 16),
+                        (int)(lb.x & 0xffffu) + (int)(lb.y & 0xffffu) - 1,
+                        batch * P.tiles_per_image);
+        rows = (int)(lb.y >> 16);
       }
-      ncand = box.z * (ty1 - ty0 + 1) - n_inner;
-      const ConicSlopes k = conic_slopes(s.a, s.b, s.c);
-      g1 = make_float4(s.c, tau, k.kc, k.ka);
-      flags = (k.use_c ? 1 : 0) | (k.use_a ? 2 : 0);
+    } else {
+      const PixBox bb =
+          snugbox(s.mx, s.my, s.a, s.b, s.c, tau, P.width, P.height, P.eps);
+      if (bb.x0 <= bb.x1 && bb.y0 <= bb.y1) {
+        box = make_int4(bb.x0 >> 4, bb.y0 >> 4, bb.x1 >> 4,
+                        batch * P.tiles_per_image);
+        rows = (bb.y1 >> 4) - box.y + 1;
+      }
     }
   }
-  int inc = ncand, inc_i = n_inner;
+  int inc = rows;
 #pragma unroll
   for (int off = 1; off < kS; off <<= 1) {
     const int y = __shfl_up(inc, off, 64);
-    const int yi = __shfl_up(inc_i, off, 64);
-    if (lane >= off) {
-      inc += y;
-      inc_i += yi;
-    }
+    if (lane >= off) inc += y;
   }
   if (lane < kS) {
+    ConicSlopes k{0.0f, 0.0f, false, false};
+    float margin = -1.0f;
+    float4 span = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+    if (rows > 0) {
+      k = conic_slopes(s.a, s.b, s.c);
+      span = span_constants(s, tau, k, margin);
+    }
     W.g0[lane] = make_float4(s.mx, s.my, s.a, s.b);
-    W.g1[lane] = g1;
+    W.g1[lane] = make_float4(s.c, tau, k.kc, k.ka);
+    W.span[lane] = span;
     W.box[lane] = box;
-    W.inner[lane] = inner;
-    W.flags[lane] = flags;
+    W.margin[lane] = margin;
+    W.flags[lane] = (k.use_c ? 1 : 0) | (k.use_a ? 2 : 0);
     W.cend[lane] = inc;
-    W.first[lane] = inc - ncand;
-    W.ni_incl[lane] = inc_i;
+    W.first[lane] = inc - rows;
   }
   __builtin_amdgcn_wave_barrier();
   return __shfl(inc, kS - 1, 64);
 }
 
-// Tests the wavefront's candidates 64 at a time and calls on_hit(slot, tile)
-// for every hit (slot = 0..kS-1, the splat's lane in walk_setup).
-// A candidate's slot is the last splat whose first candidate is at or
-// before it (a splat without candidates shares its first index with the
-// next one and loses to it): the owner of the step's first candidate is
-// counted with a ballot, the splats that start inside the step mark their
-// position with an LDS max, and a prefix maximum over the lanes spreads the
-// marks -- one LDS round trip per step instead of a binary search.
-//
-// on_step(hm, hit, sl, tile, c0) is called by every lane once per step, hm
-// being the step's ballot of hits (hit, sl and tile: this lane's
-// candidate's; sl and tile mean nothing without the hit).  Candidates are enumerated splat by
-// splat, so the wavefront's hits arrive in splat order: the hits before a
-// position are counted with one running total and a lane-masked popcount,
-// without per-splat counters (whose atomics would serialise the lanes of one
-// splat on one LDS address).
-//
-// rec (may be null): the wavefront's recorded ballots (kHitSlab words, step
-// k's ballot at rec[k], as count_block records them for the same splats):
-// the steps they cover take their hits from there instead of the exact
-// test, and steps without a hit are skipped (on_step is not called).
+// The lane whose items cover position base + lane, given every lane's first
+// item (ascending; a lane without items shares its first with the next one
+// and loses to it): the owner of position base is counted with a ballot, the
+// lanes that start inside the 64 positions mark theirs with an LDS max, and a
+// prefix maximum spreads the marks -- one LDS round trip instead of a binary
+// search.
+__device__ __forceinline__ int owner_lane(uint32_t* own, int first, int base) {
+  const int lane = threadIdx.x & 63;
+  const int owner0 = __popcll(__ballot(first <= base)) - 1;  // first[0] = 0
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  own[lane] = lane == 0 ? (uint32_t)owner0 : 0u;
+  if (first > base && first < base + 64)
+    atomicMax(&own[first - base], (uint32_t)lane);
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+  return (int)wave_prefix_max(own[lane]);
+}
+
+// The wavefront's rows 64 at a time: on_rows(r0, sl, ty, span) is called by
+// every lane once per step with its row r0 + lane: the slot, the tile row and
+// the span (empty beyond the last row).
 template <int kS, typename Fn>
-__device__ __forceinline__ void walk_candidates(const RasterParams& P,
-                                                WalkSlots<kS>& W, int total,
-                                                const uint64_t* __restrict__ rec,
-                                                Fn&& on_step) {
-#pragma clang fp contract(off)
-  static_assert(kHitSlab % 64 == 0, "a slab is loaded 64 words at a time");
+__device__ __forceinline__ void walk_rows(const RasterParams& P,
+                                          WalkSlots<kS>& W, int total,
+                                          Fn&& on_rows) {
   const int lane = threadIdx.x & 63;
   const int first = lane < kS ? W.first[lane] : 0x7fffffff;
-  // (without certain hits in the wavefront every box is walked whole)
-  const bool any_inner = W.ni_incl[kS - 1] != 0;
-  uint64_t chunk = 0ull;  // lane l: the recorded ballot of step 64 (k / 64) + l
-  for (int c0 = 0; c0 < total; c0 += 64) {
-    const int step = c0 >> 6;
-    const bool recorded = rec != nullptr && step < kHitSlab;
-    uint64_t hm = 0ull;
-    if (recorded) {
-      if ((step & 63) == 0) chunk = rec[step + lane];  // < kHitSlab
-      hm = readlane64(chunk, step & 63);
-      if (hm == 0ull) continue;  // no hit among these candidates
+  for (int r0 = 0; r0 < total; r0 += 64) {
+    const int sl = owner_lane(W.own, first, r0);
+    const int r = r0 + lane;
+    RowSpan span{0, -1, 0x7fffffff, 0x7fffffff};
+    int ty = 0;
+    if (r < total) {
+      ty = W.box[sl].y + (r - W.first[sl]);
+      span = row_span(P, W, sl, ty);
     }
-    const int owner0 = __popcll(__ballot(first <= c0)) - 1;  // first[0] = 0
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    W.own[lane] = lane == 0 ? (uint32_t)owner0 : 0u;
-    if (first > c0 && first < c0 + 64)
-      atomicMax(&W.own[first - c0], (uint32_t)lane);
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-    const int sl = (int)wave_prefix_max(W.own[lane]);
-    const int c = c0 + lane;
-    bool hit = false;
-    int tile = 0;
-    if (c < total) {
-      // Candidate k of the splat's box less its certain hits (an inner
-      // rectangle at (ix, iy), iw x ih, in box coordinates): the rows above
-      // it in full, then ih rows of bw - iw tiles, then the rows below in
-      // full.
-      const int k = c - W.first[sl];
-      const int4 bx = W.box[sl];
-      int tx, ty;
-      if (any_inner) {
-        const int4 in = W.inner[sl];
-        const int top = bx.z * in.y;
-        const int mid_w = bx.z - in.z;
-        const int mid = mid_w * in.w;
-        const bool in_mid = k >= top && k < top + mid;
-        const bool below = k >= top + mid;
-        const int kk = below ? k - top - mid : (in_mid ? k - top : k);
-        const int w = in_mid ? mid_w : bx.z;
-        const int q = div_small(kk, w);
-        const int j = kk - q * w;
-        tx = bx.x + ((in_mid && j >= in.x) ? j + in.z : j);
-        ty = bx.y + q + (below ? in.y + in.w : (in_mid ? in.y : 0));
-      } else {
-        const int q = div_small(k, bx.z);
-        tx = bx.x + (k - q * bx.z);
-        ty = bx.y + q;
-      }
-      tile = bx.w + ty * P.tiles_x + tx;
-      if (recorded) {
-        // (of the live tiles' hits, with P.live)
-        hit = ((hm >> lane) & 1ull) != 0ull;
-      } else if (P.live == nullptr ||
-                 ((P.live[tile >> 5] >> (tile & 31)) & 1u) != 0u) {
-        const float4 g0 = W.g0[sl], g1 = W.g1[sl];
-        const int fl = W.flags[sl];
-        ConicSlopes ks;
-        ks.kc = g1.z;
-        ks.ka = g1.w;
-        ks.use_c = (fl & 1) != 0;
-        ks.use_a = (fl & 2) != 0;
-        float rx0, ry0, rx1, ry1;
-        tile_rect(tx, ty, P.width, P.height, rx0, ry0, rx1, ry1);
-        hit = ellipse_hits_rect(g0.x, g0.y, g0.z, g0.w, g1.x, ks, g1.y, rx0,
-                                ry0, rx1, ry1);
-      }
-    }
-    if (!recorded) hm = __ballot(hit);
-    on_step(hm, hit, sl, tile, c0);
+    on_rows(r0, sl, ty, span);
   }
+}
+
+// One row's hits, as runs of tiles: seg(first tile, tiles).  Lanes run on
+// their own rows.
+template <int kS, typename Fn>
+__device__ __forceinline__ void row_hits(const RasterParams& P,
+                                         const WalkSlots<kS>& W, int sl,
+                                         int ty, const RowSpan& r, Fn&& seg) {
+  if (r.m0 > r.m1) return;
+  const int tile0 = W.box[sl].w + ty * P.tiles_x;
+  auto live_runs = [&](int t, int n) {
+    if (P.live == nullptr) {
+      seg((uint32_t)(tile0 + t), (uint32_t)n);
+      return;
+    }
+    for (int i = tile0 + t; i < tile0 + t + n;) {  // word by word
+      const int end = min(tile0 + t + n, (i | 31) + 1);
+      uint32_t bits = P.live[i >> 5] >> (i & 31);
+      if (end - i < 32) bits &= (1u << (end - i)) - 1u;
+      while (bits != 0u) {
+        const int at = __builtin_ctz(bits);
+        const uint32_t rest = ~(bits >> at);
+        const int len = rest == 0u ? 32 : __builtin_ctz(rest);
+        seg((uint32_t)(i + at), (uint32_t)len);
+        bits = at + len >= 32 ? 0u : bits >> (at + len) << (at + len);
+      }
+      i = end;
+    }
+  };
+  for (int t = r.m0; t <= r.m1; ++t) {
+    if (t == r.c0) {
+      live_runs(r.c0, r.c1 - r.c0 + 1);
+      t = r.c1;
+    } else if (tile_hit(P, W, sl, t, ty)) {
+      live_runs(t, 1);
+    }
+  }
+}
+
+// Adds seg to the two copies of an LDS histogram of tile digits, cut where
+// the digit changes.
+__device__ __forceinline__ void add_digits(uint32_t* hist, int shift,
+                                           uint32_t t0, uint32_t n) {
+  uint32_t* const h = hist + (threadIdx.x & 1) * 257;
+  const uint32_t t1 = t0 + n;
+  while (t0 < t1) {
+    const uint32_t end = min(t1, ((t0 >> shift) + 1u) << shift);
+    atomicAdd(&h[(t0 >> shift) & 255u], end - t0);
+    t0 = end;
+  }
+}
+
+// Hands out the wavefront's hits 64 at a time: the rows' spans of a step are
+// laid end to end and the lanes take consecutive tiles, so that the wavefront
+// writes consecutive pairs.  on_step(hm, hit, sl, tile) is called by every
+// lane once per 64 tiles, hm being the ballot of hits (sl and tile mean
+// nothing without a hit).  Spans are enumerated splat by splat, so the hits
+// before a position are counted with one running total and a lane-masked
+// popcount.
+template <int kS, typename Fn>
+__device__ __forceinline__ void walk_hits(const RasterParams& P,
+                                          WalkSlots<kS>& W, int total,
+                                          Fn&& on_step) {
+  const int lane = threadIdx.x & 63;
+  walk_rows(P, W, total, [&](int, int sl, int ty, const RowSpan& r) {
+    const int n = max(r.m1 - r.m0 + 1, 0);
+    const int inc = wave_prefix_sum(n);
+    const int start = inc - n;
+    const int tiles = __builtin_amdgcn_readlane(inc, 63);
+    const int tile0 = W.box[sl].w + ty * P.tiles_x + r.m0;
+    const bool unsure = n > 0 && (r.c0 != r.m0 || r.c1 != r.m1);
+    const bool any_unsure = __ballot(unsure) != 0ull;  // uniform
+    for (int e0 = 0; e0 < tiles; e0 += 64) {
+      const int ow = owner_lane(W.own, start, e0);
+      const int off = e0 + lane - __shfl(start, ow, 64);
+      const int tile = __shfl(tile0, ow, 64) + off;
+      const int osl = __shfl(sl, ow, 64);
+      bool hit = e0 + lane < tiles;
+      if (any_unsure) {
+        const int tx = __shfl(r.m0, ow, 64) + off, oy = __shfl(ty, ow, 64);
+        const int c0 = __shfl(r.c0, ow, 64), c1 = __shfl(r.c1, ow, 64);
+        if (hit && (tx < c0 || tx > c1)) hit = tile_hit(P, W, osl, tx, oy);
+      }
+      if (P.live != nullptr && hit)
+        hit = ((P.live[tile >> 5] >> (tile & 31)) & 1u) != 0u;
+      on_step(__ballot(hit), hit, osl, tile);
+    }
+  });
 }
 
 // Hits among the lanes below `rel` of a step's hit ballot hm (rel in 0..64).
@@ -415,9 +479,7 @@ __device__ __forceinline__ void pack_record(
 // to hist_row[0..255]: the pair sort's histogram, in partials that a later
 // launch sums (it counts every hit, the emit only those below its capacity:
 // the two differ only when the capacity is short, and then the binning is
-// redone).  With hit_bits the block records each wavefront's first kHitSlab
-// step ballots at hit_bits[w * kHitSlab + step] (w = vb * kW + wavefront:
-// the splats' index / kS), for an emit that walks the same splats.
+// redone).
 template <int kW, int kS>
 __device__ __forceinline__ void count_block(
     const RasterParams& P, const float* __restrict__ means2d,
@@ -426,8 +488,7 @@ __device__ __forceinline__ void count_block(
     int32_t* __restrict__ splat_count, int32_t* __restrict__ block_sums,
     uint32_t* __restrict__ zero_words, int64_t n_zero_words, int vb, int nvb,
     CountLds<kW, kS>& S, uint32_t* lds_hist = nullptr,
-    uint32_t* __restrict__ hist_row = nullptr, int hist_shift = 0,
-    uint64_t* __restrict__ hit_bits = nullptr) {
+    uint32_t* __restrict__ hist_row = nullptr, int hist_shift = 0) {
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   for (int64_t i = (int64_t)vb * (64 * kW) + threadIdx.x; i < n_zero_words;
        i += (int64_t)nvb * (64 * kW))
@@ -447,54 +508,33 @@ __device__ __forceinline__ void count_block(
   s.c = conics[3 * o + 2];
   s.o = opacities[o];
   WalkSlots<kS>& W = S.walk[wave];
-  int n_inner;
   const int total =
       walk_setup(P, valid, s, o / P.gpb,
-                 P.orig_map != nullptr ? P.orig_map[o] : o, W, n_inner);
-  // Hits before the end of this lane's splat's candidates (lanes below
-  // kS): the running total of the steps before plus the hits below
-  // the end inside its step; a splat's count is the difference to the
-  // previous lane's.
+                 P.orig_map != nullptr ? P.orig_map[o] : o, W);
+  // Hits before the end of this lane's splat's rows (lanes below kS): the
+  // running total of the steps before plus the hits of the step's rows below
+  // the end; a splat's count is the difference to the previous lane's.
   const int my_end = lane < kS ? W.cend[lane] : 0;
   int run = 0, hits_to_end = 0;
-  // the recorded ballots, one store by the first lane per step (holding
-  // them in the lanes until 64 are stored together costs the walk more)
-  uint64_t* const rec =
-      hit_bits != nullptr ? hit_bits + (int64_t)(vb * kW + wave) * kHitSlab
-                          : nullptr;
-  walk_candidates(P, W, total, nullptr, [&](uint64_t hm, bool hit, int,
-                                            int tile, int c0) {
-    const int rel = my_end - c0;
-    if (rel > 0 && rel <= 64) hits_to_end = run + hits_below(hm, rel);
-    run += __popcll(hm);
-    if (rec != nullptr && lane == 0 && (c0 >> 6) < kHitSlab)
-      rec[c0 >> 6] = hm;
-    if (lds_hist != nullptr && hit)
-      atomicAdd(&lds_hist[(lane & 1) * 257 + (((uint32_t)tile >> hist_shift) & 255u)], 1u);
+  walk_rows(P, W, total, [&](int r0, int sl, int ty, const RowSpan& r) {
+    int n = 0;
+    row_hits(P, W, sl, ty, r, [&](uint32_t t0, uint32_t k) {
+      n += (int)k;
+      if (lds_hist != nullptr) add_digits(lds_hist, hist_shift, t0, k);
+    });
+    const int inc = wave_prefix_sum(n);
+    const int rel = my_end - r0;
+    const int below = __shfl(inc, min(max(rel - 1, 0), 63), 64);
+    if (rel > 0 && rel <= 64) hits_to_end = run + below;
+    run += __builtin_amdgcn_readlane(inc, 63);
   });
   if (lds_hist != nullptr) {
-    // the certain hits: each row of the splat's inner rectangle, cut where
-    // the digit changes
-    if (lane < kS && n_inner > 0) {
-      const int4 in = W.inner[lane];
-      const int4 bx = W.box[lane];
-      for (int r = 0; r < in.w; ++r) {
-        uint32_t t0 = (uint32_t)(bx.w + (bx.y + in.y + r) * P.tiles_x + bx.x + in.x);
-        const uint32_t t1 = t0 + (uint32_t)in.z;
-        while (t0 < t1) {
-          const uint32_t seg = min(t1, ((t0 >> hist_shift) + 1u) << hist_shift);
-          atomicAdd(&lds_hist[(lane & 1) * 257 + ((t0 >> hist_shift) & 255u)], seg - t0);
-          t0 = seg;
-        }
-      }
-    }
     __syncthreads();
     if (threadIdx.x < 256)
       hist_row[threadIdx.x] = lds_hist[threadIdx.x] + lds_hist[257 + threadIdx.x];
   }
   const int prev_end = __shfl_up(hits_to_end, 1, 64);
-  const int n =
-      valid ? hits_to_end - (lane == 0 ? 0 : prev_end) + n_inner : 0;
+  const int n = valid ? hits_to_end - (lane == 0 ? 0 : prev_end) : 0;
   if (valid) splat_count[orig] = n;
   // (the attributes are read again here rather than kept across the walk)
   if (valid && rec_orig != nullptr)
@@ -520,13 +560,11 @@ __global__ __launch_bounds__(kThreads) void count_kernel(
     const float* __restrict__ conics, const float* __restrict__ opacities,
     const float* __restrict__ colors, float4* __restrict__ rec_orig,
     int32_t* __restrict__ splat_count, int32_t* __restrict__ block_sums,
-    uint32_t* __restrict__ zero_words, int64_t n_zero_words,
-    uint64_t* __restrict__ hit_bits) {
+    uint32_t* __restrict__ zero_words, int64_t n_zero_words) {
   __shared__ CountLds<kWaves, kWalkSplats> S;
   count_block<kWaves, kWalkSplats>(P, means2d, conics, opacities, colors, rec_orig,
                       splat_count, block_sums, zero_words, n_zero_words,
-                      (int)blockIdx.x, (int)gridDim.x, S, nullptr, nullptr, 0,
-                      hit_bits);
+                      (int)blockIdx.x, (int)gridDim.x, S);
 }
 
 // The count next to the run step of the small-image depth order, in one
@@ -757,12 +795,11 @@ __global__ __launch_bounds__(kThreads) void pack_records_kernel(
 }
 
 // emit_kernel<false, true>: the walk in original order over the count's
-// records, with the count's recorded step ballots.
+// records.
 struct EmitOrig {
   const float4* rec;       // the count's original-order records (hit count
                            // in the slot)
   const int2* slot;        // per orig: {pair offset, gid} (pack_kernel)
-  const uint64_t* bits;    // the count's step ballots (count_block), or null
 };
 
 // emit_kernel<true>: the pair offsets are scanned by the emit itself.
@@ -801,10 +838,7 @@ __device__ __forceinline__ void put_pair(uint32_t* __restrict__ keys,
 // below N by construction).  Otherwise splat_offsets (and N in
 // splat_offsets[num_splats]) come from pack_kernel.  kOrig (not with kScan):
 // the workgroups walk the splats in original order, the count's walk, from
-// its records (eo.rec) with its recorded ballots (eo.bits): a splat's pairs
-// start at eo.slot[orig].x, its certain hits first, then its walk hits,
-// numbered by the wavefront's walk hits of the splats before it (its count
-// less its certain hits).
+// its records (eo.rec): a splat's pairs start at eo.slot[orig].x.
 template <bool kScan, bool kOrig, int kS>
 __global__ __launch_bounds__(kThreads) void emit_kernel(
     RasterParams P, const float4* __restrict__ packed,
@@ -817,8 +851,8 @@ __global__ __launch_bounds__(kThreads) void emit_kernel(
   static_assert(!(kScan && kOrig), "one source of offsets");
   __shared__ WalkSlots<kS> walk[kWaves];
   __shared__ int base[kWaves][kS];
-  // kOrig: per splat the first position of its walk hits less the wave's
-  // walk hits before it, and its gid
+  // kOrig: per splat its first position less the wavefront's hits before it,
+  // and its gid
   __shared__ int wbase[kOrig ? kWaves : 1][kS];
   __shared__ int wgid[kOrig ? kWaves : 1][kS];
   // the pair sort's digit histograms in kHistCopies copies (lane l adds to
@@ -847,7 +881,7 @@ __global__ __launch_bounds__(kThreads) void emit_kernel(
   const SplatGeom s{p0.x, p0.y, p0.z, p0.w, p1.x, p1.y};
   WalkSlots<kS>& W = walk[wave];
   int64_t n_eff;
-  int total, n_inner;
+  int total;
   if (kScan) {
     // exclusive offsets of the workgroup's gids: wavefront scans, the
     // workgroup's scan, and the totals of the workgroups before it (loaded
@@ -863,7 +897,7 @@ __global__ __launch_bounds__(kThreads) void emit_kernel(
     }
     if (lane == kS - 1) wsum[wave] = inc;
     total = walk_setup(P, valid, s, g / P.gpb,
-                       P.live != nullptr ? source_of(src, g) : 0, W, n_inner);
+                       P.live != nullptr ? source_of(src, g) : 0, W);
 #pragma unroll
     for (int off = 32; off > 0; off >>= 1) before += __shfl_xor(before, off, 64);
     if (lane == 0) wbefore[wave] = before;
@@ -893,46 +927,34 @@ __global__ __launch_bounds__(kThreads) void emit_kernel(
     const int2 sg = valid ? eo.slot[g] : make_int2(0, 0);
     n_eff = min(capacity, (int64_t)max(splat_offsets[P.num_splats], 0));
     total = walk_setup(P, valid, s, g / P.gpb,
-                       P.orig_map != nullptr ? P.orig_map[g] : g, W, n_inner);
-    // walk hits of the wavefront's splats up to this one
-    const int w = n - n_inner;
-    int inc = w;
+                       P.orig_map != nullptr ? P.orig_map[g] : g, W);
+    // hits of the wavefront's splats up to this one
+    int inc = n;
 #pragma unroll
     for (int off = 1; off < kS; off <<= 1) {
       const int y = __shfl_up(inc, off, 64);
       if (lane >= off) inc += y;
     }
     if (lane < kS) {
-      base[wave][lane] = sg.x;
-      wbase[kOrig ? wave : 0][lane] = sg.x + n_inner - (inc - w);
+      wbase[kOrig ? wave : 0][lane] = sg.x - (inc - n);
       wgid[kOrig ? wave : 0][lane] = sg.y;
     }
   } else {
     if (lane < kS) base[wave][lane] = splat_offsets[g];
     n_eff = min(capacity, (int64_t)max(splat_offsets[P.num_splats], 0));
     total = walk_setup(P, valid, s, g / P.gpb,
-                       P.live != nullptr ? source_of(src, g) : 0, W, n_inner);
+                       P.live != nullptr ? source_of(src, g) : 0, W);
   }
   const int gid0 = gid - lane;
   // The wavefront's splats own consecutive ranges starting at the first
-  // one's offset; each range starts with the splat's certain hits
-  // (inner_tiles, written below) and the walk's hits follow, arriving in
-  // splat order: a walk hit's position is that offset plus the hits before
-  // it (running total + lanes below) plus the certain hits of the splats up
-  // to its own.
-  const int64_t wave_base = base[wave][0];
+  // one's offset, and the hits arrive in splat order: a hit's position is
+  // that offset plus the hits before it.
+  const int64_t wave_base = kOrig ? 0 : base[wave][0];
   int64_t run = 0;
-  const uint64_t* const rec =
-      (kOrig && eo.bits != nullptr)
-          ? eo.bits + (int64_t)(vb * kWaves + wave) * kHitSlab
-          : nullptr;
-  walk_candidates(P, W, total, rec, [&](uint64_t hm, bool hit, int sl,
-                                        int tile, int) {
+  walk_hits(P, W, total, [&](uint64_t hm, bool hit, int sl, int tile) {
     const int64_t pos =
-        kOrig ? (hit ? (int64_t)wbase[kOrig ? wave : 0][sl] : 0) + run +
-                    hits_below(hm, lane)
-              : wave_base + run + hits_below(hm, lane) +
-                    (hit ? W.ni_incl[sl] : 0);
+        (kOrig ? (hit ? (int64_t)wbase[kOrig ? wave : 0][sl] : 0) : wave_base) +
+        run + hits_below(hm, lane);
     run += __popcll(hm);
     // (pos >= 0 whenever n_eff > 0, unless a look-back of the depth sort
     // gave up and left the original-order offsets unwritten)
@@ -946,30 +968,6 @@ __global__ __launch_bounds__(kThreads) void emit_kernel(
                   1u);
     }
   });
-  // The certain hits of each splat, row by row at the start of its range.
-  uint64_t with_inner = __ballot(lane < kS && n_inner > 0);
-  for (; with_inner != 0ull; with_inner &= with_inner - 1ull) {
-    const int sl = (int)__builtin_ctzll(with_inner);
-    const int4 in = W.inner[sl];
-    const int ni = in.z * in.w;
-    const int4 bx = W.box[sl];
-    const int64_t off = base[wave][sl];
-    const uint32_t sg = kOrig ? (uint32_t)wgid[kOrig ? wave : 0][sl]
-                              : (uint32_t)(gid0 + sl);
-    for (int i = lane; i < ni; i += 64) {
-      const int dy = div_small(i, in.z);
-      const int tile = bx.w + (bx.y + in.y + dy) * P.tiles_x +
-                       (bx.x + in.x + (i - dy * in.z));
-      const int64_t pos = off + i;
-      if (pos < n_eff && (!kOrig || pos >= 0)) {
-        put_pair(keys, vals, key_bytes, pos, (uint32_t)tile, sg);
-        for (int p = 0; p < pair_passes; ++p)
-          atomicAdd(&h[p][lane % kHistCopies]
-                       [((uint32_t)tile >> (hist_shift + 8 * p)) & 255u],
-                    1u);
-      }
-    }
-  }
   // (3) this workgroup's digit histograms for the pair sort: added to the
   // zeroed global histograms (ghist_direct, few workgroups) or stored as
   // hist_partials[(p * 256 + d) * nblk + workgroup] for hist_reduce_kernel
@@ -1367,7 +1365,7 @@ template <int kS>
 __device__ __forceinline__ int tile_walk_setup(
     const RasterParams& P, const float* __restrict__ means2d,
     const float* __restrict__ conics, const float* __restrict__ opacities,
-    int orig, bool valid, WalkSlots<kS>& W, int& n_inner) {
+    int orig, bool valid, WalkSlots<kS>& W) {
   const int o = valid ? orig : P.num_splats - 1;
   SplatGeom s;
   s.mx = means2d[2 * o + 0];
@@ -1376,7 +1374,7 @@ __device__ __forceinline__ int tile_walk_setup(
   s.b = conics[3 * o + 1];
   s.c = conics[3 * o + 2];
   s.o = opacities[o];
-  return walk_setup(P, valid, s, o / P.gpb, o, W, n_inner);
+  return walk_setup(P, valid, s, o / P.gpb, o, W);
 }
 
 template <int kS>
@@ -1399,29 +1397,13 @@ __global__ __launch_bounds__(kTileThreads) void tile_count_kernel(
   const int orig = ((int)blockIdx.x * kTileWaves + wave) * kS + lane;
   const bool valid = lane < kS && orig < P.num_splats;
   WalkSlots<kS>& W = walk[wave];
-  int n_inner;
-  const int total = tile_walk_setup(P, means2d, conics, opacities, orig, valid,
-                                    W, n_inner);
-  walk_candidates(P, W, total, nullptr,
-                  [&](uint64_t, bool hit, int, int tile, int) {
-                    if (hit)
-                      atomicAdd(&hist[(lane & 1) * 257 +
-                                      (((uint32_t)tile >> shift) & 255u)],
-                                1u);
-                  });
-  if (lane < kS && n_inner > 0) {
-    const int4 in = W.inner[lane];
-    const int4 bx = W.box[lane];
-    for (int r = 0; r < in.w; ++r) {
-      uint32_t t0 = (uint32_t)(bx.w + (bx.y + in.y + r) * P.tiles_x + bx.x + in.x);
-      const uint32_t t1 = t0 + (uint32_t)in.z;
-      while (t0 < t1) {
-        const uint32_t seg = min(t1, ((t0 >> shift) + 1u) << shift);
-        atomicAdd(&hist[(lane & 1) * 257 + ((t0 >> shift) & 255u)], seg - t0);
-        t0 = seg;
-      }
-    }
-  }
+  const int total =
+      tile_walk_setup(P, means2d, conics, opacities, orig, valid, W);
+  walk_rows(P, W, total, [&](int, int sl, int ty, const RowSpan& r) {
+    row_hits(P, W, sl, ty, r, [&](uint32_t t0, uint32_t n) {
+      add_digits(hist, shift, t0, n);
+    });
+  });
   if (valid)
     store_record(packed, orig,
                  record_of(P, means2d, conics, colors, opacities, orig,
@@ -1466,9 +1448,8 @@ __global__ __launch_bounds__(kTileThreads) void tile_emit_kernel(
     red[1][t] = before;
   }
   WalkSlots<kS>& W = walk[wave];
-  int n_inner;
-  const int total = tile_walk_setup(P, means2d, conics, opacities, orig, valid,
-                                    W, n_inner);
+  const int total =
+      tile_walk_setup(P, means2d, conics, opacities, orig, valid, W);
   if (lane < kS) dkey[wave][lane] = valid ? depth_key(depths[orig]) : 0u;
   __syncthreads();
   unsigned long long inc = 0;
@@ -1504,28 +1485,13 @@ __global__ __launch_bounds__(kTileThreads) void tile_emit_kernel(
   }
   __syncthreads();
   const uint32_t low = (1u << shift) - 1u;
-  auto put = [&](uint32_t tile, int sl) {
-    const uint32_t pos = atomicAdd(&cursor[(tile >> shift) & 255u], 1u);
+  walk_hits(P, W, total, [&](uint64_t, bool hit, int sl, int tile) {
+    if (!hit) return;
+    const uint32_t pos = atomicAdd(&cursor[((uint32_t)tile >> shift) & 255u], 1u);
     if (pos < (uint32_t)capacity)
-      pairs[pos] = make_uint2(dkey[wave][sl],
-                              (tile & low) << 24 | (uint32_t)(orig0 + sl));
-  };
-  walk_candidates(P, W, total, nullptr,
-                  [&](uint64_t, bool hit, int sl, int tile, int) {
-                    if (hit) put((uint32_t)tile, sl);
-                  });
-  uint64_t with_inner = __ballot(lane < kS && n_inner > 0);
-  for (; with_inner != 0ull; with_inner &= with_inner - 1ull) {
-    const int sl = (int)__builtin_ctzll(with_inner);
-    const int4 in = W.inner[sl];
-    const int4 bx = W.box[sl];
-    for (int i = lane; i < in.z * in.w; i += 64) {
-      const int dy = div_small(i, in.z);
-      put((uint32_t)(bx.w + (bx.y + in.y + dy) * P.tiles_x +
-                     (bx.x + in.x + (i - dy * in.z))),
-          sl);
-    }
-  }
+      pairs[pos] = make_uint2(dkey[wave][sl], ((uint32_t)tile & low) << 24 |
+                                                  (uint32_t)(orig0 + sl));
+  });
 }
 
 __global__ __launch_bounds__(kTileThreads) void tile_sort_kernel(
@@ -1663,21 +1629,17 @@ int count_blocks(const RasterParams& P) {
   return (P.num_splats + kWalkBlockSplats - 1) / kWalkBlockSplats;
 }
 
-size_t hit_bits_words(const RasterParams& P) {
-  return (size_t)count_blocks(P) * kWaves * kHitSlab;
-}
-
 int launch_count(const RasterParams& P, const float* means2d,
                  const float* conics, const float* opacities,
                  int32_t* splat_count, int32_t* block_sums,
                  int32_t* pair_count, uint32_t* zero_words,
                  int64_t n_zero_words, hipStream_t stream,
-                 const float* colors, float* rec_orig, uint64_t* hit_bits) {
+                 const float* colors, float* rec_orig) {
   const int nblk = count_blocks(P);
   launch_traced("count_kernel", count_kernel, dim3((unsigned)nblk),
                 dim3(kThreads), 0, stream, P, means2d, conics, opacities,
                 colors, reinterpret_cast<float4*>(rec_orig), splat_count,
-                block_sums, zero_words, n_zero_words, hit_bits);
+                block_sums, zero_words, n_zero_words);
   int rc = check_launch("count_kernel");
   if (rc || pair_count == nullptr) return rc;
   launch_traced("sum_kernel", sum_kernel, dim3(1), dim3(kThreads), 0, stream,
@@ -1686,10 +1648,10 @@ int launch_count(const RasterParams& P, const float* means2d,
 }
 
 // Splats of many tiles each: a wavefront of 32 of them walks for long while
-// few wavefronts run (two images of 100K 3D splats at 35 pairs per splat:
-// emit 80 us with 32, 68 with 16), and with few splats in all fewer per
-// wavefront only fill the chip (512 splats: emit 8.5 us with 32, 6.6 with
-// 16).  64K splats of 5 to 13 pairs are as fast or faster with 32 (their
+// few wavefronts run (two images of 100K 3D splats at 29 pairs per splat:
+// emit 80 us with 32, 68 with 16 when every tile was tested, 45 with 16 now),
+// and with few splats in all fewer per wavefront only fill the chip (512
+// splats: emit 8.5 us with 32, 6.6 with 16).  64K splats of 5 to 13 pairs are as fast or faster with 32 (their
 // rank launch adds to more totals otherwise, 15 against 22 us).
 constexpr int kFewSplatPairs = 24;
 constexpr int kFewSplats = 1 << 14;
@@ -1817,8 +1779,7 @@ int launch_emit(const RasterParams& P, const float* packed,
                   sc, EmitOrig{});
   } else if (orig != nullptr) {
     const EmitOrig eo{reinterpret_cast<const float4*>(orig->rec_orig),
-                      reinterpret_cast<const int2*>(orig->orig_slot),
-                      orig->hit_bits};
+                      reinterpret_cast<const int2*>(orig->orig_slot)};
     launch_traced("emit_kernel<orig>", emit_kernel<false, true, kWalkSplats>,
                   dim3((unsigned)nblk), dim3(kThreads), 0, stream, P,
                   reinterpret_cast<const float4*>(packed), splat_offsets,

@@ -186,7 +186,7 @@ struct CountLayout {
   gs::RadixPlan depth;
   size_t scan_status, scan_ticket, pair_ghist, pair_tickets, ctl_end;
   size_t splat_count, block_sums, gid_count, depth_buffers, rec_orig;
-  size_t orig_slot, hit_bits, total;
+  size_t orig_slot, total;
 };
 
 CountLayout count_layout(const RasterParams& P) {
@@ -219,12 +219,9 @@ CountLayout count_layout(const RasterParams& P) {
   L.rec_orig = off;  // the count's original-order records (gsplat_hip_bin)
   off += gs::align_up((size_t)P.num_splats * GSPLAT_RECORD_FLOATS * sizeof(float),
                       256);
-  // gsplat_hip_bin's original-order emit: per splat {pair offset, gid}, and
-  // the count's recorded step ballots
+  // gsplat_hip_bin's original-order emit: per splat {pair offset, gid}
   L.orig_slot = off;
   off += gs::align_up((size_t)P.num_splats * 2 * sizeof(int32_t), 256);
-  L.hit_bits = off;
-  off += gs::align_up(gs::hit_bits_words(P) * sizeof(uint64_t), 256);
   L.total = off;
   return L;
 }
@@ -376,9 +373,6 @@ int bin_count_impl(const gsplat_raster_meta* meta, const float* means2d,
                           colors,
                           colors != nullptr
                               ? reinterpret_cast<float*>(base + L.rec_orig)
-                              : nullptr,
-                          colors != nullptr
-                              ? reinterpret_cast<uint64_t*>(base + L.hit_bits)
                               : nullptr);
 }
 }  // namespace
@@ -600,8 +594,7 @@ int bin_emit_impl(const gsplat_raster_meta* meta, const float* packed,
   const int32_t* n_dev = splat_offsets + P.num_splats;
   const gs::EmitOrigArgs orig_args{
       reinterpret_cast<const float*>(cbase + C.rec_orig),
-      reinterpret_cast<const int32_t*>(cbase + C.orig_slot),
-      reinterpret_cast<const uint64_t*>(cbase + C.hit_bits)};
+      reinterpret_cast<const int32_t*>(cbase + C.orig_slot)};
   const gs::EmitOrigArgs* orig =
       orig_walk && scan == nullptr ? &orig_args : nullptr;
   // Images of 2^9..2^16 tiles whose buffers hold at most kBucketChunk pairs

@@ -219,19 +219,13 @@ int launch_slice_gather(const RasterParams& P, const SliceBuffers& Q,
 int count_blocks(const RasterParams& P);
 // With colors and rec_orig (float [BG*16]) the count also writes each
 // splat's packed record in original order with its hit count in the orig
-// slot, for launch_pack's rec_orig.  With hit_bits (hit_bits_words(P)
-// words) it records each wavefront's first kHitSlab walk steps' hit
-// ballots, which launch_emit's original-order walk then reads instead of
-// testing those candidates again.
-constexpr int kHitSlab = 128;
-size_t hit_bits_words(const RasterParams& P);
+// slot, for launch_pack's rec_orig.
 int launch_count(const RasterParams& P, const float* means2d,
                  const float* conics, const float* opacities,
                  int32_t* splat_count, int32_t* block_sums,
                  int32_t* pair_count, uint32_t* zero_words,
                  int64_t n_zero_words, hipStream_t stream,
-                 const float* colors = nullptr, float* rec_orig = nullptr,
-                 uint64_t* hit_bits = nullptr);
+                 const float* colors = nullptr, float* rec_orig = nullptr);
 // count_depth_runs: the count (splat_count, zero_words as above; no block
 // sums and no N) and the first launch of the small-image depth order (runs
 // into depth_buffers) as one launch.  Requires P.num_splats > 0 and
@@ -306,13 +300,11 @@ struct EmitScanArgs {
   int walk;  // splats per wavefront (walk_splats)
 };
 // With orig (not with scan), the emit walks the splats in original order,
-// as the count did: from the count's records (rec_orig, launch_count's),
-// the pack's orig_slot and the count's hit_bits (may be null: every
-// candidate is tested), writing the same pairs at the same positions.
+// as the count did: from the count's records (rec_orig, launch_count's) and
+// the pack's orig_slot, writing the same pairs in the same splats' ranges.
 struct EmitOrigArgs {
   const float* rec_orig;
   const int32_t* orig_slot;
-  const uint64_t* hit_bits;
 };
 int launch_emit(const RasterParams& P, const float* packed,
                 const int32_t* splat_offsets, int64_t capacity, uint32_t* keys,
