@@ -1325,7 +1325,7 @@ __global__ __launch_bounds__(kBucketThreads) void bucket_sort_kernel(
 }
 
 // ---- The tile-sorted binning (launch_tile_sorted): three launches instead of
-// five for scenes of up to 128K splats.  Latency bounds them: a chain of
+// five for scenes of up to 256K splats.  Latency bounds them: a chain of
 // dependent loads and LDS steps each, 3 to 9 MB moved.  The splats keep their
 // original order, so there is no depth order to wait for (run sort and ranks,
 // 30 us of serial chains at 64K splats); instead each pair carries its splat's depth
@@ -1344,21 +1344,26 @@ __global__ __launch_bounds__(kBucketThreads) void bucket_sort_kernel(
 //
 // Measured against the one-call binning (us for count, emit and sort; the five
 // launches): 64K splats at 1080p 11.9 + 13.1 + 6.5 against 60 in all, at 4096 x
-// 4096 14.3 + 17.8 + 7.3 against 68; 128K splats at 1080p 15.0 + 15.2 + 11.8
+// 4096 11.1 + 15.9 + 7.3 against 63; 128K splats at 1080p 15.0 + 15.2 + 11.8
 // against 83; 5000 splats at 1080p 8.1 + 8.4 + 4.2 against 43; 16K splats at
 // 512 x 512 8.7 + 8.7 + 6.1 against 45; two images of 32K splats at 600 x 800
-// 10.0 + 12.4 + 8.7 against 55.
+// 10.0 + 12.4 + 8.7 against 55; 262K splats in seven images of 769 x 729 14.8 +
+// 19.2 + 26.7 against 122, in four of 1811 x 1632 14.7 + 17.8 + 11.0 against 112.
 constexpr int kTileWaves = 16;
 constexpr int kTileThreads = 64 * kTileWaves;
-// A bucket that the sort's LDS does not hold (64 KB of pairs, 8 in registers
-// per thread), or a tile list so long that ranking its entries against each
-// other (its length per entry: a full bucket of lists of 512 takes 8 x 512
-// steps) costs more than the depth order, sets kTileSkewed in the long-range
-// flag and leaves its tiles empty; the caller bins such a scene by the other
-// path.
-constexpr int kTileRounds = 8;
-constexpr int kTileBucket = kTileRounds * kTileThreads;
-constexpr int kTileList = 512;
+// A bucket that the sort's LDS does not hold (128 KB of pairs, 16 in registers
+// per thread), a tile list above kTileList, or a bucket whose lists take
+// longer to rank (their lengths squared, about 40 us per million, bound by
+// the 64-bit compares; two 32-bit subtractions, or four entries per thread
+// that share their reads, were slower) than the depth order and the pair sort
+// of the one-call binning, sets kTileSkewed in the long-range flag and leaves
+// its tiles empty; the caller bins such a scene by the other path.  1.2M
+// squares (131K splats at 2000 x 2000, 121 pairs a tile): sort 43 us, 76 in
+// all against 120; 1.9M (131K at 1080p, 241 a tile): 72, 106 against 119;
+// 60K splats at 745 x 837 (220 a tile, 0.5M): 33, 58 against 76.
+constexpr int kTileRounds = kTileBucket / kTileThreads;
+constexpr uint32_t kTileWorkSmall = 1u << 20;  // up to 64K splats
+constexpr uint32_t kTileWork = 3u << 19;
 
 // The wavefront's splats staged for the walk, in original order.
 template <int kS>
@@ -1496,13 +1501,14 @@ __global__ __launch_bounds__(kTileThreads) void tile_emit_kernel(
 
 __global__ __launch_bounds__(kTileThreads) void tile_sort_kernel(
     const uint2* __restrict__ pairs, const uint32_t* __restrict__ bucket_start,
-    int64_t capacity, int num_tiles, int low_bits,
+    int64_t capacity, int num_tiles, int low_bits, uint32_t most_work,
     uint32_t* __restrict__ binned_ids, int32_t* __restrict__ tile_offsets,
     int32_t* __restrict__ ctl) {
   __shared__ uint64_t list[kTileBucket];  // depth key << 32 | tile << 24 | index
   __shared__ uint32_t cnt[256], start[256];
   __shared__ uint32_t wsum[4];
   __shared__ int skewed;
+  __shared__ uint32_t work;  // below 2^28: a bucket's lists' lengths squared
   const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
   const int b = (int)blockIdx.x;
   const int tile0 = b << low_bits, ndig = 1 << low_bits;
@@ -1511,7 +1517,10 @@ __global__ __launch_bounds__(kTileThreads) void tile_sort_kernel(
   const uint32_t end = min(bucket_start[b + 1], cap);
   const uint32_t size = end - base;
   if (t < 256) cnt[t] = 0u;
-  if (t == 0) skewed = size > (uint32_t)kTileBucket;
+  if (t == 0) {
+    skewed = size > (uint32_t)kTileBucket;
+    work = 0u;
+  }
   if (b == (int)gridDim.x - 1 && t == 0) tile_offsets[num_tiles] = (int32_t)end;
   __syncthreads();
   const bool fits = size <= (uint32_t)kTileBucket;
@@ -1540,9 +1549,10 @@ __global__ __launch_bounds__(kTileThreads) void tile_sort_kernel(
   if (t < 256) {
     if (lane == 63) wsum[wave] = inc;
     if (n > (uint32_t)kTileList) skewed = 1;
+    if (n > 0u) atomicAdd(&work, n * n);
   }
   __syncthreads();
-  const bool skip = skewed != 0;  // uniform
+  const bool skip = skewed != 0 || work > most_work;  // uniform
   if (t < 256) {
     for (int w = 0; w < wave; ++w) inc += wsum[w];
     start[t] = inc - n;
@@ -1890,9 +1900,9 @@ int launch_bucket_sort(const BucketSortArgs& A, hipStream_t stream) {
 
 // Splats per wavefront: 16 up to 64K splats (a block per CU: count + emit at
 // 64K splats 25.0 us at 1080p, 32.1 at 4096 x 4096, with 32 25.5 and 35.7), 32
-// above (each emit block reads every block's counts).
+// and 64 above (each emit block reads every block's counts: at most 256).
 static int tile_walk(const RasterParams& P) {
-  return P.num_splats <= (1 << 16) ? 16 : 32;
+  return P.num_splats <= (1 << 16) ? 16 : P.num_splats <= (1 << 17) ? 32 : 64;
 }
 
 int tile_blocks(const RasterParams& P) {
@@ -1908,16 +1918,20 @@ int launch_tile_sorted(const RasterParams& P, const float* means2d,
                        void* pairs, int32_t* binned_ids, int32_t* tile_offsets,
                        const ZeroSpan zero[2], hipStream_t stream) {
   const unsigned blocks = (unsigned)tile_blocks(P);
-  const bool narrow = tile_walk(P) == 16;
+  const int walk = tile_walk(P);
   launch_traced("tile_count_kernel",
-                narrow ? tile_count_kernel<16> : tile_count_kernel<32>,
+                walk == 16   ? tile_count_kernel<16>
+                : walk == 32 ? tile_count_kernel<32>
+                             : tile_count_kernel<64>,
                 dim3(blocks), dim3(kTileThreads), 0, stream, P, means2d,
                 conics, colors, opacities, reinterpret_cast<float4*>(packed),
                 parts, low_bits, ctl, zero[0], zero[1]);
   int rc = check_launch("tile_count_kernel");
   if (rc) return rc;
   launch_traced("tile_emit_kernel",
-                narrow ? tile_emit_kernel<16> : tile_emit_kernel<32>,
+                walk == 16   ? tile_emit_kernel<16>
+                : walk == 32 ? tile_emit_kernel<32>
+                             : tile_emit_kernel<64>,
                 dim3(blocks), dim3(kTileThreads), 0, stream, P, means2d,
                 conics, opacities, depths, parts, low_bits, capacity,
                 reinterpret_cast<uint2*>(pairs), bucket_start, ctl);
@@ -1928,8 +1942,9 @@ int launch_tile_sorted(const RasterParams& P, const float* means2d,
                                 low_bits)),
                 dim3(kTileThreads), 0, stream,
                 reinterpret_cast<const uint2*>(pairs), bucket_start, capacity,
-                P.num_tiles, low_bits, reinterpret_cast<uint32_t*>(binned_ids),
-                tile_offsets, ctl);
+                P.num_tiles, low_bits,
+                P.num_splats <= (1 << 16) ? kTileWorkSmall : kTileWork,
+                reinterpret_cast<uint32_t*>(binned_ids), tile_offsets, ctl);
   return check_launch("tile_sort_kernel");
 }
 

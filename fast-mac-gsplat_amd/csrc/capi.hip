@@ -150,8 +150,7 @@ int make_params(const gsplat_raster_meta* m, RasterParams& P) {
 // faster one at every size measured (5000 splats in 2048 tiles 20.6 us against
 // 42.4, 16K in 1024 tiles 23.5 against 45.4); the scenes below both lines keep
 // the one-call binning's launches, whose trace at 512 x 512 with 8000 splats
-// callers rely on.  Above 128K splats the counts that every emit block reads
-// (1 KB per block of 512 splats) are what grows: 15 us of emit at 128K.
+// callers rely on.
 constexpr int kTileMinSplats = 1 << 14;
 constexpr int kTileMinTiles = 1 << 11;
 
@@ -1658,13 +1657,23 @@ TileLayout tile_layout(const RasterParams& P, int64_t capacity) {
   L.total = L.pairs + gs::align_up((size_t)capacity * 8, 256);
   return L;
 }
-// The scenes that go by the tile-sorted binning, and the pair buffers of the
-// bucket form.
+// Buckets of 2^low_bits tiles, at most 256, as bucket_low_bits; -1 when the
+// buffer holds more pairs than the tile-sorted path's buckets and lists do.
+int tile_low_bits(const RasterParams& P, int64_t capacity) {
+  const int tile_bits = bits_for((int64_t)P.num_tiles - 1);
+  const int low_bits = tile_bits - 8;
+  if (low_bits < 1 || tile_bits > 16) return -1;
+  const int64_t buckets = ((int64_t)P.num_tiles + (1 << low_bits) - 1) >> low_bits;
+  return capacity <= buckets * gs::kTileBucket &&
+                 capacity <= (int64_t)P.num_tiles * gs::kTileList
+             ? low_bits
+             : -1;
+}
+// The scenes that go by the tile-sorted binning.
 bool tile_ok(const RasterParams& P, int64_t capacity) {
   return (P.num_splats >= kTileMinSplats || P.num_tiles >= kTileMinTiles) &&
          P.num_splats <= gs::kTileMaxSplats &&
-         capacity > 0 && capacity <= 0x7fffffffLL &&
-         bucket_low_bits(P, capacity) >= 1;
+         capacity > 0 && tile_low_bits(P, capacity) >= 1;
 }
 }  // namespace
 
@@ -1693,9 +1702,10 @@ int gsplat_hip_tile_render(const gsplat_raster_meta* meta,
   int rc = make_params(meta, P);
   if (rc) return rc;
   if (!tile_ok(P, capacity)) {
-    gs::set_error("%s: needs %d splats or %d tiles, at most %d splats and the "
-                  "bucket form's pair buffers", what, kTileMinSplats,
-                  kTileMinTiles, gs::kTileMaxSplats);
+    gs::set_error("%s: needs %d splats or %d tiles, at most %d splats, 2^9 to "
+                  "2^16 tiles and at most %d pairs per bucket", what,
+                  kTileMinSplats, kTileMinTiles, gs::kTileMaxSplats,
+                  gs::kTileBucket);
     return GSPLAT_ERR_INVALID_ARGUMENT;
   }
   rc = null_check({means2d, conics, colors, opacities, depths, binned_ids,
@@ -1721,7 +1731,7 @@ int gsplat_hip_tile_render(const gsplat_raster_meta* meta,
                                 out_final_T != nullptr, zero);
   rc = gs::launch_tile_sorted(
       P, means2d, conics, colors, opacities, depths,
-      bucket_low_bits(P, capacity), capacity, packed,
+      tile_low_bits(P, capacity), capacity, packed,
       reinterpret_cast<uint32_t*>(b + L.parts),
       reinterpret_cast<uint32_t*>(b + L.start), ctl, b + L.pairs, binned_ids,
       tile_offsets, zero, s);

@@ -346,7 +346,9 @@ int launch_bucket_sort(const BucketSortArgs& A, hipStream_t stream);
 // above int32), ctl[1] = 0, ctl[2]: bit 0 a list longer than kHandoffPairs,
 // kTileSkewed a bucket or list too long (its tiles are then empty, and the
 // binning is to be done otherwise).  The first launch zeroes the two spans.
-constexpr int kTileMaxSplats = 1 << 17;
+constexpr int kTileMaxSplats = 1 << 18;
+constexpr int kTileBucket = 16384;  // pairs a bucket holds
+constexpr int kTileList = 512;      // pairs a tile's list holds
 constexpr int kTileSkewed = GSPLAT_TILE_SKEWED;
 int tile_blocks(const RasterParams& P);
 int launch_tile_sorted(const RasterParams& P, const float* means2d,

@@ -605,7 +605,7 @@ int gsplat_hip_direct_render(const gsplat_raster_meta* meta,
                              size_t render_workspace_bytes, void* stream);
 
 /* ---- Tile-sorted rendering ------------------------------------------------
- * gsplat_hip_bin_render_forward in fewer launches for scenes of up to 128K
+ * gsplat_hip_bin_render_forward in fewer launches for scenes of up to 256K
  * splats in all, of at least 16K splats or 2048 tiles: no depth order of the splats, each tile's list is sorted by
  * depth instead.  Same image, stops and gradients.  It has no counterpart in
  * the reference. */

@@ -118,7 +118,9 @@ def test_strides_hooks_and_streams(B, G, H, W):
 @pytest.mark.parametrize("kind,B,G,H,W", [
     ("uniform", 1, 16384, 512, 272),     # the fewest splats, 2^9 + 32 tiles
     ("ties", 1, 4999, 512, 1024),        # the fewest tiles
-    ("uniform", 1, 131072, 1080, 1920),  # the most
+    ("uniform", 1, 131072, 1080, 1920),
+    ("uniform", 2, 131072, 700, 1000),   # the most
+    ("uniform", 1, 131072, 4096, 4095),  # buckets above 8192 pairs
     ("ties", 3, 21845, 300, 400),        # depth ties, three images
     ("special", 2, 20001, 333, 517),     # NaN, infinite and signed zero depths
     ("uniform", 1, 70001, 4096, 4096),   # 2^16 tiles, 256 a bucket
