@@ -68,13 +68,16 @@ def kernel_work(name, BG, N, walked, T):
         "emit_kernel<false>": ("hbm", 28.0 * BG + (5.0 if N >= 1 << 23 else 8.0) * N,
                                "28 B/splat (record 24, offset 4) + 8 B/pair (key, value), or 5 B/pair (packed word "
                                "+ low tile byte) for the two-pass sort of 2^23+ pairs"),
-        "emit_kernel<orig>": ("hbm", 44.0 * BG + (5.0 if N >= 1 << 23 else 8.0) * N + N / 8.0,
+        "emit_kernel<orig>": ("hbm", 44.0 * BG + (5.0 if N >= 1 << 23 else 8.0) * N,
                               "44 B/splat (the count's record 36, offset + gid 8) + 5 or 8 B/pair as "
-                              "emit_kernel<false> + the count's hit ballots (1 bit per candidate, at least one "
-                              "per pair)"),
-        "count_kernel": ("hbm", 104.0 * BG + N / 8.0, "104 B/splat (one-call path): means 8, conic 12, opacity 4, "
-                                                      "colours 12 read, count 4 and the 64-B record written; "
-                                                      "+ the hit ballots (1 bit per candidate, at least one per pair)"),
+                              "emit_kernel<false>"),
+        "count_kernel": ("hbm", 104.0 * BG, "104 B/splat (one-call path): means 8, conic 12, opacity 4, "
+                                            "colours 12 read, count 4 and the 64-B record written"),
+        "tile_count_kernel": ("hbm", 164.0 * BG, "164 B/splat: means 8, conic 12, opacity 4, colours 12 read; record 64 "
+                                                 "written, gradient record 64 zeroed"),
+        "tile_emit_kernel": ("hbm", 28.0 * BG + 8.0 * N, "28 B/splat (means 8, conic 12, opacity 4, depth 4 read) + "
+                                                         "8 B/pair (depth key, tile and index written)"),
+        "tile_sort_kernel": ("hbm", 12.0 * N + 4.0 * T, "12 B/pair (pair read, id written) + 4 B/tile"),
         "depth_run_sort_kernel": ("hbm", 12.0 * BG, "12 B/splat: depth 4 read, run key + value 8 written"),
         "depth_run_rank_kernel": ("hbm", 12.0 * BG, "12 B/splat: run key + value 8 read, perm 4 written"),
         "pack_kernel": ("hbm", 144.0 * BG, "144 B/splat: perm 4 and the count's 64-B record read; record 64, "

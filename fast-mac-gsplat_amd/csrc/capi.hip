@@ -527,9 +527,9 @@ int bucket_low_bits(const RasterParams& P, int64_t n_pairs) {
 
 // hist_counted: the bucket form's histogram is already in the control block
 // (counted by the count launch, summed by the rank launch).  orig_walk: the
-// count wrote its records and step ballots and the pack the original-order
-// offsets (bin_count_impl with colors, bin_pack_impl with use_records), so
-// the emit walks in original order and reuses the ballots.
+// count wrote its records and the pack the original-order offsets
+// (bin_count_impl with colors, bin_pack_impl with use_records), so the emit
+// walks in original order.
 int bin_emit_impl(const gsplat_raster_meta* meta, const float* packed,
                   const int32_t* splat_offsets, int64_t n_pairs,
                   int32_t* binned_ids, int32_t* tile_counts,
