@@ -1344,7 +1344,7 @@ __global__ __launch_bounds__(kBucketThreads) void bucket_sort_kernel(
 //
 // Measured against the one-call binning (us for count, emit and sort; the five
 // launches): 64K splats at 1080p 11.9 + 13.1 + 6.5 against 60 in all, at 4096 x
-// 4096 11.1 + 15.9 + 7.3 against 63; 128K splats at 1080p 15.0 + 15.2 + 11.8
+// 4096 11.8 + 15.9 + 9.3 against 63; 128K splats at 1080p 15.0 + 15.2 + 11.8
 // against 83; 5000 splats at 1080p 8.1 + 8.4 + 4.2 against 43; 16K splats at
 // 512 x 512 8.7 + 8.7 + 6.1 against 45; two images of 32K splats at 600 x 800
 // 10.0 + 12.4 + 8.7 against 55; 262K splats in seven images of 769 x 729 14.8 +
