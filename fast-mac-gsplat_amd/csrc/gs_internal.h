@@ -197,8 +197,8 @@ int launch_slice_front(const RasterParams& P, const SliceBuffers& Q,
                        const float* depths, int slots, int64_t max_tiles,
                        hipStream_t stream);
 // After the front's forward: live_bits, live_list, back_list and the host's
-// report (the words of gsplat_hip_front_render); tile_stop of a live tile
-// becomes 0.
+// report (the words of gsplat_hip_front_render); with word 3 set tile_stop of
+// a live tile becomes 0.
 int launch_slice_back(const RasterParams& P, const SliceBuffers& Q,
                       const float* depths, const uint32_t* tile_live,
                       int32_t* tile_stop, const int32_t* bin_status,
@@ -539,8 +539,8 @@ int launch_render_backward(const RasterParams& P, const float* packed,
                            float* g_conics, float* g_colors, float* g_opac,
                            int64_t n_pairs, void* workspace,
                            hipStream_t stream);
-// The backward of a sliced forward, one launch: the front's tiles (a live
-// tile's stop is 0 there) and the live tiles of the back (live.n = 0: no
+// The backward of a sliced forward, one launch: the front's tiles (with a back
+// a live tile's stop is 0 there) and the live tiles of the back (live.n = 0: no
 // back).  Adds to the gradient records at acc ([splats of the whole scene],
 // zero on entry).
 struct BackwardSlice {

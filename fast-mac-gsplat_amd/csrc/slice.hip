@@ -25,12 +25,15 @@
 //   slice_select_kernel   compacts the splats whose box holds a live tile, cuts
 //     their boxes down to those tiles and sums the live tiles in them (a
 //     bound on the back's pairs)
-//   slice_report_kernel   what the host needs to launch the back
+//   slice_report_kernel   what the host needs to launch the back, and a stop of
+//     0 for the live tiles if there is one
 //   slice_gather_kernel   the back's attributes, once the host knows its size
 //
 // The budget counts box tiles, at least the pairs the binning emits, so the
 // buffers of a slice never overflow.  Every kernel here reads each splat
 // once or twice (44 bytes) and is bound by that and by its launch.
+#include <algorithm>
+
 #include "gs_internal.h"
 #include "gs_predicate.h"
 #include "lookback.h"
@@ -356,13 +359,11 @@ __global__ __launch_bounds__(kThreads) void slice_front_kernel(
   }
 }
 
-// 1024 tiles per workgroup: the live tiles' bits, their list (ascending
-// inside a workgroup) and, for training, a stop of 0 for them, so that the
-// front's backward passes over them.  Also the sum and number of the opaque
-// tiles' stops.
+// 1024 tiles per workgroup: the live tiles' bits and their list (ascending
+// inside a workgroup).  Also the sum and number of the opaque tiles' stops.
 __global__ __launch_bounds__(kThreads) void slice_live_kernel(
     RasterParams P, SliceBuffers Q, const uint32_t* __restrict__ tile_live,
-    int32_t* __restrict__ tile_stop) {
+    const int32_t* __restrict__ tile_stop) {
   __shared__ uint32_t wsum[kWaves];
   __shared__ uint32_t s_base;
   __shared__ uint32_t s_stops, s_opaque;
@@ -385,7 +386,6 @@ __global__ __launch_bounds__(kThreads) void slice_live_kernel(
       stops += (uint32_t)tile_stop[t];
       ++opaque_n;
     }
-    if (live) tile_stop[t] = 0;
   }
   if (lane == 0) wsum[wave] = n;
 #pragma unroll
@@ -557,11 +557,22 @@ __global__ __launch_bounds__(kThreads) void slice_select_kernel(
   }
 }
 
-// What the host reads (SliceReport of the C ABI), the ready word last.
-__global__ void slice_report_kernel(SliceBuffers Q,
-                                    const int32_t* __restrict__ bin_status,
-                                    int32_t* host) {
-  if (threadIdx.x != 0) return;
+// What the host reads (the words of gsplat_hip_front_render), the ready word
+// last; and, if a live tile needs splats that the front does not hold, a stop
+// of 0 for the live tiles, so that the front's backward leaves them to the
+// back's.  Without such a splat there is no back (the host goes by the same
+// word), and the front's stops stand.
+__global__ __launch_bounds__(kThreads) void slice_report_kernel(
+    RasterParams P, SliceBuffers Q, const uint32_t* __restrict__ tile_live,
+    int32_t* __restrict__ tile_stop, const int32_t* __restrict__ bin_status,
+    int32_t* host) {
+  const uint32_t fresh = Q.ctl[kSliceFresh];
+  if (fresh != 0u) {
+    for (int t = (int)blockIdx.x * kThreads + (int)threadIdx.x;
+         t < P.num_tiles; t += (int)gridDim.x * kThreads)
+      if (tile_live[t] != 0u) tile_stop[t] = 0;
+  }
+  if (blockIdx.x != 0 || threadIdx.x != 0) return;
   auto put = [&](int k, uint32_t v) {
     __hip_atomic_store(host + k, (int32_t)v, __ATOMIC_RELAXED,
                        __HIP_MEMORY_SCOPE_SYSTEM);
@@ -569,7 +580,7 @@ __global__ void slice_report_kernel(SliceBuffers Q,
   put(0, (uint32_t)*bin_status | Q.ctl[kSliceErr]);
   put(1, Q.ctl[kSliceLive]);
   put(2, Q.ctl[kSliceBackMax]);
-  put(3, Q.ctl[kSliceFresh]);
+  put(3, fresh);
 #pragma unroll
   for (int k = 0; k < kSliceSums; ++k) {
     put(4 + 2 * k, (uint32_t)Q.sums[k]);
@@ -667,8 +678,11 @@ int launch_slice_back(const RasterParams& P, const SliceBuffers& Q,
                 words);
   rc = check_launch("slice_select_kernel");
   if (rc) return rc;
-  launch_traced("slice_report_kernel", slice_report_kernel, dim3(1), dim3(64),
-                0, stream, Q, bin_status, host_words);
+  launch_traced("slice_report_kernel", slice_report_kernel,
+                dim3((unsigned)std::min((P.num_tiles + kThreads - 1) / kThreads,
+                                        256)),
+                dim3(kThreads), 0, stream, P, Q, tile_live, tile_stop,
+                bin_status, host_words);
   return check_launch("slice_report_kernel");
 }
 

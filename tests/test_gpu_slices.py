@@ -26,6 +26,14 @@ def _scene(B, G, H, W, seed, sigma=(4.0, 20.0), logit=0.0, depth="uniform", cove
     if depth == "veil":  # the left 45% nearly transparent: most of its splats touch live tiles
         opac = torch.where(means[..., 0] < 0.45 * W, 0.02 * opac, opac)
         depths = torch.rand(B, G, generator=g) * 10
+    if depth == "split":  # near: the left half opaque, the right 40% translucent; behind, inside the left half: the rest
+        part = torch.rand(B, G, generator=g)
+        x, y = means.unbind(-1)
+        far = part >= 0.7
+        x = torch.where(far, 0.15 * W + 0.15 * x, torch.where(part < 0.6, 0.5 * x, W - 0.4 * x))
+        means = torch.stack([x, torch.where(far, 0.25 * H + 0.45 * y, y)], -1)
+        opac = torch.where((part >= 0.6) & ~far, 0.02 + 0.0 * opac, opac)
+        depths = torch.rand(B, G, generator=g) + 5.0 * far
     t = [means, conics, torch.rand(B, G, 3, generator=g), opac, depths]
     return [x.cuda().contiguous() for x in t]
 
@@ -67,7 +75,9 @@ CASES = [
     (3, 5000, 64, 80, (2.0, 9.0), 0.0, "planes", 1.0, 300),         # tiles of three images in one bitmap word
     (1, 30000, 160, 160, (4.0, 30.0), -1.0, "uniform", 0.8, 900),   # lists over 128: continuation, segments
     (1, 350000, 512, 512, (1.0, 6.0), 0.5, "veil", 1.0, 400),       # a back of over 131,072 splats
-    (1, 20000, 200, 300, (4.0, 20.0), 0.0, "uniform", 1.0, 100000),  # the front holds every splat
+    (1, 20000, 200, 300, (4.0, 20.0), 0.0, "uniform", 1.0, 100000),  # the front holds every splat, no live tile
+    (1, 20000, 200, 300, (4.0, 20.0), 0.0, "uniform", 0.6, 100000),  # the same with live tiles: no back either
+    (1, 20000, 200, 300, (2.0, 5.0), 0.0, "split", 1.0, 390),        # what the front leaves out touches no live tile
 ]
 
 
@@ -77,14 +87,20 @@ def test_sliced_matches_unsliced(monkeypatch, B, G, H, W, sigma, logit, depth, c
     meta = _lib.make_raster_meta(H, W, B, G, 1 / 255, 1e-4, (0.1, 0.2, 0.3))
     w = torch.rand(B, H, W, 3, generator=torch.Generator().manual_seed(1)).cuda()
     st, img, T, stop, ref = _unsliced(meta, ts, w)
-    cap = max(st.n_pairs, 2 * budget * st.num_tiles)
+    # (the front's slots grow with budget / capacity: at this ratio they hold every splat)
+    whole = budget >= 100000 or depth == "split"
+    cap = max(st.n_pairs, (4 * budget * st.num_tiles // 3 + 1) if whole else 2 * budget * st.num_tiles)
     got, grads = _sliced(monkeypatch, meta, ts, w, budget, cap)
     key = (0, B, G, H, W)
     assert got is not None, f"the scene was meant to be sliced (budget now {_slices._plans[key].budget})"
     state, (img2, T2, last2) = got
     assert torch.equal(img, img2) and torch.equal(T, T2)
-    if budget >= 100000:
+    if whole:
         assert not state.has_back
+        assert bool((T > 1e-4).any()) == (cover < 1 or depth == "split")
+        layout = state.plain()[1][0][0]
+        front_offsets = state.tensors()[2][layout[2]:layout[2] + 4 * (st.num_tiles + 1)].view(torch.int32)
+        assert (int(front_offsets[-1]) < st.n_pairs) == (depth == "split")
     if depth == "veil":
         assert state.plain()[1][1][1] > 131072  # the back's slots
     for a, b in zip(grads, ref):
@@ -137,6 +153,39 @@ def test_public_calls_take_the_slices(monkeypatch):
     for g in grads[1:]:
         for a, b in zip(g, grads[0]):
             torch.testing.assert_close(a, b, rtol=1e-4, atol=1e-5 * float(b.abs().max()))
+
+
+def test_views_of_different_density(monkeypatch):
+    """A dense view and one with few visible splats by turns on one shape, whose remembered capacity is
+    the dense one's when the sparse one comes: each call gives the unsliced image and gradients."""
+    monkeypatch.setattr(_slices, "MIN_PAIRS", 1 << 18)
+    monkeypatch.setattr(_slices, "FIRST_BUDGET", 96)
+    seen = []
+    orig = _slices.render
+    monkeypatch.setattr(_slices, "render", lambda *a, **k: seen.append(orig(*a, **k)) or seen[-1])
+    B, G, H, W = 1, 40003, 190, 310
+    cfg = RasterConfig(height=H, width=W, background=(0.1, 0.2, 0.3))
+    meta = _lib.make_raster_meta(H, W, B, G, 1 / 255, 1e-4, (0.1, 0.2, 0.3))
+    monkeypatch.delitem(_ops._capacity, (0, B, G, H, W), raising=False)
+    monkeypatch.delitem(_slices._plans, (0, B, G, H, W), raising=False)
+    dense = _scene(B, G, H, W, 11)
+    sparse = _scene(B, G, H, W, 12, sigma=(1.0, 3.0))
+    sparse[3] = torch.where(torch.arange(G, device="cuda") < 3000, sparse[3], 0.0 * sparse[3]).contiguous()
+    w = torch.rand(B, H, W, 3, generator=torch.Generator().manual_seed(1)).cuda()
+    want = {}
+    for name, ts in (("dense", dense), ("sparse", sparse)):
+        monkeypatch.delitem(_ops._capacity, (0, B, G, H, W), raising=False)
+        _, img, _, _, ref = _unsliced(meta, ts, w)
+        want[name] = img, ref
+    monkeypatch.delitem(_ops._capacity, (0, B, G, H, W), raising=False)
+    for name in 4 * ("dense",) + ("sparse", "dense", "sparse", "dense", "dense", "sparse"):
+        leaves = [t.clone().requires_grad_(k < 4) for k, t in enumerate(dense if name == "dense" else sparse)]
+        img = rasterize_projected_gaussians(*leaves, cfg)
+        img.backward(w)
+        assert torch.equal(img, want[name][0])
+        for a, b in zip(leaves[:4], want[name][1]):
+            torch.testing.assert_close(a.grad, b, rtol=1e-4, atol=1e-5 * float(b.abs().max()))
+    assert any(x is not None for x in seen[1:4]) and seen[4] is not None   # dense ones and the first sparse one
 
 
 @pytest.mark.parametrize("B,G,H,W,sigma", [
