@@ -1503,7 +1503,7 @@ __global__ __launch_bounds__(kTileThreads) void tile_sort_kernel(
     const uint2* __restrict__ pairs, const uint32_t* __restrict__ bucket_start,
     int64_t capacity, int num_tiles, int low_bits, uint32_t most_work,
     uint32_t* __restrict__ binned_ids, int32_t* __restrict__ tile_offsets,
-    int32_t* __restrict__ ctl) {
+    int32_t* __restrict__ tile_ends, int32_t* __restrict__ ctl) {
   __shared__ uint64_t list[kTileBucket];  // depth key << 32 | tile << 24 | index
   __shared__ uint32_t cnt[256], start[256];
   __shared__ uint32_t wsum[4];
@@ -1556,9 +1556,12 @@ __global__ __launch_bounds__(kTileThreads) void tile_sort_kernel(
   if (t < 256) {
     for (int w = 0; w < wave; ++w) inc += wsum[w];
     start[t] = inc - n;
-    // (a skewed bucket's tiles are empty, at its end)
-    if (t < ndig && tile0 + t < num_tiles)
+    // (a skewed bucket's tiles are empty, at its end; the tile before them
+    // ends at the bucket's base, which only its tile_ends says)
+    if (t < ndig && tile0 + t < num_tiles) {
       tile_offsets[tile0 + t] = (int32_t)(skip ? end : base + inc - n);
+      tile_ends[tile0 + t] = (int32_t)(skip ? end : base + inc);
+    }
     const bool is_long = n > (uint32_t)kHandoffPairs;
     if (__ballot(is_long) != 0ull && lane == 0) atomicOr(ctl + 2, 1);
   }
@@ -1916,7 +1919,8 @@ int launch_tile_sorted(const RasterParams& P, const float* means2d,
                        int low_bits, int64_t capacity, float* packed,
                        uint32_t* parts, uint32_t* bucket_start, int32_t* ctl,
                        void* pairs, int32_t* binned_ids, int32_t* tile_offsets,
-                       const ZeroSpan zero[2], hipStream_t stream) {
+                       int32_t* tile_ends, const ZeroSpan zero[2],
+                       hipStream_t stream) {
   const unsigned blocks = (unsigned)tile_blocks(P);
   const int walk = tile_walk(P);
   launch_traced("tile_count_kernel",
@@ -1944,7 +1948,8 @@ int launch_tile_sorted(const RasterParams& P, const float* means2d,
                 reinterpret_cast<const uint2*>(pairs), bucket_start, capacity,
                 P.num_tiles, low_bits,
                 P.num_splats <= (1 << 16) ? kTileWorkSmall : kTileWork,
-                reinterpret_cast<uint32_t*>(binned_ids), tile_offsets, ctl);
+                reinterpret_cast<uint32_t*>(binned_ids), tile_offsets, tile_ends,
+                ctl);
   return check_launch("tile_sort_kernel");
 }
 

@@ -1646,14 +1646,15 @@ int gsplat_hip_direct_render(const gsplat_raster_meta* meta,
 namespace {
 // The tile-sorted path's workspace.
 struct TileLayout {
-  size_t ctl, start, parts, pairs, total;
+  size_t ctl, start, parts, ends, pairs, total;
 };
 TileLayout tile_layout(const RasterParams& P, int64_t capacity) {
   TileLayout L{};
   L.ctl = 0;
   L.start = 256;
   L.parts = L.start + gs::align_up(257 * sizeof(uint32_t), 256);
-  L.pairs = L.parts + (size_t)gs::tile_blocks(P) * 256 * sizeof(uint32_t);
+  L.ends = L.parts + (size_t)gs::tile_blocks(P) * 256 * sizeof(uint32_t);
+  L.pairs = L.ends + gs::align_up((size_t)P.num_tiles * sizeof(int32_t), 256);
   L.total = L.pairs + gs::align_up((size_t)capacity * 8, 256);
   return L;
 }
@@ -1725,6 +1726,7 @@ int gsplat_hip_tile_render(const gsplat_raster_meta* meta,
   host_words[3] = 0;
   char* b = static_cast<char*>(workspace);
   int32_t* ctl = reinterpret_cast<int32_t*>(b + L.ctl);
+  int32_t* ends = reinterpret_cast<int32_t*>(b + L.ends);
   hipStream_t s = static_cast<hipStream_t>(stream);
   gs::ZeroSpan zero[2];
   gs::render_forward_zero_spans(P, capacity, render_workspace,
@@ -1734,14 +1736,15 @@ int gsplat_hip_tile_render(const gsplat_raster_meta* meta,
       tile_low_bits(P, capacity), capacity, packed,
       reinterpret_cast<uint32_t*>(b + L.parts),
       reinterpret_cast<uint32_t*>(b + L.start), ctl, b + L.pairs, binned_ids,
-      tile_offsets, zero, s);
+      tile_offsets, ends, zero, s);
   if (rc) return rc;
   const gs::HostReport report{ctl, ctl + 1, ctl + 2, host_words};
+  const gs::TileSet tiles{nullptr, 0, nullptr, ends};
   return gs::launch_render_forward(
       P, packed, tile_offsets, binned_ids, out_rgb, out_final_T, out_last,
       out_tile_stop, capacity, render_workspace, s,
       gs::kForwardPreZeroed | gs::kForwardNoLong | gs::kForwardStoppedLast,
-      &report);
+      &report, &tiles);
 }
 
 }  // extern "C"

@@ -341,11 +341,12 @@ struct BucketSortArgs {
 int launch_bucket_sort(const BucketSortArgs& A, hipStream_t stream);
 // The tile-sorted binning of at most kTileMaxSplats splats, low_bits as the
 // bucket form's: records in original order, binned_ids original indices in
-// depth order per tile, tile_offsets.  Scratch: parts (tile_blocks(P) * 256
+// depth order per tile from tile_offsets[t] to tile_ends[t].  Scratch: parts (tile_blocks(P) * 256
 // words), bucket_start (257), pairs (capacity * 8 bytes).  ctl[0] = N (-1
 // above int32), ctl[1] = 0, ctl[2]: bit 0 a list longer than kHandoffPairs,
-// kTileSkewed a bucket or list too long (its tiles are then empty, and the
-// binning is to be done otherwise).  The first launch zeroes the two spans.
+// kTileSkewed a bucket or list too long (its tiles' ranges are then empty,
+// and the binning is to be done otherwise); without it tile_ends[t] =
+// tile_offsets[t + 1].  The first launch zeroes the two spans.
 constexpr int kTileMaxSplats = 1 << 18;
 constexpr int kTileBucket = 16384;  // pairs a bucket holds
 constexpr int kTileList = 512;      // pairs a tile's list holds
@@ -357,7 +358,8 @@ int launch_tile_sorted(const RasterParams& P, const float* means2d,
                        int low_bits, int64_t capacity, float* packed,
                        uint32_t* parts, uint32_t* bucket_start, int32_t* ctl,
                        void* pairs, int32_t* binned_ids, int32_t* tile_offsets,
-                       const ZeroSpan zero[2], hipStream_t stream);
+                       int32_t* tile_ends, const ZeroSpan zero[2],
+                       hipStream_t stream);
 // rank_pack: the second launch of the small-image depth order (runs in
 // depth_buffers, as launch_count_depth_runs leaves them) with the records
 // packed at the ranks: perm, packed, gid_count[gid] = splat_count[orig], and

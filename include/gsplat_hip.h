@@ -606,13 +606,13 @@ int gsplat_hip_direct_render(const gsplat_raster_meta* meta,
 
 /* ---- Tile-sorted rendering ------------------------------------------------
  * gsplat_hip_bin_render_forward in fewer launches for scenes of up to 256K
- * splats in all, of at least 16K splats or 2048 tiles: no depth order of the splats, each tile's list is sorted by
- * depth instead.  Same image, stops and gradients.  It has no counterpart in
- * the reference. */
+ * splats in all, of at least 16K splats or 2048 tiles: no depth order of the
+ * splats, each tile's list is sorted by depth instead.  Same image, stops and
+ * gradients.  It has no counterpart in the reference. */
 
 /* Set in host_words[2] where a scene has tiles or groups of tiles with too
- * many pairs for it: the image is then incomplete, and the scene is to be
- * rendered by gsplat_hip_bin_render_forward. */
+ * many pairs for it: these groups are composited as if they had none, and the
+ * scene is to be rendered by gsplat_hip_bin_render_forward. */
 #define GSPLAT_TILE_SKEWED 2
 
 /* 0 where the path does not apply to the shape and capacity. */
