@@ -1331,8 +1331,9 @@ int slice_params(const gsplat_raster_meta* meta, const gsplat_slice* slice,
   rc = null_check({slice}, what);
   if (rc) return rc;
   if (!gs::slice_ok(P)) {
-    gs::set_error("%s: needs at most 64 images of at most 2^18 tiles "
-                  "and fewer than 2^22 splats", what);
+    gs::set_error("%s: needs at most 64 images of at most 2^18 tiles and "
+                  "fewer than 2^22 splats, and an alpha threshold of at "
+                  "least 0", what);
     return GSPLAT_ERR_INVALID_ARGUMENT;
   }
   ms = *meta;

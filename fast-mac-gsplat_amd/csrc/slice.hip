@@ -615,10 +615,11 @@ __global__ __launch_bounds__(kThreads) void slice_gather_kernel(
 // Per image fewer than 2^22 splats (kCountShift: 2^22 boxes of 2^18 tiles)
 // and at most 2^18 tiles (the select kernel keeps an image's live bits
 // in LDS, and a block's 2048 boxes of that many tiles fit 32-bit sums) and
-// 2^16 - 1 tiles a side (16-bit boxes).
+// 2^16 - 1 tiles a side (16-bit boxes).  The slots left over hold opacity 0,
+// which is without tiles only at a threshold of 0 or more.
 bool slice_ok(const RasterParams& P) {
   return P.num_tiles > 0 && P.num_splats > 0 && P.batch <= 64 &&
-         P.gpb < (1 << 22) &&
+         P.gpb < (1 << 22) && P.alpha_thr >= 0.0f &&
          P.tiles_per_image <= (1 << 18) && P.tiles_x < (1 << 16) &&
          P.tiles_y < (1 << 16);
 }

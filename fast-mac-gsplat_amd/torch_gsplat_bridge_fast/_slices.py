@@ -48,7 +48,7 @@ class _Plan:
 _plans: dict = {}
 
 
-def _budget(meta: _lib.RasterMeta, key: tuple, tiles: int) -> Optional[_Plan]:
+def _budget(key: tuple, tiles: int) -> Optional[_Plan]:
     """The plan of a shape that is to be sliced, else None."""
     cap = _ops._capacity.get(key)
     # (the capacity is a quarter above the pairs it was taken from)
@@ -56,8 +56,6 @@ def _budget(meta: _lib.RasterMeta, key: tuple, tiles: int) -> Optional[_Plan]:
         return None
     plan = _plans.get(key)
     if plan is None or cap > 2 * plan.capacity or 2 * cap < plan.capacity:
-        if _lib.lib().gsplat_hip_slice_workspace_bytes(meta) == 0:
-            return None
         if len(_plans) > 256:
             _plans.clear()
         plan = _plans[key] = _Plan(cap)
@@ -214,10 +212,13 @@ def render(meta: _lib.RasterMeta, flat, *, save_state: bool):
     B, G, H, W = meta.batch, meta.gaussians_per_batch, meta.height, meta.width
     key = (dev.index, B, G, H, W)
     tpi = ((H + 15) // 16) * ((W + 15) // 16)
-    plan = _budget(meta, key, B * tpi)
+    plan = _budget(key, B * tpi)
     if plan is None:
         return None
     L = _lib.lib()
+    ws_bytes = L.gsplat_hip_slice_workspace_bytes(meta)
+    if ws_bytes == 0:   # not a scene that can be sliced
+        return None
     cap = _ops._capacity[key]
     budget = plan.budget
     # as many splats as the budget holds at the scene's mean pairs per splat (the nearest are larger)
@@ -232,7 +233,7 @@ def render(meta: _lib.RasterMeta, flat, *, save_state: bool):
         last = torch.empty((B, H, W), dtype=torch.int32, device=dev)
         records = torch.empty((B * G, _lib.GRAD_RECORD_FLOATS), dtype=torch.float32, device=dev)
     live_list = _ops._empty(B * tpi, torch.int32, dev)
-    ws = _ops._empty(L.gsplat_hip_slice_workspace_bytes(meta), torch.uint8, dev)
+    ws = _ops._empty(ws_bytes, torch.uint8, dev)
     rows = _rows.get(dev.index)
     if rows is None:
         rows = _rows[dev.index] = _SliceRows()

@@ -527,8 +527,8 @@ typedef struct gsplat_slice {
   int32_t slots;
 } gsplat_slice;
 
-/* 0 where the scene cannot be sliced (more than 64 images, or images of more
- * than 2^18 tiles or of 2^22 splats or more). */
+/* 0 where the scene cannot be sliced (more than 64 images, images of more than
+ * 2^18 tiles or of 2^22 splats or more, or a negative alpha threshold). */
 size_t gsplat_hip_slice_workspace_bytes(const gsplat_raster_meta* meta);
 size_t gsplat_hip_slice_splats_bytes(int32_t batch, int32_t slots);
 

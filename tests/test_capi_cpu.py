@@ -49,6 +49,9 @@ def test_workspace_queries():
     assert L.gsplat_hip_radix_sort_workspace_bytes(100_000, 3) > 0
     # invalid meta -> 0 bytes
     assert L.gsplat_hip_bin_count_workspace_bytes(_meta(tile_size=8)) == 0
+    # a slice's padding (opacity 0) needs a threshold of 0 or more
+    for thr, ok in ((1 / 255, True), (0.0, True), (-0.1, False), (float("nan"), False)):
+        assert (L.gsplat_hip_slice_workspace_bytes(_meta(alpha_threshold=thr)) > 0) == ok
 
 
 @pytest.mark.parametrize("field,value,msg", [

@@ -127,6 +127,18 @@ def test_fronts_that_do_not_suit_return_none(monkeypatch):
         assert _slices._plans[(0, 1, 20000, 200, 300)].budget in (0, 64)
 
 
+def test_negative_threshold_is_not_sliced(monkeypatch):
+    """The slots a slice leaves over hold splats of opacity 0, visible below a threshold of 0: such a config
+    goes unsliced, also where the shape has been sliced with another threshold."""
+    ts = _scene(1, 20000, 200, 300, 3)
+    meta = _lib.make_raster_meta(200, 300, 1, 20000, 1 / 255, 1e-4, (0, 0, 0))
+    n = _ops.bin_gaussians(meta, *_flat(ts)).n_pairs
+    cap = max(n, 2 * 256 * 247)
+    assert _sliced(monkeypatch, meta, ts, None, 256, cap, save_state=False)[0] is not None
+    meta = _lib.make_raster_meta(200, 300, 1, 20000, -0.1, 1e-4, (0, 0, 0))
+    assert _slices.render(meta, _flat(ts), save_state=False) is None
+
+
 def test_public_calls_take_the_slices(monkeypatch):
     """rasterize_projected_gaussians on a dense scene: the second and later calls of the shape are
     sliced and give the first call's image, through autograd too."""
