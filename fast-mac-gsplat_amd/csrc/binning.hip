@@ -1665,13 +1665,17 @@ int launch_count(const RasterParams& P, const float* means2d,
 // emit 80 us with 32, 68 with 16 when every tile was tested, 45 with 16 now),
 // and with few splats in all fewer per wavefront only fill the chip (512
 // splats: emit 8.5 us with 32, 6.6 with 16).  64K splats of 5 to 13 pairs are as fast or faster with 32 (their
-// rank launch adds to more totals otherwise, 15 against 22 us).
+// rank launch adds to more totals otherwise, 15 against 22 us).  No fewer than
+// keep the emit launch within kScanEmitMaxBlocks workgroups: with more the
+// batch would leave the small-image path (binning of four images of 131,000
+// splats at 25 pairs each 338 us, 406 outside it; of three of 100,003 243, 285).
 constexpr int kFewSplatPairs = 24;
 constexpr int kFewSplats = 1 << 14;
 
 int walk_splats(const RasterParams& P, int64_t capacity) {
   if (capacity >= (int64_t)kFewSplatPairs * P.num_splats)
-    return P.num_splats <= kWaves * 8 * kScanEmitMaxBlocks ? 8 : 16;
+    for (int walk = 8; walk <= 16; walk *= 2)
+      if (emit_blocks(P, walk) <= kScanEmitMaxBlocks) return walk;
   return P.num_splats <= kFewSplats ? 16 : kWalkSplats;
 }
 

@@ -203,6 +203,7 @@ def test_views_of_different_density(monkeypatch):
 @pytest.mark.parametrize("B,G,H,W,sigma", [
     (1, 2999, 300, 500, (6.0, 20.0)),     # 8 splats per wavefront: dozens of pairs per splat
     (2, 70001, 400, 500, (8.0, 16.0)),    # 16: as dense, over 131,072 splats in the batch
+    (3, 90001, 400, 500, (8.0, 16.0)),    # 32: as dense, over 262,144 splats in the batch
     (1, 16384, 300, 500, (0.5, 2.0)),     # 16: few splats
     (1, 16385, 300, 500, (0.5, 2.0)),     # 32
 ])
@@ -218,7 +219,9 @@ def test_walk_widths(monkeypatch, B, G, H, W, sigma):
     if sigma[0] > 1:
         assert n >= 24 * B * G
     for cap in (n, n + 1, n + n // 4):
-        got = _ops._bin_fast(meta, *_flat(ts), cap, key)
+        with _ops.LaunchTrace() as trace:
+            got = _ops._bin_fast(meta, *_flat(ts), cap, key)
+        assert "emit_kernel<true>" in [name for name, _ in trace.launches]
         assert got.n_pairs == n
         got.check_status()
         assert torch.equal(got.perm, ref.perm)
