@@ -13,6 +13,7 @@
 // forward-mode duals), batches to be split, the first binning of a shape,
 // images above the two-launch depth order, dense scenes to be sliced, staged
 // timing.
+#include <ATen/SavedTensorHooks.h>
 #include <ATen/core/grad_mode.h>
 #include <c10/core/DeviceGuard.h>
 #include <c10/core/impl/PythonDispatcherTLS.h>
@@ -706,6 +707,10 @@ py::object project(py::handle means3d, py::handle scales, py::handle quats,
 PYBIND11_MODULE(_host, m) {
   m.def("bind", &bind);
   m.def("set_timed", [](bool on) { g_timed.store(on); });
+  // Whether saved tensors go through hooks of the caller's (checkpointing,
+  // offloading).
+  m.def("saved_tensor_hooks",
+        [] { return at::SavedTensorDefaultHooks::get_hooks(true).has_value(); });
   m.def("project_images", &project_images);
   m.def("project", &project);
   py::class_<Plan>(m, "Plan")

@@ -9,6 +9,11 @@ unsliced path.  A shape is sliced when the pair count of its last binning
 makes the front a small part of it; the front's budget per tile follows the
 stops that the shape's last sliced call reported, and a shape whose tiles do
 not turn opaque early goes back to the unsliced path.
+
+What a sliced forward saves differs from call to call (the budget follows the
+calls before it, and there may be no back).  Where saved tensors go through
+hooks, a training forward is not sliced: non-reentrant checkpointing compares
+what its recomputation saves with what the first pass saved.
 """
 from __future__ import annotations
 
@@ -213,7 +218,7 @@ def render(meta: _lib.RasterMeta, flat, *, save_state: bool):
     key = (dev.index, B, G, H, W)
     tpi = ((H + 15) // 16) * ((W + 15) // 16)
     plan = _budget(key, B * tpi)
-    if plan is None:
+    if plan is None or (save_state and _lib.host().saved_tensor_hooks()):
         return None
     L = _lib.lib()
     ws_bytes = L.gsplat_hip_slice_workspace_bytes(meta)

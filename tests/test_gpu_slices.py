@@ -3,6 +3,7 @@ the image bit for bit (both walk the same splats of every tile in the same
 order), the gradients up to the order of their atomic sums."""
 import pytest
 import torch
+import torch.utils.checkpoint
 
 from torch_gsplat_bridge_fast import RasterConfig, _lib, _ops, _slices, rasterize_projected_gaussians
 
@@ -165,6 +166,35 @@ def test_public_calls_take_the_slices(monkeypatch):
     for g in grads[1:]:
         for a, b in zip(g, grads[0]):
             torch.testing.assert_close(a, b, rtol=1e-4, atol=1e-5 * float(b.abs().max()))
+
+
+def test_checkpointed_calls(monkeypatch):
+    """Non-reentrant checkpointing of a shape that is sliced otherwise: the recomputation saves what the
+    first pass saved, call after call."""
+    monkeypatch.setattr(_slices, "MIN_PAIRS", 1 << 18)
+    monkeypatch.setattr(_slices, "FIRST_BUDGET", 96)   # too small: the first sliced call raises it
+    seen = []
+    orig = _slices.render
+    monkeypatch.setattr(_slices, "render", lambda *a, **k: seen.append(orig(*a, **k)) or seen[-1])
+    B, G, H, W = 1, 40005, 190, 310
+    cfg = RasterConfig(height=H, width=W, background=(0.1, 0.2, 0.3))
+    ts = _scene(B, G, H, W, 11)
+    w = torch.rand(B, H, W, 3, generator=torch.Generator().manual_seed(1)).cuda()
+
+    def step(checkpointed):
+        leaves = [t.clone().requires_grad_(k < 4) for k, t in enumerate(ts)]
+        img = torch.utils.checkpoint.checkpoint(rasterize_projected_gaussians, *leaves, cfg, use_reentrant=False) \
+            if checkpointed else rasterize_projected_gaussians(*leaves, cfg)
+        img.backward(w)
+        return [img.detach()] + [t.grad for t in leaves[:4]]
+
+    want = step(False)
+    for checkpointed in (True, False, True, False, True):
+        got = step(checkpointed)
+        assert torch.equal(got[0], want[0])
+        for a, b in zip(got[1:], want[1:]):
+            torch.testing.assert_close(a, b, rtol=1e-4, atol=1e-5 * float(b.abs().max()))
+    assert any(x is not None for x in seen)
 
 
 def test_views_of_different_density(monkeypatch):
