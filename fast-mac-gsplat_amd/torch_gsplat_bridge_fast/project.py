@@ -195,6 +195,12 @@ def rasterize_pinhole_gaussians(means3d: Tensor, scales: Tensor, quats: Tensor, 
     if config is None:
         raise ValueError("config is required")
     plan = _plan(config)
+    if plan is None:
+        _check_3d_inputs(means3d, scales, quats, opacities)
+        m_b, *_, was_batched = _normalize_3d_inputs(means3d, scales, quats, opacities)
+        _check_colors(colors, m_b, was_batched)
+        _runtime_validate(config)
+        plan = _make_plan(config)
     if plan is not None:
         flat = _project_plain(means3d, scales, quats, opacities, fx, fy, cx, cy, camera_to_world, near_plane)
         if flat is not None:
@@ -209,8 +215,6 @@ def rasterize_pinhole_gaussians(means3d: Tensor, scales: Tensor, quats: Tensor, 
     _check_3d_inputs(means3d, scales, quats, opacities)
     m_b, s_b, q_b, o_b, was_batched = _normalize_3d_inputs(means3d, scales, quats, opacities)
     _check_colors(colors, m_b, was_batched)
-    _runtime_validate(config)
-    _make_plan(config)
     means2d, conics, opac, depths = _project_pinhole_gaussians_batched(
         m_b.contiguous(), s_b.contiguous(), q_b.contiguous(), o_b.contiguous(), fx, fy, cx, cy, camera_to_world,
         near_plane)

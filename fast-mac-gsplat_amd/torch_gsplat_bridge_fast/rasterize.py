@@ -428,8 +428,7 @@ def _rasterize_batched(means2d_b, conics_b, colors_b, opacities_b, depths_b, con
     return torch.cat(outs, dim=0) if len(outs) > 1 else outs[0]
 
 
-# Configs whose first call has gone through the checks below: the host path's plan of each (None: not
-# for this config).
+# Validated configs: the host path's plan of each (None: not for this config).
 _plans: dict = {}
 
 
@@ -444,14 +443,16 @@ def _plan(config: RasterConfig):
         return None
 
 
-def _make_plan(config: RasterConfig) -> None:
-    """Remembers the plan of a config that a whole call has just used."""
+def _make_plan(config: RasterConfig):
+    """The plan of a config that has just been validated, remembered for its later calls.  Its first call
+    takes it too: checkpointing compares what a recomputation saves with what the first pass saved, and
+    the two paths save different tensors."""
     key = (config, os.environ.get("GSP_TILE_SIZE"), os.environ.get("GSP_CHUNK"), os.environ.get("GSP_FAST_CAP"))
     try:
         if key in _plans:
-            return
+            return _plan(config)
     except TypeError:
-        return
+        return None
     plan = None
     if config.enable_overflow_fallback:   # (else the tiles' pair counts are checked)
         plan = _lib.host().Plan(
@@ -464,20 +465,24 @@ def _make_plan(config: RasterConfig) -> None:
     if len(_plans) > 256:
         _plans.clear()
     _plans[key] = plan
+    return _plan(config)
 
 
 def rasterize_projected_gaussians(means2d: Tensor, conics: Tensor, colors: Tensor, opacities: Tensor,
                                   depths: Tensor, config: RasterConfig) -> Tensor:
     plan = _plan(config)
-    if plan is not None:
-        out = plan.run(means2d, conics, colors, opacities, depths, True)
-        if out is not None:
-            return out
+    out = None if plan is None else plan.run(means2d, conics, colors, opacities, depths, True)
+    if out is not None:
+        return out
     _check_inputs(means2d, conics, colors, opacities, depths)
     means2d_b, conics_b, colors_b, opacities_b, depths_b, was_batched = _normalize_inputs(
         means2d, conics, colors, opacities, depths)
     _runtime_validate(config)
-    _make_plan(config)
+    if plan is None:
+        plan = _make_plan(config)
+        out = None if plan is None else plan.run(means2d, conics, colors, opacities, depths, True)
+        if out is not None:
+            return out
     out = _rasterize_batched(means2d_b, conics_b, colors_b, opacities_b, depths_b, config)
     # squeeze, not out[0]: the backward of an index zero-fills an image and copies the gradient into
     # it (26 + 91 us at 4096 x 4096), that of squeeze is a view

@@ -5,6 +5,7 @@ import threading
 
 import pytest
 import torch
+from torch.utils.checkpoint import checkpoint
 
 from torch_gsplat_bridge_fast import (RasterConfig, project_pinhole_gaussians, rasterize_pinhole_gaussians,
                                       rasterize_projected_gaussians)
@@ -173,6 +174,36 @@ def test_tile_sorted_matches_python(kind, B, G, H, W):
             torch.testing.assert_close(x.grad, y.grad, rtol=1e-4, atol=1e-5 * float(y.grad.abs().max()) + 1e-7)
         with torch.no_grad():
             assert torch.equal(plan.run(*ts, True), ref)
+
+
+@pytest.mark.parametrize("B,G,H,W", SIZES)
+def test_new_configs_checkpointed(B, G, H, W):
+    """A background per step on a shape whose capacity is known: each config's first call is checkpointed,
+    and its recomputation saves what it saved."""
+    ts = _scene(B, G, H, W)
+    with torch.no_grad():
+        rasterize_projected_gaussians(*ts, RasterConfig(height=H, width=W))
+    w = torch.rand(B, H, W, 3, generator=torch.Generator().manual_seed(2)).cuda()
+    for step in range(3):
+        cfg = RasterConfig(height=H, width=W, background=(0.5, 0.25, 0.125 * step))
+        a, b = _leaves(ts, (1, 1, 1, 1, 0)), _leaves(ts, (1, 1, 1, 1, 0))
+        img = checkpoint(rasterize_projected_gaussians, *a, cfg, use_reentrant=False)
+        img.backward(w)
+        ref = _python(b, cfg)
+        ref.backward(w)
+        assert torch.equal(img, ref)
+        for x, y in zip(a[:4], b[:4]):
+            torch.testing.assert_close(x.grad, y.grad, rtol=1e-4, atol=1e-5 * float(y.grad.abs().max()) + 1e-7)
+    sc = make_scene_3d(seed=4, G=G, H=H, W=W)
+    ts = [torch.cat([sc[k].cuda()] * B) for k in ("means3d", "scales", "quats", "opacities", "colors")]
+    cam = (250.0, 250.0, W / 2, H / 2)
+    with torch.no_grad():
+        rasterize_pinhole_gaussians(*ts, *cam, config=RasterConfig(height=H, width=W))
+    for step in range(2):
+        cfg = RasterConfig(height=H, width=W, background=(0.75, 0.25, 0.125 * step))
+        x = _leaves(ts, (1, 1, 1, 1, 1))
+        checkpoint(lambda *t: rasterize_pinhole_gaussians(*t, *cam, config=cfg), *x, use_reentrant=False).backward(w)
+        assert all(bool(t.grad.abs().sum() > 0) for t in x)
 
 
 def test_threads_share_a_plan():
