@@ -1585,6 +1585,12 @@ size_t gsplat_hip_direct_workspace_bytes(const gsplat_raster_meta* meta) {
   return direct_layout(P).total;
 }
 
+int64_t gsplat_hip_direct_pairs(const gsplat_raster_meta* meta) {
+  RasterParams P;
+  if (make_params(meta, P) || !gs::direct_ok(P)) return 0;
+  return gs::direct_pairs(P);
+}
+
 int gsplat_hip_direct_render(const gsplat_raster_meta* meta,
                              const float* means2d, const float* conics,
                              const float* colors, const float* opacities,
@@ -1605,7 +1611,7 @@ int gsplat_hip_direct_render(const gsplat_raster_meta* meta,
                   (long long)gs::kDirectMaxTests);
     return GSPLAT_ERR_INVALID_ARGUMENT;
   }
-  const int64_t n_pairs = (int64_t)P.num_tiles * P.gpb;
+  const int64_t n_pairs = gs::direct_pairs(P);
   rc = null_check({means2d, conics, colors, opacities, depths, binned_ids,
                    workspace, render_workspace},
                   what);

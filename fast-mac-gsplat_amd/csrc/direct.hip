@@ -21,6 +21,8 @@
 //
 // Compiled with -ffp-contract=off, like binning.hip: the lists are those of
 // the other paths bit for bit.
+#include <algorithm>
+
 #include "gs_internal.h"
 #include "record.h"
 
@@ -182,6 +184,19 @@ bool direct_ok(const RasterParams& P) {
   return P.num_tiles > 0 && P.num_splats > 0 && P.gpb <= kDirectMaxSplats &&
          P.tiles_x < (1 << 16) && P.tiles_y < (1 << 16) &&
          (int64_t)P.num_tiles * P.gpb <= kDirectMaxTests;
+}
+
+// The pairs that the compositors' workspace and variants go by: no count is
+// taken here, and the lists' room (tiles x splats) is no measure of it.  Going
+// by that room, images of more than a few tiles got a segment record per tile
+// and, above 2048 tiles, the backward for long lists: 300 splats at 2048 x
+// 2048 193 MB held for the backward and its kernel 18.7 us, now 134 and 15.5
+// (by the pair count 102 and 14.7); 100 at 4096 x 4096 705 MB and 69, now 455
+// and 57 (405, 57).  Faint scenes of 500 pairs a tile lose nothing by the
+// fewer records: 2000 splats at 1080 x 1080 118 -> 117 us.
+int64_t direct_pairs(const RasterParams& P) {
+  return std::min((int64_t)P.num_tiles * P.gpb,
+                  4 * (int64_t)P.num_tiles + (1 << 17));
 }
 
 int launch_direct_lists(const RasterParams& P, const float* means2d,

@@ -474,6 +474,7 @@ struct DirectSplats {
   float4* test;  // [num_splats]
 };
 bool direct_ok(const RasterParams& P);
+int64_t direct_pairs(const RasterParams& P);
 // Depth order, records and tile lists: tile t's gids, ascending, at
 // pairs[tile_starts[t] .. tile_ends[t]) with tile_starts[t] = t * gpb.  The
 // first launch zeroes the two spans.

@@ -50,6 +50,7 @@ using torch::autograd::variable_list;
   F(render_forward_long)                \
   F(render_backward)                    \
   F(direct_workspace_bytes)             \
+  F(direct_pairs)                       \
   F(direct_render)                      \
   F(tile_workspace_bytes)               \
   F(tile_render)                        \
@@ -205,7 +206,7 @@ enum class Mode { kDirect, kTiled, kBinned };
 struct Call {
   gsplat_raster_meta meta;
   Sizes sizes;
-  int64_t n_pairs = 0;  // pair capacity (direct: T * G)
+  int64_t n_pairs = 0;  // pair capacity (direct: gsplat_hip_direct_pairs)
   Mode mode = Mode::kBinned;
   bool batched = false, depth_grad = true;
 };
@@ -497,7 +498,7 @@ class Plan {
       const Sizes& s = sizes_of(c.meta, Mode::kDirect, tiles_ * B * G, train);
       if (s.keep[5] > 0) {
         c.mode = Mode::kDirect;
-        c.n_pairs = tiles_ * B * G;
+        c.n_pairs = api.direct_pairs(&c.meta);
         c.sizes = s;
         return true;
       }
@@ -539,8 +540,9 @@ class Plan {
                          : mode == Mode::kTiled ? (int64_t)api.tile_workspace_bytes(&m, n)
                                                 : (int64_t)api.bin_workspace_bytes(&m, n);
     if (work > 0) {
+      const int64_t walked = mode == Mode::kDirect ? api.direct_pairs(&m) : n;
       const int64_t part[5] = {BG * GSPLAT_RECORD_FLOATS * 4, n * 4, (T + 1) * 4, train ? T * 4 : 0,
-                               (int64_t)api.render_workspace_bytes(&m, train ? n : 0)};
+                               (int64_t)api.render_workspace_bytes(&m, train ? walked : 0)};
       for (int i = 0; i < 5; ++i) s.keep[i + 1] = s.keep[i] + align256(part[i]);
       const bool direct = mode != Mode::kBinned;  // (no depth order or offsets)
       s.use[1] = direct ? 0 : align256(BG * 4);

@@ -105,6 +105,7 @@ SIGNATURES = {
     ),
     "gsplat_hip_sliced_backward": (ctypes.c_int, [_PM, _PS, _PS, _vp, _i32] + [_vp] * 9),
     "gsplat_hip_direct_workspace_bytes": (_sz, [_PM]),
+    "gsplat_hip_direct_pairs": (_i64, [_PM]),
     "gsplat_hip_direct_render": (ctypes.c_int, [_PM] + [_vp] * 13 + [_sz, _vp, _sz, _vp]),
     "gsplat_hip_tile_workspace_bytes": (_sz, [_PM, _i64]),
     "gsplat_hip_tile_render": (ctypes.c_int, [_PM] + [_vp] * 5 + [_i64] + [_vp] * 9 + [_sz, _vp, _sz, _vp]),

@@ -334,7 +334,8 @@ _direct_bytes: dict = {}
 def direct_render(meta: _lib.RasterMeta, flat, *, save_state: bool):
     """(BinState, render_forward outputs) of a small scene by gsplat_hip_direct_render, where every tile
     scans its image's splats: no pair count, so the host waits for nothing and nothing can overflow.
-    None for scenes above its limits.  The state's lists start at tile_offsets[t] = t * G."""
+    None for scenes above its limits.  The state's lists start at tile_offsets[t] = t * G; its capacity is
+    gsplat_hip_direct_pairs."""
     means2d, conics, colors, opacities, depths = flat
     dev = means2d.device
     B, G, H, W = meta.batch, meta.gaussians_per_batch, meta.height, meta.width
@@ -346,18 +347,18 @@ def direct_render(meta: _lib.RasterMeta, flat, *, save_state: bool):
         L = _lib.lib()
         ws_bytes = L.gsplat_hip_direct_workspace_bytes(meta)
         tiles = B * ((H + 15) // 16) * ((W + 15) // 16)
-        n = tiles * G if ws_bytes else 0
-        sizes = (ws_bytes, L.gsplat_hip_render_workspace_bytes(meta, n if save_state else 0) if ws_bytes else 0,
-                 tiles, n)
+        walked = L.gsplat_hip_direct_pairs(meta)
+        sizes = (ws_bytes, L.gsplat_hip_render_workspace_bytes(meta, walked if save_state else 0) if ws_bytes else 0,
+                 tiles, walked)
         if len(_direct_bytes) > 256:
             _direct_bytes.clear()
         _direct_bytes[key] = sizes
-    ws_bytes, rws_bytes, tiles, n = sizes
+    ws_bytes, rws_bytes, tiles, walked = sizes
     if ws_bytes == 0:
         return None
     packed = torch.empty((B * G, _lib.RECORD_FLOATS), dtype=torch.float32, device=dev)
     starts = _empty(tiles + 1, torch.int32, dev)
-    pairs = _empty(n, torch.int32, dev)
+    pairs = _empty(tiles * G, torch.int32, dev)
     ws = _empty(ws_bytes, torch.uint8, dev)
     rws = _empty(rws_bytes, torch.uint8, dev)
     img = torch.empty((B, H, W, 3), dtype=torch.float32, device=dev)
@@ -370,7 +371,7 @@ def direct_render(meta: _lib.RasterMeta, flat, *, save_state: bool):
         meta, ptr(means2d), ptr(conics), ptr(colors), ptr(opacities), ptr(depths), ptr(packed), ptr(starts), ptr(pairs),
         ptr(img), ptr(final_T), ptr(last), ptr(tile_stop), ptr(ws), ws_bytes, ptr(rws), rws_bytes,
         torch.cuda.current_stream(dev).cuda_stream), "gsplat_hip_direct_render")
-    return (BinState(None, packed, None, starts, pairs, n),
+    return (BinState(None, packed, None, starts, pairs, walked),
             (img, final_T, last, tile_stop, (rws if save_state else None)))
 
 

@@ -320,6 +320,7 @@ class _RasterizeProjectedGaussians(torch.autograd.Function):
             st, (img, final_T, last, tile_stop, ws) = whole
             ctx.save_for_backward(st.packed, st.tile_offsets, st.pairs, final_T, last, tile_stop, ws)
             ctx.sliced = None
+            ctx.capacity = st.capacity
         # the binning's status is read before the backward (by then the GPU is done with it)
         ctx.check_status = st.check_status
         ctx.meta = meta
@@ -340,7 +341,7 @@ class _RasterizeProjectedGaussians(torch.autograd.Function):
                 bufs if bufs is not None else _ops.gradient_buffers(*ctx.shape, grad_out.device))
         else:
             packed, tile_offsets, pairs, final_T, last, tile_stop, ws = saved
-            st = _ops.BinState(None, packed, None, tile_offsets, pairs, pairs.numel())
+            st = _ops.BinState(None, packed, None, tile_offsets, pairs, ctx.capacity)
             g_m, g_q, g_c, g_o = _ops.render_backward(ctx.meta, st, final_T, last, tile_stop, grad_out, ws, out=bufs)
         need = ctx.needs_input_grad
         # The depth gradient is zero (the reference returns zeros, v8 rasterize.py:680).  For depths

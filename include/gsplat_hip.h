@@ -588,11 +588,16 @@ int gsplat_hip_sliced_backward(const gsplat_raster_meta* meta,
  * splats per image). */
 size_t gsplat_hip_direct_workspace_bytes(const gsplat_raster_meta* meta);
 
+/* The n_pairs of this path's render workspace and backward (0 where the path
+ * does not apply): no count of the scene's pairs, which is not taken. */
+int64_t gsplat_hip_direct_pairs(const gsplat_raster_meta* meta);
+
 /* packed float [B*G*16]; tile_starts int32 [T], binned_ids int32 [T*G]: tile
  * t's gids in depth order from tile_starts[t] = t*G on; the outputs and the
- * render workspace as gsplat_hip_render_forward's with n_pairs = T*G, out_last
- * as gsplat_hip_bin_render_forward's.  gsplat_hip_render_backward takes
- * tile_starts as its tile_offsets and n_pairs = T*G. */
+ * render workspace as gsplat_hip_render_forward's with n_pairs =
+ * gsplat_hip_direct_pairs, out_last as gsplat_hip_bin_render_forward's.
+ * gsplat_hip_render_backward takes tile_starts as its tile_offsets and the
+ * same n_pairs. */
 int gsplat_hip_direct_render(const gsplat_raster_meta* meta,
                              const float* means2d, const float* conics,
                              const float* colors, const float* opacities,

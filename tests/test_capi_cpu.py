@@ -49,6 +49,14 @@ def test_workspace_queries():
     assert L.gsplat_hip_radix_sort_workspace_bytes(100_000, 3) > 0
     # invalid meta -> 0 bytes
     assert L.gsplat_hip_bin_count_workspace_bytes(_meta(tile_size=8)) == 0
+    # the direct path's workspace and backward do not go by its lists' room (tiles x splats), which made the
+    # workspace of 300 splats at 2048 x 2048 89 MB
+    m = _lib.make_raster_meta(2048, 2048, 1, 300, 1 / 255, 1e-4, (0, 0, 0))
+    n = L.gsplat_hip_direct_pairs(m)
+    assert 0 < n < 64 * 16384 and n < 16384 * 300
+    assert L.gsplat_hip_render_workspace_bytes(m, n) - L.gsplat_hip_render_workspace_bytes(m, 0) < 16 << 20
+    assert L.gsplat_hip_direct_pairs(_lib.make_raster_meta(40, 50, 2, 100, 1 / 255, 1e-4, (0, 0, 0))) == 24 * 100
+    assert L.gsplat_hip_direct_pairs(_lib.make_raster_meta(40, 50, 2, 4097, 1 / 255, 1e-4, (0, 0, 0))) == 0
     # a slice's padding (opacity 0) needs a threshold of 0 or more
     for thr, ok in ((1 / 255, True), (0.0, True), (-0.1, False), (float("nan"), False)):
         assert (L.gsplat_hip_slice_workspace_bytes(_meta(alpha_threshold=thr)) > 0) == ok

@@ -28,6 +28,7 @@ def _flat(sc, B, G):
     (2, 4096, 150, 200, "uniform"),   # the most splats
     (1, 768, 2048, 2048, "uniform"),  # the most tiles x splats
     (1, 900, 48, 48, "faint"),        # lists of hundreds: continuation and segments
+    (1, 4000, 850, 870, "faint"),     # the same in 2970 tiles: more segments than records
     (1, 50, 32, 32, "culled"),        # nothing visible
 ])
 def test_direct_matches_staged(B, G, H, W, kind):
