@@ -254,10 +254,13 @@ def render(meta: _lib.RasterMeta, flat, *, save_state: bool):
     if status:
         raise RuntimeError(f"binning failed with device status {status:#x} (a decoupled look-back wait gave up); the "
                            "results of this call are invalid")
-    _adapt(plan, B * tpi, live, box, back_tiles, stops, opaque)
-    # (the box tiles bound the pairs: a much sparser scene lowers the shape's capacity)
+    # (the box tiles bound the pairs: a much sparser scene lowers the shape's capacity, and says nothing
+    # about the scenes that raise it again)
     if _ops._headroom(box) < cap // 2:
         _ops._capacity[key] = _ops._headroom(box)
+        _plans.pop(key, None)
+    else:
+        _adapt(plan, B * tpi, live, box, back_tiles, stops, opaque)
     if live == 0 or fresh == 0:
         return SlicedState(front, None, live_list, 0, records, None), (img, final_T, last)
     if 2 * back_tiles > box or back_tiles > _ops.MAX_PAIRS:

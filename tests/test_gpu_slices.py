@@ -199,12 +199,17 @@ def test_checkpointed_calls(monkeypatch):
 
 def test_views_of_different_density(monkeypatch):
     """A dense view and one with few visible splats by turns on one shape, whose remembered capacity is
-    the dense one's when the sparse one comes: each call gives the unsliced image and gradients."""
+    the dense one's when the sparse one comes: each call gives the unsliced image and gradients, and the
+    dense view is sliced whenever the capacity is its own."""
     monkeypatch.setattr(_slices, "MIN_PAIRS", 1 << 18)
-    monkeypatch.setattr(_slices, "FIRST_BUDGET", 96)
-    seen = []
+    seen = {}
     orig = _slices.render
-    monkeypatch.setattr(_slices, "render", lambda *a, **k: seen.append(orig(*a, **k)) or seen[-1])
+
+    def render(*a, **k):
+        seen[call] = orig(*a, **k)
+        return seen[call]
+
+    monkeypatch.setattr(_slices, "render", render)
     B, G, H, W = 1, 40003, 190, 310
     cfg = RasterConfig(height=H, width=W, background=(0.1, 0.2, 0.3))
     meta = _lib.make_raster_meta(H, W, B, G, 1 / 255, 1e-4, (0.1, 0.2, 0.3))
@@ -220,14 +225,16 @@ def test_views_of_different_density(monkeypatch):
         _, img, _, _, ref = _unsliced(meta, ts, w)
         want[name] = img, ref
     monkeypatch.delitem(_ops._capacity, (0, B, G, H, W), raising=False)
-    for name in 4 * ("dense",) + ("sparse", "dense", "sparse", "dense", "dense", "sparse"):
+    names = ("dense", "dense", "sparse", "dense", "sparse", "dense", "dense", "sparse")
+    for call, name in enumerate(names):
         leaves = [t.clone().requires_grad_(k < 4) for k, t in enumerate(dense if name == "dense" else sparse)]
         img = rasterize_projected_gaussians(*leaves, cfg)
         img.backward(w)
         assert torch.equal(img, want[name][0])
         for a, b in zip(leaves[:4], want[name][1]):
             torch.testing.assert_close(a.grad, b, rtol=1e-4, atol=1e-5 * float(b.abs().max()))
-    assert any(x is not None for x in seen[1:4]) and seen[4] is not None   # dense ones and the first sparse one
+    for call in (1, 2, 4, 6, 7):   # (3 and 5 find the capacity that the sparse view left)
+        assert seen[call] is not None, (call, names[call])
 
 
 @pytest.mark.parametrize("B,G,H,W,sigma", [
