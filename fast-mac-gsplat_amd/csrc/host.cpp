@@ -313,7 +313,7 @@ Call unskewed(Plan& plan, const Call& c, const Tensor&, bool train);
 Result render_all(Plan& plan, Call& c, const std::array<Tensor, 5>& in, bool train) {
   Result r = render(c, in, train);
   if (c.mode == Mode::kDirect) return r;
-  if (r.skewed) {  // (remembered: the shape's next calls are binned at once)
+  if (r.skewed) {
     c = unskewed(plan, c, in[0], train);
     r = render(c, in, train);
   }
@@ -462,13 +462,20 @@ class Plan {
     return next;
   }
 
-  // The call of a skewed scene by the one-call binning; the shape's later
-  // calls go there at once.
+  // The call of a skewed scene by the one-call binning; the shape's next
+  // calls go there at once: kSkewedCalls of them, twice as many each time it
+  // turns out skewed again (a try costs a tile-sorted binning and a forward).
   Call binned(const Call& c, bool train) {
     {
       std::lock_guard<std::mutex> lock(mu_);
-      if (skewed_.size() >= 64) skewed_.erase(skewed_.begin());
-      skewed_.emplace_back(c.meta.batch, c.meta.gaussians_per_batch);
+      Skewed* e = skewed(c);
+      if (e == nullptr) {
+        if (skewed_.size() >= 64) skewed_.erase(skewed_.begin());
+        skewed_.push_back({c.meta.batch, c.meta.gaussians_per_batch, kSkewedCalls / 2, 0});
+        e = &skewed_.back();
+      }
+      e->calls = std::min(2 * e->calls, 1 << 20);
+      e->left = e->calls;
     }
     Call next = c;
     next.mode = Mode::kBinned;
@@ -477,6 +484,18 @@ class Plan {
   }
 
  private:
+  // A shape with skewed scenes: calls it is to be binned for, and those left.
+  struct Skewed {
+    int32_t B, G;
+    int calls, left;
+  };
+  static constexpr int kSkewedCalls = 1024;
+  Skewed* skewed(const Call& c) {  // with mu_ held
+    for (auto& e : skewed_)
+      if (e.B == c.meta.batch && e.G == c.meta.gaussians_per_batch) return &e;
+    return nullptr;
+  }
+
   // Whether the batch goes in one launch (the chunking of the Python layer).
   bool one_launch(int64_t B, int64_t G) const {
     if (split_pairs_ && B > 1) return false;
@@ -512,13 +531,16 @@ class Plan {
     if (c.n_pairs <= 0 || c.n_pairs > 0x7fffffff ||
         4 * c.n_pairs >= 5 * (sliced_pairs_ + sliced_pairs_per_tile_ * tiles_ * B))
       return false;
-    bool skewed = false;
+    bool binned = false;
     {
       std::lock_guard<std::mutex> lock(mu_);
-      for (const auto& e : skewed_)
-        skewed |= e.first == c.meta.batch && e.second == c.meta.gaussians_per_batch;
+      Skewed* e = skewed(c);
+      if (e != nullptr && e->left > 0) {
+        binned = true;
+        --e->left;
+      }
     }
-    if (!skewed) {
+    if (!binned) {
       c.mode = Mode::kTiled;
       c.sizes = sizes_of(c.meta, Mode::kTiled, c.n_pairs, train);
       if (c.sizes.keep[5] > 0) return true;
@@ -564,7 +586,7 @@ class Plan {
   py::function note_pairs_;
   std::mutex mu_;
   std::vector<std::pair<std::array<int64_t, 5>, Sizes>> sizes_;
-  std::vector<std::pair<int32_t, int32_t>> skewed_;  // (B, G) of skewed scenes
+  std::vector<Skewed> skewed_;
 };
 
 Call grown(Plan& plan, const Call& c, const Tensor& like, int32_t n, bool train) {

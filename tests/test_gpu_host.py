@@ -176,6 +176,35 @@ def test_tile_sorted_matches_python(kind, B, G, H, W):
             assert torch.equal(plan.run(*ts, True), ref)
 
 
+def test_skewed_shape_is_tried_again():
+    """A scene with a tile list too long for the tile sort sends its shape's next 1024 calls to the one-call
+    binning, then the tile sort is tried again, and 2048 calls after a second such scene."""
+    B, G, H, W = 1, 20007, 600, 600
+    even, hot = _scene(B, G, H, W), _scene(B, G, H, W)
+    hot[0][:, :900] = 300.0 + 2.0 * torch.rand(B, 900, 2, generator=torch.Generator().manual_seed(5)).cuda()
+    hot[3] = 0.3 * hot[3]
+    cfg = RasterConfig(height=H, width=W, background=(0.1, 0.3, 0.3))
+    plan = _plan(cfg, even)
+    want = _python(even, cfg), _python(hot, cfg)
+
+    def launches(ts, ref):
+        with _ops.LaunchTrace() as trace, torch.no_grad():
+            img = plan.run(*ts, True)
+        assert torch.equal(img, ref)
+        return [name for name, _ in trace.launches]
+
+    for calls in (1024, 2048):
+        assert "tile_sort_kernel" in launches(even, want[0])
+        names = launches(hot, want[1])
+        assert "tile_sort_kernel" in names and "emit_kernel<true>" in names
+        assert "tile_sort_kernel" not in launches(even, want[0])
+        with torch.no_grad():
+            for _ in range(calls - 2):
+                plan.run(*even, True)
+        assert "tile_sort_kernel" not in launches(even, want[0])
+    assert "tile_sort_kernel" in launches(even, want[0])
+
+
 @pytest.mark.parametrize("B,G,H,W", SIZES)
 def test_new_configs_checkpointed(B, G, H, W):
     """A background per step on a shape whose capacity is known: each config's first call is checkpointed,
