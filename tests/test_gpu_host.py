@@ -120,7 +120,7 @@ def test_strides_hooks_and_streams(B, G, H, W):
     ("uniform", 1, 16384, 512, 272),     # the fewest splats, 2^9 + 32 tiles
     ("ties", 1, 4999, 512, 1024),        # the fewest tiles
     ("uniform", 1, 131072, 1080, 1920),
-    ("uniform", 2, 131072, 700, 1000),   # the most
+    ("uniform", 2, 131072, 800, 1100),   # the most
     ("uniform", 1, 131072, 4096, 4095),  # buckets above 8192 pairs
     ("ties", 3, 21845, 300, 400),        # depth ties, three images
     ("special", 2, 20001, 333, 517),     # NaN, infinite and signed zero depths
@@ -128,7 +128,7 @@ def test_strides_hooks_and_streams(B, G, H, W):
     ("long", 1, 30000, 400, 400),        # lists above the hand-off length, below the limit
     ("hot tile", 1, 20000, 600, 600),    # a tile above the limit: binned by the other path
     ("hot bucket", 1, 60000, 600, 600),  # a bucket above the limit
-    ("culled", 1, 20000, 600, 600),
+    ("culled", 1, 20002, 600, 600),
 ])
 def test_tile_sorted_matches_python(kind, B, G, H, W):
     g = torch.Generator().manual_seed(5)
@@ -151,7 +151,9 @@ def test_tile_sorted_matches_python(kind, B, G, H, W):
         sc["opacities"] = 0.0 * sc["opacities"]
     ts = [sc[k].cuda() for k in KEYS]
     cfg = RasterConfig(height=H, width=W, background=(0.1, 0.2, 0.3))
-    plan = _plan(cfg, ts)
+    _plan(cfg, ts)
+    rasterize_mod._plans.clear()           # (a plan that has seen no skewed scene)
+    plan = rasterize_mod._make_plan(cfg)
     L = _lib.lib()
     meta = rasterize_mod._meta(cfg, B, G)
     key = (0, B, G, H, W)
@@ -164,10 +166,16 @@ def test_tile_sorted_matches_python(kind, B, G, H, W):
     ref = _python(b, cfg)
     ref.backward(w)
     n = _ops.bin_gaussians(meta, *[t.reshape(B * G, -1).squeeze(-1) for t in ts]).n_pairs
-    for cap in (cap, cap, max(1, n), max(1, n // 2)):   # the last: too small, binned again
+    hot = kind.startswith("hot")
+    for k, cap in enumerate((cap, cap, max(1, n), max(1, n // 2))):   # the last: too small, binned again
         _ops._capacity[key] = cap
         a = _leaves(ts, (1, 1, 1, 1, 0))
-        img = plan.run(*a, True)
+        with _ops.LaunchTrace() as trace:
+            img = plan.run(*a, True)
+        names = [name for name, _ in trace.launches]
+        # (a skewed scene is tried once, then binned at once)
+        assert ("tile_sort_kernel" in names) == (not hot or k == 0)
+        assert ("emit_kernel<true>" in names) == (hot or cap < n)
         assert torch.equal(img, ref)
         img.backward(w)
         for x, y in zip(a[:4], b[:4]):
