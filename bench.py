@@ -310,8 +310,8 @@ def main() -> int:
 
     world = int(os.environ.get("WORLD_SIZE", "1"))
     if args.gpus != 1 or world != 1:
-        print(f"bench.py measures one GPU: every box in this build has one MI355X and the path has no "
-              f"cross-GPU step (got --gpus {args.gpus}, WORLD_SIZE {world}); run with --gpus 1.", file=sys.stderr)
+        print(f"bench.py measures one GPU: the path has no cross-GPU step (got --gpus {args.gpus}, "
+              f"WORLD_SIZE {world}); run with --gpus 1.", file=sys.stderr)
         return 2
 
     import numpy as np

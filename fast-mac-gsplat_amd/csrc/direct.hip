@@ -192,8 +192,9 @@ bool direct_ok(const RasterParams& P) {
 // and, above 2048 tiles, the backward for long lists: 300 splats at 2048 x
 // 2048 193 MB held for the backward and its kernel 18.7 us, now 134 and 15.5
 // (by the pair count 102 and 14.7); 100 at 4096 x 4096 705 MB and 69, now 455
-// and 57 (405, 57).  Faint scenes of 500 pairs a tile lose nothing by the
-// fewer records: 2000 splats at 1080 x 1080 118 -> 117 us.
+// and 57 (405, 57).  Long lists of faint splats lose nothing by the fewer
+// records: 2000 large ones at 1080 x 1080 119 -> 117 us, 4096 at 850 x 850 329
+// -> 246.
 int64_t direct_pairs(const RasterParams& P) {
   return std::min((int64_t)P.num_tiles * P.gpb,
                   4 * (int64_t)P.num_tiles + (1 << 17));

@@ -30,8 +30,10 @@
 //   slice_gather_kernel   the back's attributes, once the host knows its size
 //
 // The budget counts box tiles, at least the pairs the binning emits, so the
-// buffers of a slice never overflow.  Every kernel here reads each splat
-// once or twice (44 bytes) and is bound by that and by its launch.
+// buffers of a slice never overflow.  The histograms and the front read each
+// splat once (18 to 38 MB at 2^20 splats) in 16 to 18 us, 1.0 to 2.2 TB/s where
+// a large copy reaches 4.9: launch and load latency; the selection (45 us, 10
+// MB, vector units busy for 38%) is bound by its walk over the boxes' rows.
 #include <algorithm>
 
 #include "gs_internal.h"

@@ -118,7 +118,9 @@ int gsplat_hip_time_next_launch(int which, void* start_event,
  * the kernel's.  Launches after the n-th run untraced.  n = 0 disarms.
  * gsplat_hip_trace_count() gives the launches traced since the trace was
  * armed (at most n), gsplat_hip_trace_name(k) the k-th one's kernel name
- * (static storage; NULL for k out of range).  A traced launch costs the
+ * (static storage; NULL for k out of range; the forward's first launch is
+ * "render_fwd_kernel" also in images of few tiles, where it is the whole-tile
+ * form of the continuation's kernel).  A traced launch costs the
  * stream ~10 us more than an untraced one; do not arm it around a timed
  * region.  Arm and read it while no other thread launches work of the
  * library. */
